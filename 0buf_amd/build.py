@@ -89,7 +89,7 @@ def build_oracle(with_ref=True):
     odir = os.path.join(ROOT, "oracle")
     _run(["make", "-s", "-C", odir, "-B", "libpic_oracle.so"])
     ref = os.environ.get("PIC_REFERENCE_DIR", "/root/reference")
-    if with_ref and os.path.isdir(ref):
+    if with_ref and os.path.isfile(os.path.join(ref, "particle.h")):
         _run(["make", "-s", "-C", odir, "-B", "ref", f"REF={ref}"])
 
 
