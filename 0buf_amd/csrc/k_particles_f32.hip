@@ -988,57 +988,6 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_scatter_ids32(const long *off, lo
     p.id[e] = src[off[c] + j];
 }
 
-__global__ __launch_bounds__(PIC_BLOCK) void k_moments32(Grid g, long ncell, PartPtrs32 p,
-                                                        SpeciesTable sp, const int *slot_sort,
-                                                        double *partials) {
-    __shared__ double red[PIC_BLOCK];
-    double acc[27];
-    for (int k = 0; k < 27; k++) acc[k] = 0.0;
-    for (long e = (long)blockIdx.x * PIC_BLOCK + threadIdx.x; e < ncell * p.cap;
-         e += (long)gridDim.x * PIC_BLOCK) {
-        const long c = e / p.cap;
-        const int j = (int)(e % p.cap);
-        if (j >= p.count[c]) continue;
-        const int s = p.sp[e];
-        int srt = slot_sort[s];
-        srt = srt < 0 ? 0 : (srt > 2 ? 2 : srt);
-        const int i = (int)(c / ((long)g.Ny * g.Nz)), l = (int)((c / g.Nz) % g.Ny),
-                  k = (int)(c % g.Nz);
-        const double px = p.p[3][e], py = p.p[4][e], pz = p.p[5][e];
-        const double gm = sqrt(1.0 + px * px + py * py + pz * pz);
-        double v[9] = {1.0,
-                       ((double)i + (double)p.p[0][e]) * g.hx,
-                       ((double)l + (double)p.p[1][e]) * g.hy,
-                       ((double)k + (double)p.p[2][e]) * g.hz,
-                       px, py, pz,
-                       (sp.m[s] / sp.q_m[s]) * (gm - 1.0),
-                       fabs(px) + fabs(py) + fabs(pz)};
-        for (int q = 0; q < 9; q++) {
-            acc[0 * 9 + q] += (srt == 0) ? v[q] : 0.0;
-            acc[1 * 9 + q] += (srt == 1) ? v[q] : 0.0;
-            acc[2 * 9 + q] += (srt == 2) ? v[q] : 0.0;
-        }
-    }
-    for (int q = 0; q < 27; q++) {
-        red[threadIdx.x] = acc[q];
-        __syncthreads();
-        for (int w = PIC_BLOCK / 2; w > 0; w >>= 1) {
-            if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) partials[(long)blockIdx.x * 27 + q] = red[0];
-        __syncthreads();
-    }
-}
-
-__global__ void k_moments_final32(const double *partials, int nblocks, double *out27) {
-    const int k = threadIdx.x;
-    if (k >= 27) return;
-    double s = 0.0;
-    for (int b = 0; b < nblocks; b++) s += partials[(long)b * 27 + k];
-    out27[k] = s;
-}
-
 inline unsigned blocks_for(long n) { return (unsigned)((n + PIC_BLOCK - 1) / PIC_BLOCK); }
 
 }  // namespace
@@ -1183,12 +1132,4 @@ void launch_scatter_ids32(const long *offsets, long ncell, const int *src, PartP
                           hipStream_t s) {
     hipLaunchKernelGGL(k_scatter_ids32, dim3(blocks_for(ncell * p.cap)), dim3(PIC_BLOCK), 0, s,
                        offsets, ncell, src, p);
-}
-
-void launch_moments32(const Grid &g, long ncell, PartPtrs32 p, SpeciesTable sp,
-                      const int *slot_sort, double *partials, int nblocks, double *out27,
-                      hipStream_t s) {
-    hipLaunchKernelGGL(k_moments32, dim3(nblocks), dim3(PIC_BLOCK), 0, s, g, ncell, p, sp,
-                       slot_sort, partials);
-    hipLaunchKernelGGL(k_moments_final32, dim3(1), dim3(32), 0, s, partials, nblocks, out27);
 }

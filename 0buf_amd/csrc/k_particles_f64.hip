@@ -683,51 +683,6 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_gather_particles(long ncell, cons
     if (did) did[dst] = p.id ? p.id[e] : -1;
 }
 
-/* FP64 moments per sort: N, sum x,y,z, sum p, sum (m/q_m)(gamma-1), sum |p| */
-__global__ __launch_bounds__(PIC_BLOCK) void k_moments(long ncell, PartPtrs p, SpeciesTable sp,
-                                                      const int *slot_sort, double *partials) {
-    __shared__ double red[PIC_BLOCK];
-    double acc[27];
-    for (int k = 0; k < 27; k++) acc[k] = 0.0;
-    for (long e = (long)blockIdx.x * PIC_BLOCK + threadIdx.x; e < ncell * p.cap;
-         e += (long)gridDim.x * PIC_BLOCK) {
-        const long c = e / p.cap;
-        const int j = (int)(e % p.cap);
-        if (j >= p.count[c]) continue;
-        const int s = p.sp[e];
-        int srt = slot_sort[s];
-        srt = srt < 0 ? 0 : (srt > 2 ? 2 : srt);
-        const double px = p.p[3][e], py = p.p[4][e], pz = p.p[5][e];
-        const double gm = sqrt(1.0 + px * px + py * py + pz * pz);
-        double v[9] = {1.0, p.p[0][e], p.p[1][e], p.p[2][e], px, py, pz,
-                       (sp.m[s] / sp.q_m[s]) * (gm - 1.0), fabs(px) + fabs(py) + fabs(pz)};
-        for (int k = 0; k < 9; k++) {
-            double add = v[k];
-            acc[0 * 9 + k] += (srt == 0) ? add : 0.0;
-            acc[1 * 9 + k] += (srt == 1) ? add : 0.0;
-            acc[2 * 9 + k] += (srt == 2) ? add : 0.0;
-        }
-    }
-    for (int k = 0; k < 27; k++) {
-        red[threadIdx.x] = acc[k];
-        __syncthreads();
-        for (int w = PIC_BLOCK / 2; w > 0; w >>= 1) {
-            if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) partials[(long)blockIdx.x * 27 + k] = red[0];
-        __syncthreads();
-    }
-}
-
-__global__ void k_moments_final(const double *partials, int nblocks, double *out27) {
-    const int k = threadIdx.x;
-    if (k >= 27) return;
-    double s = 0.0;
-    for (int b = 0; b < nblocks; b++) s += partials[(long)b * 27 + k];
-    out27[k] = s;
-}
-
 inline unsigned blocks_for(long n) { return (unsigned)((n + PIC_BLOCK - 1) / PIC_BLOCK); }
 
 }  // namespace
@@ -800,13 +755,6 @@ void launch_scatter_ids(const long *offsets, long ncell, const int *src, PartPtr
 void launch_copy_parts(long ncell, PartPtrs from, PartPtrs to, hipStream_t s) {
     hipLaunchKernelGGL(k_copy_parts, dim3(blocks_for(ncell * from.cap)), dim3(PIC_BLOCK), 0, s,
                        ncell, from, to);
-}
-
-void launch_moments(long ncell, PartPtrs p, SpeciesTable sp, const int *slot_sort,
-                    double *partials, int nblocks, double *out27, hipStream_t s) {
-    hipLaunchKernelGGL(k_moments, dim3(nblocks), dim3(PIC_BLOCK), 0, s, ncell, p, sp, slot_sort,
-                       partials);
-    hipLaunchKernelGGL(k_moments_final, dim3(1), dim3(32), 0, s, partials, nblocks, out27);
 }
 
 TileGeom make_tile_geom(int Nx, int Ny, int Nz) {

@@ -859,6 +859,8 @@ int pic_destroy(pic_ctx *c) {
     free_queue(c->q32);
     if (c->d_rho) (void)hipFree(c->d_rho);
     if (c->d_gres) (void)hipFree(c->d_gres);
+    if (c->d_gres_ref) (void)hipFree(c->d_gres_ref);
+    if (c->d_cmom) (void)hipFree(c->d_cmom);
     if (c->d_st) hipFree(c->d_st);
     if (c->h_st) hipHostFree(c->h_st);
     if (c->d_part) hipFree(c->d_part);
@@ -1283,7 +1285,7 @@ int pic_moments(pic_ctx *c, double *out27) {
         launch_moments32(c->g, c->NC, c->p32, c->sp, c->d_slot_sort, c->d_part, c->npart,
                          c->d_red, c->stream);
     else
-        launch_moments(c->NC, c->p, c->sp, c->d_slot_sort, c->d_part, c->npart, c->d_red,
+        launch_moments(c->g, c->NC, c->p, c->sp, c->d_slot_sort, c->d_part, c->npart, c->d_red,
                        c->stream);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(c->h_red, c->d_red, 27 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -1298,18 +1300,15 @@ int pic_cell_moments(pic_ctx *c, int sort, int op, double *out) {
     if (!out || sort < 0 || sort > 2 || op < PIC_DENSITY || op > PIC_CURRENT) return PIC_ERR_INVALID;
     if ((rc = settle(c))) return rc;
     const long n = (op >= PIC_VELOCITY ? 3 : 1) * c->NC;
-    double *d = nullptr;
-    HIPCHK(hipMalloc(&d, n * sizeof(double)));
+    if (!c->d_cmom) HIPCHK(hipMalloc(&c->d_cmom, 3 * c->NC * sizeof(double)));
     if (c->fp32)
-        launch_cell_moments32(c->NC, c->p32, c->sp, c->d_slot_sort, sort, op, d, c->stream);
+        launch_cell_moments32(c->NC, c->p32, c->sp, c->d_slot_sort, sort, op, c->d_cmom, c->stream);
     else
-        launch_cell_moments64(c->NC, c->p, c->sp, c->d_slot_sort, sort, op, d, c->stream);
+        launch_cell_moments64(c->NC, c->p, c->sp, c->d_slot_sort, sort, op, c->d_cmom, c->stream);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->stream));
-    rc = PIC_SUCCESS;
-    if (hipMemcpy(out, d, n * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess) rc = PIC_ERR_HIP;
-    (void)hipFree(d);
-    return rc;
+    HIPCHK(hipMemcpy(out, c->d_cmom, n * sizeof(double), hipMemcpyDeviceToHost));
+    return PIC_SUCCESS;
 }
 
 /* ------------------------------------------------------- decision tape */
@@ -1400,23 +1399,28 @@ int pic_gauss_residual(pic_ctx *c, double *res, double *max_drift, int set_refer
     const Grid &g = c->g;
     if (!c->d_rho) HIPCHK(hipMalloc(&c->d_rho, g.G * sizeof(long long)));
     if (!c->d_gres) HIPCHK(hipMalloc(&c->d_gres, c->NC * sizeof(double)));
+    const bool first = set_reference || !c->gres_ref_set;
+    if (first && !c->d_gres_ref) HIPCHK(hipMalloc(&c->d_gres_ref, c->NC * sizeof(double)));
     HIPCHK(hipMemsetAsync(c->d_rho, 0, g.G * sizeof(long long), c->stream));
+    HIPCHK(hipMemsetAsync(c->d_red, 0, sizeof(double), c->stream));
+    const double *ref = first ? nullptr : c->d_gres_ref;
+    unsigned long long *drift = (unsigned long long *)c->d_red;
     if (c->fp32) {
-        launch_rho32(g, c->NC, c->p32, c->sp, c->d_rho, c->stream);
-        launch_gauss32(g, c->f32, c->d_rho, c->d_gres, c->stream);
+        launch_rho32(g, c->t, c->p32, c->sp, c->d_rho, c->stream);
+        launch_gauss32(g, c->f32, c->d_rho, c->d_gres, ref, drift, c->stream);
     } else {
-        launch_rho64(g, c->NC, c->p, c->sp, c->d_rho, c->stream);
-        launch_gauss64(g, c->f, c->d_rho, c->d_gres, c->stream);
+        launch_rho64(g, c->t, c->p, c->sp, c->d_rho, c->stream);
+        launch_gauss64(g, c->f, c->d_rho, c->d_gres, ref, drift, c->stream);
     }
     HIPCHK(hipGetLastError());
-    std::vector<double> h(c->NC);
+    if (first)
+        HIPCHK(hipMemcpyAsync(c->d_gres_ref, c->d_gres, c->NC * sizeof(double),
+                              hipMemcpyDeviceToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(c->h_red, c->d_red, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
-    HIPCHK(hipMemcpy(h.data(), c->d_gres, c->NC * sizeof(double), hipMemcpyDeviceToHost));
-    if (res) std::memcpy(res, h.data(), c->NC * sizeof(double));
-    if (set_reference || c->gres_ref.size() != h.size()) c->gres_ref = h;
-    double d = 0.0;
-    for (long k = 0; k < c->NC; k++) d = std::max(d, std::fabs(h[k] - c->gres_ref[k]));
-    if (max_drift) *max_drift = d;
+    if (first) c->gres_ref_set = true;
+    if (res) HIPCHK(hipMemcpy(res, c->d_gres, c->NC * sizeof(double), hipMemcpyDeviceToHost));
+    if (max_drift) *max_drift = c->h_red[0];
     return PIC_SUCCESS;
 }
 

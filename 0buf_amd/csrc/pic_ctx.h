@@ -53,7 +53,9 @@ struct pic_ctx {
     QueuePtrs32 q32{};
     long long *d_rho = nullptr;   /* Gauss residual scratch */
     double *d_gres = nullptr;
-    std::vector<double> gres_ref;
+    double *d_gres_ref = nullptr; /* the residual drifts are taken from */
+    bool gres_ref_set = false;
+    double *d_cmom = nullptr;     /* per-cell moments before their copy to the host */
     /* differentiable form: particle ids, fixed-point current (the FP64 form's
      * int64 J arrays; the FP32 form's J is fixed point already), adjoint state */
     bool diff = false;

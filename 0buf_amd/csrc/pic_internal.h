@@ -428,8 +428,6 @@ void launch_gather_particles(long ncell, const long *offsets, PartPtrs p, double
                              unsigned char *dsp, int *dcell, int *did, hipStream_t s);
 void launch_scatter_ids(const long *offsets, long ncell, const int *src, PartPtrs p,
                         hipStream_t s);
-void launch_moments(long ncell, PartPtrs p, SpeciesTable sp, const int *slot_sort,
-                    double *partials, int nblocks, double *out27, hipStream_t s);
 
 /* FP32 form (k_particles_f32.hip) */
 /* diff: differentiable form (ids; compact record of the pre-step state into
@@ -472,6 +470,10 @@ void launch_gather_raw32(long ncell, const long *offsets, PartPtrs32 p, float *d
                          unsigned char *dsp, int *did, hipStream_t s);
 void launch_scatter_ids32(const long *offsets, long ncell, const int *src, PartPtrs32 p,
                           hipStream_t s);
+
+/* per-sort moments (k_gauss.hip): nblocks x 27 partial sums, then their sums */
+void launch_moments(const Grid &g, long ncell, PartPtrs p, SpeciesTable sp, const int *slot_sort,
+                    double *partials, int nblocks, double *out27, hipStream_t s);
 void launch_moments32(const Grid &g, long ncell, PartPtrs32 p, SpeciesTable sp,
                       const int *slot_sort, double *partials, int nblocks, double *out27,
                       hipStream_t s);
@@ -493,15 +495,16 @@ void launch_generate_species(const Grid &g, const pic_species_spec &spec, const 
 
 /* Gauss-law residual div E - rho, FP64 (k_gauss.hip): rho by CIC on the
  * cell-centre lattice into an int64 fixed-point array of G entries, then
- * per bulk centre res = div E - rho; returns max |res - ref| if ref != 0 */
-void launch_rho64(const Grid &g, long ncell, PartPtrs p, SpeciesTable sp, long long *rho,
+ * per bulk centre res = div E - rho; with ref, *drift (0 before) receives
+ * the bits of max |res - ref| */
+void launch_rho64(const Grid &g, const TileGeom &t, PartPtrs p, SpeciesTable sp, long long *rho,
                   hipStream_t s);
-void launch_rho32(const Grid &g, long ncell, PartPtrs32 p, SpeciesTable sp, long long *rho,
+void launch_rho32(const Grid &g, const TileGeom &t, PartPtrs32 p, SpeciesTable sp, long long *rho,
                   hipStream_t s);
 void launch_gauss64(const Grid &g, FieldPtrs f, const long long *rho, double *res,
-                    hipStream_t s);
+                    const double *ref, unsigned long long *drift, hipStream_t s);
 void launch_gauss32(const Grid &g, FieldPtrs32 f, const long long *rho, double *res,
-                    hipStream_t s);
+                    const double *ref, unsigned long long *drift, hipStream_t s);
 
 /* Differentiable form, adjoint stages (k_adjoint.hip).  Adjoint arrays
  * have the field layout (G entries); the particle adjoints are indexed by

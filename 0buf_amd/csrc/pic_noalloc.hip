@@ -90,7 +90,8 @@ extern "C" int pic_moments_noalloc(pic_ctx *c, int nblocks, double *d_out27) {
         launch_moments32(c->g, c->NC, c->p32, c->sp, c->d_slot_sort, partials, nblocks, d_out27,
                          c->stream);
     else
-        launch_moments(c->NC, c->p, c->sp, c->d_slot_sort, partials, nblocks, d_out27, c->stream);
+        launch_moments(c->g, c->NC, c->p, c->sp, c->d_slot_sort, partials, nblocks, d_out27,
+                       c->stream);
     HIPCHK(hipGetLastError());
     return PIC_SUCCESS;
 }
