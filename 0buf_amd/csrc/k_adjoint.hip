@@ -335,8 +335,8 @@ __device__ __forceinline__ double dot3(const double a[3], const double b[3]) {
     return a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
 }
 
-template <int TX, int TY, int TZ>
-__global__ __launch_bounds__(PIC_BLOCK) void k_adj_particles(AdjArgs a) {
+template <int TX, int TY, int TZ, int NT>
+__global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
     constexpr int C = TX * TY * TZ;
     constexpr int BX = TX + 2, BY = TY + 2, BZ = TZ + 2, NB = BX * BY * BZ;
     __shared__ double sF[6 * NB];    /* E, H' of the forward step */
@@ -364,7 +364,7 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_adj_particles(AdjArgs a) {
     /* thread n takes box node n of every box (one decode, one 32-bit
      * offset: the grid has fewer than 2^31 nodes) and cell n of the tile;
      * every global load is issued before the first LDS write */
-    static_assert(NB <= PIC_BLOCK && C <= PIC_BLOCK, "one box node and one cell per thread");
+    static_assert(NB <= NT && C <= NT, "one box node and one cell per thread");
     const double *const Fsrc[6] = {a.fwd.E[0], a.fwd.E[1], a.fwd.E[2],
                                    a.fwd.H[0], a.fwd.H[1], a.fwd.H[2]};
     const int nu = tid / (BY * BZ), nv = (tid / BZ) % BY, nw = tid % BZ;
@@ -397,7 +397,7 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_adj_particles(AdjArgs a) {
         }
         if (tid < C) sCnt[tid] = cnt;
     }
-    for (int e = tid; e < ACOPIES * 6 * NB; e += PIC_BLOCK) sA[e] = 0.0;
+    for (int e = tid; e < ACOPIES * 6 * NB; e += NT) sA[e] = 0.0;
     if (tid == 0) sFlags = 0;
     __syncthreads();
     if (tid == 0) {
@@ -413,7 +413,7 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_adj_particles(AdjArgs a) {
 
     const double hx = g.hx, hy = g.hy, hz = g.hz, tau = g.tau;
     unsigned bad = 0;
-    for (int fidx = tid; fidx < T; fidx += PIC_BLOCK) {
+    for (int fidx = tid; fidx < T; fidx += NT) {
         int lo = 0, hi = C;
         while (hi - lo > 1) {
             int mid = (lo + hi) >> 1;
@@ -673,8 +673,14 @@ void launch_adj_particles_f64(const Grid &g, const TileGeom &t, AdjFwd fwd, Part
     a.lam = l;
     a.lp = lp;
     a.st = st;
-    hipLaunchKernelGGL((k_adj_particles<TXC, TYC, TZC>), dim3((unsigned)t.ntiles), dim3(PIC_BLOCK),
-                       0, s, a);
+    /* two wavefronts per SIMD at one tile per CU, as many as the registers
+     * allow: 151 against 176 us at 256 tiles of 48 particles per cell; from two
+     * tiles per CU on no gain (250 us either way at 512 tiles) */
+    if (t.ntiles <= 256)
+        hipLaunchKernelGGL((k_adj_particles<TXC, TYC, TZC, 512>), dim3((unsigned)t.ntiles), dim3(512), 0, s, a);
+    else
+        hipLaunchKernelGGL((k_adj_particles<TXC, TYC, TZC, PIC_BLOCK>), dim3((unsigned)t.ntiles),
+                           dim3(PIC_BLOCK), 0, s, a);
 }
 
 void launch_adj_curl_h(const Grid &g, AdjLam l, hipStream_t s) {

@@ -20,6 +20,7 @@
 namespace {
 
 constexpr int TXC = 2, TYC = 4, TZC = 8;
+constexpr int ADJ_NT = 512;   /* threads of a workgroup (launch_adj_particles_f32) */
 
 /* copies of the LDS adjoint box the gather adjoint scatters into: lane l adds
  * into copy l % ACOPIES, dividing the same-address conflicts of the FP64 LDS
@@ -132,8 +133,8 @@ __device__ __forceinline__ float dot3f(const float a[3], const float b[3]) {
     return a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
 }
 
-template <int TX, int TY, int TZ>
-__global__ __launch_bounds__(PIC_BLOCK) void k_adj_particles32(AdjArgs32 a) {
+template <int TX, int TY, int TZ, int NT>
+__global__ __launch_bounds__(NT) void k_adj_particles32(AdjArgs32 a) {
     constexpr int C = TX * TY * TZ;
     constexpr int BX = TX + 2, BY = TY + 2, BZ = TZ + 2, NB = BX * BY * BZ;
     /* the push's box layout: Ex, Hy, Hz (node-type along x) take x planes
@@ -167,7 +168,7 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_adj_particles32(AdjArgs32 a) {
     /* thread n takes box node n in every component box (one decode, one
      * 32-bit offset: the grid has fewer than 2^31 nodes) and cell n of the
      * tile; every global load is issued before the first LDS write */
-    static_assert(NB <= PIC_BLOCK && C <= PIC_BLOCK, "one box node and one cell per thread");
+    static_assert(NB <= NT && C <= NT, "one box node and one cell per thread");
     constexpr int FN[6] = {NBX, NB, NB, NB, NBX, NBX};   /* nodes in each box */
     const float *const Fsrc[6] = {a.fwd.E[0], a.fwd.E[1], a.fwd.E[2],
                                   a.fwd.H[0], a.fwd.H[1], a.fwd.H[2]};
@@ -203,7 +204,7 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_adj_particles32(AdjArgs32 a) {
         }
         if (tid < C) sCnt[tid] = cnt;
     }
-    for (int e = tid; e < ACOPIES * NF; e += PIC_BLOCK) sA[e] = 0.0;
+    for (int e = tid; e < ACOPIES * NF; e += NT) sA[e] = 0.0;
     __syncthreads();
     if (tid == 0) {
         int s = 0;
@@ -216,7 +217,7 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_adj_particles32(AdjArgs32 a) {
     __syncthreads();
     const int T = sOff[C];
 
-    for (int fidx = tid; fidx < T; fidx += PIC_BLOCK) {
+    for (int fidx = tid; fidx < T; fidx += NT) {
         int blo = 0, bhi = C;
         while (bhi - blo > 1) {
             int mid = (blo + bhi) >> 1;
@@ -434,8 +435,12 @@ void launch_adj_particles_f32(const Grid &g, const TileGeom &t, AdjFwd32 fwd, Pa
     a.lam = l;
     a.lp = lp;
     a.st = st;
-    hipLaunchKernelGGL((k_adj_particles32<TXC, TYC, TZC>), dim3((unsigned)t.ntiles),
-                       dim3(PIC_BLOCK), 0, s, a);
+    /* 8 wavefronts per tile: two tiles fill a CU's 16 wavefronts (the boxes
+     * allow three tiles of 4), and a lone tile has two wavefronts per SIMD.
+     * Against 4 wavefronts per tile, 48 particles per cell: 106 / 125 us at 256
+     * tiles, 250 / 262 at 1024, 437 / 446 at 2048 */
+    hipLaunchKernelGGL((k_adj_particles32<TXC, TYC, TZC, ADJ_NT>), dim3((unsigned)t.ntiles),
+                       dim3(ADJ_NT), 0, s, a);
 }
 
 void launch_lam_copy(LamParts lp, double *flat, int k, bool to_lines, hipStream_t s) {

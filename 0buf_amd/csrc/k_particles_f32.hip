@@ -23,6 +23,8 @@
  *   * migration by the cell-local offset: a particle whose offset leaves
  *     [0,1) moves to the neighbouring cell (periodic), exactly one receiver.
  */
+#include <type_traits>
+
 #include "pic_internal.h"
 #include "k_push_math32.h"
 #include "k_queue_key.h"
@@ -137,11 +139,11 @@ __device__ __forceinline__ int cell_groups_packed(int ps, int bc, int nin, int n
     return nb + (nin + IBG - 1) / IBG + (nsp + SPG - 1) / SPG;
 }
 
-template <int C>
+template <int C, int NT>
 __device__ __forceinline__ void build_groups32(const int *sCnt, const int *sBc, const int *sBase,
                                                const int *sG, bool packed, unsigned *sGrp,
                                                int tid) {
-    for (int w = tid; w < 4 * C; w += PIC_BLOCK) {
+    for (int w = tid; w < 4 * C; w += NT) {
         const int c = w >> 2, part = w & 3;
         const int cnt = sCnt[c], bc = sBc[c];
         const int nin = min(PIC_INBOX, cnt - bc), ninb = (nin + IBG - 1) / IBG,
@@ -181,8 +183,8 @@ __device__ __forceinline__ void build_groups32(const int *sCnt, const int *sBc, 
 
 /* 7 waves per SIMD (at most 72 VGPRs): about 1% faster than 8 at 64 VGPRs,
  * which spill scalar registers */
-template <int TX, int TY, int TZ, bool DIFF, bool RAW>
-__global__ __launch_bounds__(PIC_BLOCK, 7) void k_push_deposit32(PushArgs32 a) {
+template <int TX, int TY, int TZ, bool DIFF, bool RAW, int NT>
+__global__ __launch_bounds__(NT, NT == 1024 ? 4 : NT == 512 ? 6 : 7) void k_push_deposit32(PushArgs32 a) {
     constexpr int C = TX * TY * TZ;
     constexpr int BX = TX + 2, BY = TY + 2, BZ = TZ + 2, NB = BX * BY * BZ;
     /* Field boxes in LDS, one after another: a component interpolated as
@@ -194,7 +196,7 @@ __global__ __launch_bounds__(PIC_BLOCK, 7) void k_push_deposit32(PushArgs32 a) {
     constexpr int FB[6] = {0, NBX, NBX + NB, NBX + 2 * NB, NBX + 3 * NB, 2 * NBX + 3 * NB};
     constexpr int NF = 3 * NBX + 3 * NB;
     constexpr int JY0 = NBX, JZ0 = NBX + NB, NJ = NBX + 2 * NB;
-    constexpr int NW = PIC_BLOCK / 64;
+    constexpr int NW = NT / 64;
     __shared__ float2 sF[NF];   /* (value, z difference to the next node) per box node */
     /* J box copies JS elements apart: JS = NJ rounded up to 8 mod 16, so
      * that copy 1 sits 16 (of 32) or 48 (of 64) dword banks from copy 0 and
@@ -245,7 +247,7 @@ __global__ __launch_bounds__(PIC_BLOCK, 7) void k_push_deposit32(PushArgs32 a) {
      * fewer than 2^31 nodes) and cell n of the tile; every global load is
      * issued before the first LDS write, from uniform base addresses, so
      * the workgroup waits for one memory round trip here. */
-    static_assert(NB <= PIC_BLOCK && C <= PIC_BLOCK, "one box node and one cell per thread");
+    static_assert(NB <= NT && C <= NT, "one box node and one cell per thread");
     constexpr int FN[6] = {NBX, NB, NB, NB, NBX, NBX};   /* nodes in each box */
     const float *const Fsrc[6] = {a.f.E[0], a.f.E[1], a.f.E[2], a.f.H[0], a.f.H[1], a.f.H[2]};
     float fv[6], fd[6];   /* node value, next node's value (0 outside the grid) */
@@ -291,8 +293,8 @@ __global__ __launch_bounds__(PIC_BLOCK, 7) void k_push_deposit32(PushArgs32 a) {
         sBase[tid] = packed ? ps : ((ca * g.Ny + cb) * g.Nz + cc) * cap;
         sIB[tid] = ((ca * g.Ny + cb) * g.Nz + cc) * PIC_INBOX;
     }
-    for (int e = tid; e < JCOPIES * JS; e += PIC_BLOCK) sJ[e] = 0;
-    for (int h = tid; h < NB; h += PIC_BLOCK) sHalo[h] = 0;
+    for (int e = tid; e < JCOPIES * JS; e += NT) sJ[e] = 0;
+    for (int h = tid; h < NB; h += NT) sHalo[h] = 0;
     /* the per-species constants in LDS: a kernel-argument table indexed by a
      * per-particle value would be a vector memory load in the loop, and its
      * wait would also wait for the next chunk's loads issued ahead of it */
@@ -340,7 +342,7 @@ __global__ __launch_bounds__(PIC_BLOCK, 7) void k_push_deposit32(PushArgs32 a) {
         }
     }
     __syncthreads();
-    build_groups32<C>(sCnt, sBc, sBase, sG, packed, sGrp, tid);
+    build_groups32<C, NT>(sCnt, sBc, sBase, sG, packed, sGrp, tid);
     if (tid <= NW) sFirst[tid] = wave_first_cell<C>(sOff, tid, NW);
     __syncthreads();
 
@@ -638,7 +640,7 @@ __global__ __launch_bounds__(PIC_BLOCK, 7) void k_push_deposit32(PushArgs32 a) {
         dtile = ((long)(gx / TX) * a.t.nty + gy / TY) * a.t.ntz + gz / TZ;
         lc = ((gx % TX) * TY + gy % TY) * TZ + gz % TZ;
     };
-    for (int h = tid; h < NB; h += PIC_BLOCK) {
+    for (int h = tid; h < NB; h += NT) {
         const int n = sHalo[h];
         if (n > 0) {
             long cell, dt;
@@ -650,7 +652,7 @@ __global__ __launch_bounds__(PIC_BLOCK, 7) void k_push_deposit32(PushArgs32 a) {
     __syncthreads();
     const int nq = min(sQ, a.q.qcap);
     const float4 *const QE = QT;
-    for (int j = tid; j < nq; j += PIC_BLOCK) {
+    for (int j = tid; j < nq; j += NT) {
         const float4 A = QE[2 * j];
         float4 B = QE[2 * j + 1];
         const unsigned key = __float_as_uint(B.z);
@@ -1033,15 +1035,21 @@ void launch_push_deposit_f32(const Grid &g, const TileGeom &t, FieldPtrs32 f, Pa
                                                      PIC_INBOX / IBG + 1) +
                                     L.scap / SPG + 1);
     a.ngrp = (int)(lds / 4);
-    if (diff)
-        hipLaunchKernelGGL((k_push_deposit32<TXC, TYC, TZC, true, false>),
-                           dim3((unsigned)t.ntiles), dim3(PIC_BLOCK), lds, s, a);
-    else if (raw_current_sums_exact(a, p.cap))
-        hipLaunchKernelGGL((k_push_deposit32<TXC, TYC, TZC, false, true>),
-                           dim3((unsigned)t.ntiles), dim3(PIC_BLOCK), lds, s, a);
-    else
-        hipLaunchKernelGGL((k_push_deposit32<TXC, TYC, TZC, false, false>),
-                           dim3((unsigned)t.ntiles), dim3(PIC_BLOCK), lds, s, a);
+    const int nt = push_threads(t.ntiles);
+    auto launch = [&](auto diff_on, auto raw, auto threads) {
+        constexpr int NT = decltype(threads)::value;
+        hipLaunchKernelGGL((k_push_deposit32<TXC, TYC, TZC, decltype(diff_on)::value,
+                                             decltype(raw)::value, NT>),
+                           dim3((unsigned)t.ntiles), dim3(NT), lds, s, a);
+    };
+    auto with_threads = [&](auto diff_on, auto raw) {
+        if (nt == 1024) launch(diff_on, raw, std::integral_constant<int, 1024>());
+        else if (nt == 512) launch(diff_on, raw, std::integral_constant<int, 512>());
+        else launch(diff_on, raw, std::integral_constant<int, PIC_BLOCK>());
+    };
+    if (diff) with_threads(std::true_type(), std::false_type());
+    else if (raw_current_sums_exact(a, p.cap)) with_threads(std::false_type(), std::true_type());
+    else with_threads(std::false_type(), std::false_type());
 }
 
 /* Whether the push may sum its current contributions as raw offset words

@@ -17,6 +17,8 @@
  * The arithmetic mirrors cell.h / particle.h in the reference's evaluation
  * order and is built with -ffp-contract=off.
  */
+#include <type_traits>
+
 #include "k_arrive.h"
 #include "k_tape.h"
 #include "k_push_math.h"
@@ -107,8 +109,8 @@ __device__ __forceinline__ void pqr_lds(double *sJ, const Geo &c, const DivConst
 
 /* 4 waves per SIMD (at most 128 VGPRs): the FP64 chains of the push are
  * latency-bound at 3 */
-template <int TX, int TY, int TZ, bool DIFF>
-__global__ __launch_bounds__(PIC_BLOCK, 4) void k_push_deposit(PushArgs a) {
+template <int TX, int TY, int TZ, bool DIFF, int NT>
+__global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
     constexpr int C = TX * TY * TZ;
     constexpr int BX = TX + 2, BY = TY + 2, BZ = TZ + 2, NB = BX * BY * BZ;
     __shared__ double sF[6 * NB];
@@ -152,7 +154,7 @@ __global__ __launch_bounds__(PIC_BLOCK, 4) void k_push_deposit(PushArgs a) {
     /* Thread n takes box node n of the six field boxes (one decode, one
      * 32-bit offset: the grid has fewer than 2^31 nodes) and cell n of the
      * tile; every global load is issued before the first LDS write. */
-    static_assert(NB <= PIC_BLOCK && C <= PIC_BLOCK, "one box node and one cell per thread");
+    static_assert(NB <= NT && C <= NT, "one box node and one cell per thread");
     const int nu = tid / (BY * BZ), nv = (tid / BZ) % BY, nw = tid % BZ;
     const bool node_in = tid < NB && I0 + nu <= g.Nx + 1 && L0 + nv <= g.Ny + 1 &&
                          K0 + nw <= g.Nz + 1;
@@ -185,7 +187,7 @@ __global__ __launch_bounds__(PIC_BLOCK, 4) void k_push_deposit(PushArgs a) {
             sBase[tid] = ((ca * g.Ny + cb) * g.Nz + cc) * cap;
         }
     }
-    for (int e = tid; e < JCOPIES * 3 * NB; e += PIC_BLOCK) sJ[e] = 0.0;
+    for (int e = tid; e < JCOPIES * 3 * NB; e += NT) sJ[e] = 0.0;
     /* weight and q/m per species slot: a kernel-argument table indexed by a
      * per-particle value would be a vector memory load in the loop, whose
      * wait would also wait for the particle loads in flight */
@@ -213,7 +215,7 @@ __global__ __launch_bounds__(PIC_BLOCK, 4) void k_push_deposit(PushArgs a) {
         }
     }
     __syncthreads();
-    build_groups<TX, TY, TZ, GS64>(sCnt, sG, sGrp, tid, PIC_BLOCK);
+    build_groups<TX, TY, TZ, GS64>(sCnt, sG, sGrp, tid, NT);
     __syncthreads();
 
     /* per-tile bases of the particle arrays: slot rel of the tile is
@@ -232,8 +234,8 @@ __global__ __launch_bounds__(PIC_BLOCK, 4) void k_push_deposit(PushArgs a) {
      * chunks); stayers are compacted in place in flat order */
     const int lane = tid & 63, wv = tid >> 6;
     const int ghi = __builtin_amdgcn_readfirstlane(
-        sG[wave_first_cell<C>(sOff, wv + 1, PIC_BLOCK / 64)]);
-    int g0 = __builtin_amdgcn_readfirstlane(sG[wave_first_cell<C>(sOff, wv, PIC_BLOCK / 64)]);
+        sG[wave_first_cell<C>(sOff, wv + 1, NT / 64)]);
+    int g0 = __builtin_amdgcn_readfirstlane(sG[wave_first_cell<C>(sOff, wv, NT / 64)]);
     int o0 = 0;
     int carry_cell = -1, carry_cnt = 0;
     while (g0 < ghi) {
@@ -523,7 +525,7 @@ __global__ __launch_bounds__(PIC_BLOCK, 4) void k_push_deposit(PushArgs a) {
     __syncthreads();
 
     int maxout = 0;
-    for (int c = tid; c < C; c += PIC_BLOCK) {
+    for (int c = tid; c < C; c += NT) {
         const int ca = c / (TY * TZ), cb = (c / TZ) % TY, cc = c % TZ;
         const int gi = I0 + ca, gl = L0 + cb, gk = K0 + cc;
         if (gi >= g.Nx || gl >= g.Ny || gk >= g.Nz) continue;
@@ -705,12 +707,19 @@ void launch_push_deposit_f64(const Grid &g, const TileGeom &t, FieldPtrs f, Part
     a.snap_on = diff && diff->snap.p[0] != nullptr;
     /* dynamic LDS: one 4-byte entry per line group */
     const size_t lds = (size_t)4 * TXC * TYC * TZC * ((p.cap + GS64 - 1) / GS64);
-    if (diff)
-        hipLaunchKernelGGL((k_push_deposit<TXC, TYC, TZC, true>), dim3((unsigned)t.ntiles),
-                           dim3(PIC_BLOCK), lds, s, a);
-    else
-        hipLaunchKernelGGL((k_push_deposit<TXC, TYC, TZC, false>), dim3((unsigned)t.ntiles),
-                           dim3(PIC_BLOCK), lds, s, a);
+    const int nt = push_threads(t.ntiles);
+    auto launch = [&](auto diff_on, auto threads) {
+        constexpr int NT = decltype(threads)::value;
+        hipLaunchKernelGGL((k_push_deposit<TXC, TYC, TZC, decltype(diff_on)::value, NT>),
+                           dim3((unsigned)t.ntiles), dim3(NT), lds, s, a);
+    };
+    auto with_threads = [&](auto diff_on) {
+        if (nt == 1024) launch(diff_on, std::integral_constant<int, 1024>());
+        else if (nt == 512) launch(diff_on, std::integral_constant<int, 512>());
+        else launch(diff_on, std::integral_constant<int, PIC_BLOCK>());
+    };
+    if (diff) with_threads(std::true_type());
+    else with_threads(std::false_type());
 }
 
 void launch_jfix_to_f64(const Grid &g, FieldPtrs f, DiffArgs d, hipStream_t s) {

@@ -362,6 +362,21 @@ struct SpeciesTable {
     double q_m[PIC_MAX_SLOTS];
 };
 
+/* Threads of a push workgroup (one tile).  A tile's particles are shared out
+ * among the workgroup's wavefronts, so with few tiles more wavefronts per
+ * tile fill the chip: 4 give each SIMD one wavefront at 256 tiles (256 CUs),
+ * which then walks its chunks alone, their latencies exposed.  Whole steps,
+ * 48 particles per cell, us with 256 / 512 / 1024 threads:
+ *   tiles   FP64                  FP32
+ *     32    125 / 106 / 100        96 /  85 /  85
+ *    256    130 / 111 / 105        97 /  89 /  85
+ *    512    154 / 138 / 151       105 /  95 / 105
+ *    768    179 / 176 / 198       113 / 107 / 126
+ *   1024    213 / 213 / 248       121 / 128 / 149 */
+inline int push_threads(long ntiles) {
+    return ntiles <= 256 ? 1024 : ntiles <= 768 ? 512 : PIC_BLOCK;
+}
+
 /* kernel launchers (k_fields.hip) */
 /* the step's fused pass after the push: the current fold, H^{n+1} into
  * h_out (the second H arrays; the caller swaps them with the live ones), the
