@@ -1,5 +1,5 @@
 /*
- * k_arrive.h -- arrival of the departed particles, both precisions: the
+ * k_arrive.h -- arrival of the departed particles, FP64 form: the
  * receiving side of the reference's migration (GPU_ArrangeFlights /
  * Cell::Insert, kernels.cu:316-370), where each leaver joins the bucket of
  * the cell that accepts it.
@@ -18,12 +18,20 @@
 #ifndef K_ARRIVE_H
 #define K_ARRIVE_H
 
+#include "k_fold.h"
 #include "k_queue_key.h"
 #include "pic_internal.h"
 
-template <int TX, int TY, int TZ, class P, class Q>
-__global__ __launch_bounds__(PIC_BLOCK) void k_arrive_tile(Grid g, TileGeom t, P p, Q q,
-                                                           DevStatus *st) {
+/* workgroups [0, tiles): the arrivals of one tile each (tiles: all, or 0);
+ * those behind them: the periodic fold of the current */
+template <int TX, int TY, int TZ, class P, class Q, class JT>
+__global__ __launch_bounds__(PIC_BLOCK) void k_arrive_fold(Grid g, TileGeom t, P p, Q q,
+                                                           DevStatus *st, FoldJ<JT> f,
+                                                           unsigned tiles) {
+    if (blockIdx.x >= tiles) {
+        fold_class(g, f, (blockIdx.x - tiles) * PIC_BLOCK + threadIdx.x);
+        return;
+    }
     constexpr int BY = TY + 2, BZ = TZ + 2, NH = (TX + 2) * BY * BZ;
     __shared__ int hcnt[NH];
     __shared__ int hbase[NH];

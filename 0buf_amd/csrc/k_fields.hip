@@ -11,7 +11,9 @@
  * HBM roofline: streaming stencils; neighbour reads at +-1 in k, +-(nz+2) and
  * +-(ny+2)(nz+2) hit L2.
  */
-#include "pic_internal.h"
+#include <algorithm>
+
+#include "k_fold.h"
 
 #pragma clang fp contract(off)
 
@@ -98,8 +100,10 @@ struct HOut {
  * getMagneticFieldTraceShifts (722-733); fused with the J := 0 of
  * SetCurrentsToZero (gpu_plasma.h:2058-2069). */
 template <typename T, typename JT>
-__global__ __launch_bounds__(PIC_BLOCK) void k_h_half(Grid g, FV<T, JT> f, YeeC<T> c) {
+__global__ __launch_bounds__(PIC_BLOCK) void k_h_half(Grid g, FV<T, JT> f, YeeC<T> c,
+                                                     DevStatus *reset) {
     const unsigned n = xcd_block() * PIC_BLOCK + threadIdx.x;
+    if (reset && n == 0) *reset = DevStatus{0, 0, 0, 0, 0};
     if (n >= (unsigned)g.G) return;
     int i, l, k;
     decode32(g, n, i, l, k);
@@ -197,106 +201,6 @@ __device__ __forceinline__ T hn1(const Grid &g, const FV<T, JT> &f, int d, unsig
                   : d == 1 ? (i <= g.Nx && k <= g.Nz) : (i <= g.Nx && l <= g.Ny);
     if (in) h += f.Q[d][m];
     return h;
-}
-
-/* k_fold_j's four operations on one line, restricted to one partner pair:
- * r at the representative (position N or 1), p at its partner (0 or N+1),
- * for fold direction dir and current component cc:
- *   J[1] += J[N+1] (dir != cc);  J[N+1] = J[1] (unless dir = cc = y);
- *   J[0] += J[N];  J[N] = J[0]. */
-template <typename JT>
-__device__ __forceinline__ void fold_pair(JT &r, JT &p, int dir, int cc, bool at_n) {
-    if (at_n) {
-        const JT s = p + r;
-        r = s;
-        p = s;
-    } else if (dir != cc) {
-        const JT s = r + p;
-        r = s;
-        p = s;
-    } else if (dir != 1) {
-        p = r;
-    }
-}
-
-/* the classes of nodes the current fold combines: along each axis the fold
- * only ever combines position N with 0 and position 1 with N+1 (N >= 3, so
- * the pairs are distinct), so the nodes whose coordinates are a
- * representative's own or its partner's (representative in [1,N]^3) form a
- * class no other class's fold touches.  The classes of more than one node
- * have their representative on a face of [1,N]^3: 2 Ny Nz with ri in
- * {1, Nx}, 2 (Nx-2) Nz with ri inside and rl in {1, Ny}, 2 (Nx-2)(Ny-2) with
- * ri, rl inside and rk in {1, Nz}. */
-__device__ __forceinline__ unsigned shell_count(const Grid &g) {
-    return 2u * (unsigned)g.Ny * g.Nz + 2u * (unsigned)(g.Nx - 2) * g.Nz +
-           2u * (unsigned)(g.Nx - 2) * (g.Ny - 2);
-}
-
-/* SetPeriodicCurrentComponent (gpu_plasma.h:926-978), the three k_fold_j
- * launches x, y, z in one: one thread per class of more than one node, the
- * class's current folded in registers (x pairs, then y, then z, as the
- * launches run, with the same additions) and written back. */
-template <typename T, typename JT>
-__global__ __launch_bounds__(PIC_BLOCK) void k_fold_j_classes(Grid g, FV<T, JT> f) {
-    unsigned t = blockIdx.x * PIC_BLOCK + threadIdx.x;
-    if (t >= shell_count(g)) return;
-    const int Nx = g.Nx, Ny = g.Ny, Nz = g.Nz;
-    int ri, rl, rk;
-    const unsigned fx = 2u * Ny * Nz, fy = 2u * (unsigned)(Nx - 2) * Nz;
-    if (t < fx) {                                    /* ri in {1, Nx} */
-        const unsigned a = t / ((unsigned)Ny * Nz), r = t - a * ((unsigned)Ny * Nz);
-        ri = a ? Nx : 1;
-        rl = (int)(r / Nz) + 1;
-        rk = (int)(r % Nz) + 1;
-    } else if ((t -= fx) < fy) {                     /* rl in {1, Ny} */
-        const unsigned a = t / ((unsigned)(Nx - 2) * Nz), r = t - a * ((unsigned)(Nx - 2) * Nz);
-        rl = a ? Ny : 1;
-        ri = (int)(r / Nz) + 2;
-        rk = (int)(r % Nz) + 1;
-    } else {                                         /* rk in {1, Nz} */
-        t -= fy;
-        const unsigned a = t / ((unsigned)(Nx - 2) * (Ny - 2)),
-                       r = t - a * ((unsigned)(Nx - 2) * (Ny - 2));
-        rk = a ? Nz : 1;
-        ri = (int)(r / (Ny - 2)) + 2;
-        rl = (int)(r % (Ny - 2)) + 2;
-    }
-    const unsigned sy = (unsigned)g.sy, sx = (unsigned)g.sx;
-    const int px = ri == Nx ? 0 : ri == 1 ? Nx + 1 : -1;
-    const int py = rl == Ny ? 0 : rl == 1 ? Ny + 1 : -1;
-    const int pz = rk == Nz ? 0 : rk == 1 ? Nz + 1 : -1;
-    const int X[2] = {ri, px}, Y[2] = {rl, py}, Z[2] = {rk, pz};
-    auto member = [&](int s) {
-        return ((s & 1) == 0 || px >= 0) && ((s & 2) == 0 || py >= 0) && ((s & 4) == 0 || pz >= 0);
-    };
-    unsigned m[8];
-#pragma unroll
-    for (int s = 0; s < 8; s++)
-        m[s] = (unsigned)X[s & 1] * sx + (unsigned)Y[(s >> 1) & 1] * sy + (unsigned)Z[s >> 2];
-    for (int cc = 0; cc < 3; cc++) {
-        JT *J = f.J[cc];
-        JT v[8];
-#pragma unroll
-        for (int s = 0; s < 8; s++) v[s] = member(s) ? J[m[s]] : (JT)0;
-        if (px >= 0) {
-#pragma unroll
-            for (int s = 0; s < 8; s += 2)
-                if (member(s)) fold_pair(v[s], v[s | 1], 0, cc, ri == Nx);
-        }
-        if (py >= 0) {
-#pragma unroll
-            for (int s = 0; s < 8; s++)
-                if (!(s & 2) && member(s)) fold_pair(v[s], v[s | 2], 1, cc, rl == Ny);
-        }
-        if (pz >= 0) {
-#pragma unroll
-            for (int s = 0; s < 4; s++)
-                if (member(s)) fold_pair(v[s], v[s | 4], 2, cc, rk == Nz);
-        }
-#pragma unroll
-        for (int s = 0; s < 8; s++)
-            if (member(s)) J[m[s]] = v[s];
-    }
 }
 
 /* The step's field update after the current fold in one pass:
@@ -467,10 +371,24 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_fold_j(Grid g, FV<T, JT> f, int d
 /* getElectricEnergy (gpu_plasma.h:621-657) -> GPU_getCellEnergy
  * (wrap_kernel.cu:14-36): sum over every ghosted node of Ex^2+Ey^2+Ez^2,
  * accumulated in FP64 by a deterministic two-level tree instead of
- * one-address atomics. */
+ * one-address atomics.  The workgroup that finishes last adds up the
+ * partials and puts the energy, and the step's status where asked for, into
+ * pinned host memory: as a launch and two copies of their own these took
+ * about 15 us of a small step. */
+__device__ __forceinline__ double block_tree(double *red, double s) {
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int w = PIC_BLOCK / 2; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+        __syncthreads();
+    }
+    return red[0];
+}
+
 template <typename T, typename JT>
-__global__ __launch_bounds__(PIC_BLOCK) void k_energy(Grid g, FV<T, JT> f, double *partials) {
+__global__ __launch_bounds__(PIC_BLOCK) void k_energy(Grid g, FV<T, JT> f, EnergyOut o) {
     __shared__ double red[PIC_BLOCK];
+    __shared__ bool last;
     const T *ex = f.E[0], *ey = f.E[1], *ez = f.E[2];
     double s = 0.0;
     for (long n = (long)blockIdx.x * PIC_BLOCK + threadIdx.x; n < g.G;
@@ -478,27 +396,25 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_energy(Grid g, FV<T, JT> f, doubl
         double a = (double)ex[n], b = (double)ey[n], c = (double)ez[n];
         s += a * a + b * b + c * c;
     }
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = PIC_BLOCK / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
+    const double part = block_tree(red, s);
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(&o.partials[blockIdx.x], part, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+        /* the partial is released with the count and acquired by the last */
+        last = __hip_atomic_fetch_add(o.done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
+               gridDim.x - 1;
     }
-    if (threadIdx.x == 0) partials[blockIdx.x] = red[0];
-}
-
-__global__ __launch_bounds__(PIC_BLOCK) void k_reduce_final(const double *partials, int n,
-                                                            double *out) {
-    __shared__ double red[PIC_BLOCK];
-    double s = 0.0;
-    for (int j = threadIdx.x; j < n; j += PIC_BLOCK) s += partials[j];
-    red[threadIdx.x] = s;
     __syncthreads();
-    for (int w = PIC_BLOCK / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
+    if (!last) return;
+    s = 0.0;
+    for (int j = threadIdx.x; j < (int)gridDim.x; j += PIC_BLOCK)
+        s += __hip_atomic_load(&o.partials[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const double total = block_tree(red, s);
+    if (threadIdx.x == 0) {
+        *o.done = 0;
+        *o.h_energy = total;
+        if (o.st) *o.h_st = *o.st;
     }
-    if (threadIdx.x == 0) *out = red[0];
 }
 
 __global__ void k_reset_status(DevStatus *st) {
@@ -512,18 +428,16 @@ __global__ void k_reset_status(DevStatus *st) {
 inline unsigned blocks_for(long n) { return (unsigned)((n + PIC_BLOCK - 1) / PIC_BLOCK); }
 
 template <typename T, typename JT>
-void h_half(const Grid &g, FV<T, JT> f, hipStream_t s) {
+void h_half(const Grid &g, FV<T, JT> f, DevStatus *reset, hipStream_t s) {
     hipLaunchKernelGGL((k_h_half<T, JT>), dim3(blocks_for(g.G)), dim3(PIC_BLOCK), 0, s, g, f,
+                       yee_coef<T>(g), reset);
+}
+template <typename T, typename JT>
+void h2_e(const Grid &g, FV<T, JT> f, HOut<T> out, hipStream_t s) {
+    hipLaunchKernelGGL((k_h2_e<T, JT>), dim3(blocks_for(g.G)), dim3(PIC_BLOCK), 0, s, g, f, out,
                        yee_coef<T>(g));
 }
 template <typename T, typename JT>
-void fold_h2_e(const Grid &g, FV<T, JT> f, HOut<T> out, hipStream_t s) {
-    const long shell = 2L * g.Ny * g.Nz + 2L * (g.Nx - 2) * g.Nz + 2L * (g.Nx - 2) * (g.Ny - 2);
-    hipLaunchKernelGGL((k_fold_j_classes<T, JT>), dim3(blocks_for(shell)), dim3(PIC_BLOCK), 0, s,
-                       g, f);
-    hipLaunchKernelGGL((k_h2_e<T, JT>), dim3(blocks_for(g.G)), dim3(PIC_BLOCK), 0, s, g, f, out,
-                       yee_coef<T>(g));
-}template <typename T, typename JT>
 void h2(const Grid &g, FV<T, JT> f, hipStream_t s) {
     hipLaunchKernelGGL((k_h2<T, JT>), dim3(blocks_for(g.G)), dim3(PIC_BLOCK), 0, s, g, f);
 }
@@ -550,44 +464,43 @@ void fold_j(const Grid &g, FV<T, JT> f, hipStream_t s) {
                            g, f, dir);
 }
 template <typename T, typename JT>
-void energy(const Grid &g, FV<T, JT> f, double *partials, int nblocks, double *out,
-            hipStream_t s) {
-    hipLaunchKernelGGL((k_energy<T, JT>), dim3(nblocks), dim3(PIC_BLOCK), 0, s, g, f, partials);
-    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(PIC_BLOCK), 0, s, partials, nblocks, out);
+void energy(const Grid &g, FV<T, JT> f, const EnergyOut &o, int nblocks, hipStream_t s) {
+    /* (workgroups past the nodes would add exact zeros) */
+    const unsigned nb = std::min((unsigned)nblocks, blocks_for(g.G));
+    hipLaunchKernelGGL((k_energy<T, JT>), dim3(nb), dim3(PIC_BLOCK), 0, s, g, f, o);
 }
 
 }  // namespace
 
-void launch_h_half(const Grid &g, FieldPtrs f, hipStream_t s) { h_half(g, view(f), s); }
+void launch_h_half(const Grid &g, FieldPtrs f, DevStatus *reset, hipStream_t s) {
+    h_half(g, view(f), reset, s);
+}
 void launch_h2(const Grid &g, FieldPtrs f, hipStream_t s) { h2(g, view(f), s); }
 void launch_e(const Grid &g, FieldPtrs f, hipStream_t s) { e_update(g, view(f), s); }
 void launch_e_periodic(const Grid &g, FieldPtrs f, hipStream_t s) { e_periodic(g, view(f), s); }
 void launch_fold_j(const Grid &g, FieldPtrs f, hipStream_t s) { fold_j(g, view(f), s); }
-void launch_energy(const Grid &g, FieldPtrs f, double *partials, int nblocks, double *out,
-                   hipStream_t s) {
-    energy(g, view(f), partials, nblocks, out, s);
+void launch_energy(const Grid &g, FieldPtrs f, const EnergyOut &o, int nblocks, hipStream_t s) {
+    energy(g, view(f), o, nblocks, s);
 }
 
-void launch_h_half32(const Grid &g, FieldPtrs32 f, hipStream_t s) { h_half(g, view(f), s); }
+void launch_h_half32(const Grid &g, FieldPtrs32 f, DevStatus *reset, hipStream_t s) {
+    h_half(g, view(f), reset, s);
+}
 void launch_h2_32(const Grid &g, FieldPtrs32 f, hipStream_t s) { h2(g, view(f), s); }
 void launch_e32(const Grid &g, FieldPtrs32 f, hipStream_t s) { e_update(g, view(f), s); }
 void launch_e_periodic32(const Grid &g, FieldPtrs32 f, hipStream_t s) {
     e_periodic(g, view(f), s);
 }
 void launch_fold_j32(const Grid &g, FieldPtrs32 f, hipStream_t s) { fold_j(g, view(f), s); }
-void launch_energy32(const Grid &g, FieldPtrs32 f, double *partials, int nblocks, double *out,
-                     hipStream_t s) {
-    energy(g, view(f), partials, nblocks, out, s);
+void launch_energy32(const Grid &g, FieldPtrs32 f, const EnergyOut &o, int nblocks, hipStream_t s) {
+    energy(g, view(f), o, nblocks, s);
 }
 
-void launch_fold_h2_e(const Grid &g, FieldPtrs f, double *const h_out[3], hipStream_t s) {
-    fold_h2_e(g, view(f), HOut<double>{{h_out[0], h_out[1], h_out[2]}}, s);
+void launch_h2_e(const Grid &g, FieldPtrs f, double *const h_out[3], hipStream_t s) {
+    h2_e(g, view(f), HOut<double>{{h_out[0], h_out[1], h_out[2]}}, s);
 }
-void launch_fold_h2_e32(const Grid &g, FieldPtrs32 f, float *const h_out[3], hipStream_t s) {
-    fold_h2_e(g, view(f), HOut<float>{{h_out[0], h_out[1], h_out[2]}}, s);
-}
-void launch_reduce_final(const double *partials, int nblocks, double *out, hipStream_t s) {
-    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(PIC_BLOCK), 0, s, partials, nblocks, out);
+void launch_h2_e32(const Grid &g, FieldPtrs32 f, float *const h_out[3], hipStream_t s) {
+    h2_e(g, view(f), HOut<float>{{h_out[0], h_out[1], h_out[2]}}, s);
 }
 
 void launch_reset_status(DevStatus *st, hipStream_t s) {

@@ -27,6 +27,7 @@
 
 #include "pic_internal.h"
 #include "k_push_math32.h"
+#include "k_fold.h"
 #include "k_queue_key.h"
 
 /* copies of the LDS J box: lane l deposits into copy l % JCOPIES, which
@@ -761,24 +762,33 @@ __device__ __forceinline__ void cell_tile(const Grid &g, const TileGeom &t, long
     lc = ((gi % TX) * TY + gl % TY) * TZ + gk % TZ;
 }
 
-/* after a push, one workgroup per tile: each cell holds its stayers and its
+/* after a push, one wavefront per tile: each cell holds its stayers and its
  * arrivals (a count past the capacity raises PIC_F_BUCKET_OVERFLOW: the host
  * unpacks into larger buckets before the next push), and the tile's spill
  * records move from the unsorted list into the sorted one: cell c's record
  * with arrival index PIC_INBOX + k at the exclusive prefix over the tile's
  * cells of their spill counts, plus k (no atomics: the position follows
- * from the record) */
+ * from the record).  The workgroups behind those of the tiles (arrive_blocks:
+ * all of them, or 0) fold the current. */
 template <int TX, int TY, int TZ>
-__global__ __launch_bounds__(64) void k_arrivals_done32(Grid g, TileGeom t, PartPtrs32 p,
-                                                       Layout32 L, DevStatus *st) {
+__global__ __launch_bounds__(PIC_BLOCK) void k_arrive_fold32(Grid g, TileGeom t, PartPtrs32 p,
+                                                            Layout32 L, DevStatus *st,
+                                                            FoldJ<long long> f,
+                                                            unsigned arrive_blocks) {
     constexpr int C = TX * TY * TZ;
     static_assert(C <= 64, "one wavefront scans the tile's cells");
-    __shared__ int off[C];
-    const long tile = blockIdx.x;
-    const int tz = (int)(tile % t.ntz), ty = (int)((tile / t.ntz) % t.nty),
-              tx = (int)(tile / ((long)t.ntz * t.nty));
-    if (threadIdx.x < 64) {
-        const int c = threadIdx.x;
+    __shared__ int offs[PIC_BLOCK / 64][C];
+    if (blockIdx.x >= arrive_blocks) {
+        fold_class(g, f, (blockIdx.x - arrive_blocks) * PIC_BLOCK + threadIdx.x);
+        return;
+    }
+    const int c = threadIdx.x % 64;
+    int *const off = offs[threadIdx.x / 64];
+    const long tile = (long)blockIdx.x * (PIC_BLOCK / 64) + threadIdx.x / 64;
+    const bool have = tile < t.ntiles;
+    if (have) {
+        const int tz = (int)(tile % t.ntz), ty = (int)((tile / t.ntz) % t.nty),
+                  tx = (int)(tile / ((long)t.ntz * t.nty));
         int nsp = 0;
         bool over = false;
         if (c < C) {
@@ -799,10 +809,11 @@ __global__ __launch_bounds__(64) void k_arrivals_done32(Grid g, TileGeom t, Part
         if (__ballot(over) && c == 0) atomicOr(&st->flags, (unsigned)PIC_F_BUCKET_OVERFLOW);
     }
     __syncthreads();
+    if (!have) return;
     const int n = min(L.spill_u_cnt[tile], L.scap);
     const float4 *const U = L.spill_u + 2 * (tile * (long)L.scap);
     float4 *const S = L.spill_s + 2 * (tile * (long)L.scap);
-    for (int k = threadIdx.x; k < n; k += 64) {
+    for (int k = c; k < n; k += 64) {
         const float4 A = U[2 * k], B = U[2 * k + 1];
         const unsigned key = __float_as_uint(B.z);
         const int lc = key_halo(key);
@@ -813,8 +824,8 @@ __global__ __launch_bounds__(64) void k_arrivals_done32(Grid g, TileGeom t, Part
             S[2 * d + 1] = B;
         }
     }
-    __syncthreads();
-    if (threadIdx.x == 0) L.spill_u_cnt[tile] = 0;
+    /* (every lane of the wavefront holds n before this store) */
+    if (c == 0) L.spill_u_cnt[tile] = 0;
 }
 
 /* the packed live set into buckets of `to` (capacity to.cap >= every
@@ -1068,10 +1079,14 @@ static bool raw_current_sums_exact(const PushArgs32 &a, int cap) {
     return bound < 0.99 * 140737488355328.0;   /* 2^47 */
 }
 
-void launch_arrivals_done32(const Grid &g, const TileGeom &t, PartPtrs32 p, Layout32 L,
-                            DevStatus *st, hipStream_t s) {
-    hipLaunchKernelGGL((k_arrivals_done32<TXC, TYC, TZC>), dim3((unsigned)t.ntiles), dim3(64),
-                       0, s, g, t, p, L, st);
+void launch_arrive_fold_f32(const Grid &g, const TileGeom &t, PartPtrs32 p, Layout32 L,
+                            DevStatus *st, FieldPtrs32 f, int what, hipStream_t s) {
+    constexpr int per = PIC_BLOCK / 64;
+    const unsigned tiles = what & PIC_ARRIVE ? (unsigned)((t.ntiles + per - 1) / per) : 0;
+    const unsigned blocks = tiles + (what & PIC_FOLD ? fold_blocks(g) : 0);
+    const FoldJ<long long> J{{f.J[0], f.J[1], f.J[2]}};
+    hipLaunchKernelGGL((k_arrive_fold32<TXC, TYC, TZC>), dim3(blocks), dim3(PIC_BLOCK), 0, s, g, t,
+                       p, L, st, J, tiles);
 }
 
 void launch_unpack32(const Grid &g, const TileGeom &t, PartPtrs32 p, Layout32 L, PartPtrs32 to,

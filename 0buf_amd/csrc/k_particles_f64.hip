@@ -726,10 +726,13 @@ void launch_jfix_to_f64(const Grid &g, FieldPtrs f, DiffArgs d, hipStream_t s) {
     hipLaunchKernelGGL(k_jfix_to_f64, dim3(blocks_for(g.G)), dim3(PIC_BLOCK), 0, s, g.G, f, d);
 }
 
-void launch_arrive_f64(const Grid &g, const TileGeom &t, PartPtrs p, QueuePtrs q, DevStatus *st,
-                       hipStream_t s) {
-    hipLaunchKernelGGL((k_arrive_tile<TXC, TYC, TZC, PartPtrs, QueuePtrs>), dim3((unsigned)t.ntiles),
-                       dim3(PIC_BLOCK), 0, s, g, t, p, q, st);
+void launch_arrive_fold_f64(const Grid &g, const TileGeom &t, PartPtrs p, QueuePtrs q,
+                            DevStatus *st, FieldPtrs f, int what, hipStream_t s) {
+    const unsigned tiles = what & PIC_ARRIVE ? (unsigned)t.ntiles : 0;
+    const unsigned blocks = tiles + (what & PIC_FOLD ? fold_blocks(g) : 0);
+    const FoldJ<double> J{{f.f[PIC_JX], f.f[PIC_JY], f.f[PIC_JZ]}};
+    hipLaunchKernelGGL((k_arrive_fold<TXC, TYC, TZC, PartPtrs, QueuePtrs, double>), dim3(blocks),
+                       dim3(PIC_BLOCK), 0, s, g, t, p, q, st, J, tiles);
 }
 
 void launch_scatter_load(const long *offsets, long ncell, const double *src[6],

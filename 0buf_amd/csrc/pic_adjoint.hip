@@ -28,14 +28,10 @@
 #include "pic_ctx.h"
 
 namespace picx {
-void enq_h_half(pic_ctx *c);
+void enq_h_half(pic_ctx *c, bool begin_step);
 void enq_push(pic_ctx *c);
-void enq_arrive(pic_ctx *c);
-void enq_fold(pic_ctx *c);
-void enq_h2(pic_ctx *c);
-void enq_e(pic_ctx *c);
-void enq_e_periodic(pic_ctx *c);
-void enq_fold_h2_e(pic_ctx *c);
+void enq_arrive_fold(pic_ctx *c, int what);
+void enq_h2_e(pic_ctx *c);
 }  // namespace picx
 
 using namespace picx;
@@ -217,7 +213,7 @@ int restore_state(pic_ctx *c, const Compact &src, const FieldSet &f) {
 int recorded_step(pic_ctx *c, AdjointStore *s, int r) {
     FieldSet &f = s->recf[r];
     const size_t bytes = c->g.G * elem(c);
-    enq_h_half(c);
+    enq_h_half(c, false);
     const void *src[6];
     for (int k = 0; k < 6; k++) src[k] = live_field(c, k);
     launch_copy6(f.f, src, bytes, c->stream);
@@ -232,7 +228,7 @@ int recorded_step(pic_ctx *c, AdjointStore *s, int r) {
     c->rec_snap32 = PartPtrs32{};
     c->rec_off = nullptr;
     c->rec_room = 0;
-    enq_arrive(c);
+    enq_arrive_fold(c, PIC_ARRIVE | PIC_FOLD);
     if (c->fp32) {
         /* the status is checked at the segment's end; only where the first
          * forward needed the repair of a full spill list is each step's
@@ -249,7 +245,7 @@ int recorded_step(pic_ctx *c, AdjointStore *s, int r) {
             }
         }
     }
-    enq_fold_h2_e(c);
+    enq_h2_e(c);
     HIPCHK(hipGetLastError());
     return PIC_SUCCESS;
 }
@@ -398,7 +394,7 @@ int pic_forward_record(pic_ctx *c, int nsteps, int ckpt_every, double *energy) {
         }
         rc = enq_step(c);
         if (rc) return rc;
-        rc = finish_step(c);
+        rc = finish_step(c, true);
         if (rc) return rc;
         s->anomalies += c->last.dropped + c->last.duplicated;
         if (energy) energy[t] = c->h_red[0];

@@ -481,9 +481,11 @@ int despill(pic_ctx *c) { return unpack_live32(c, true); }
 int *qcount_ptr(pic_ctx *c) { return c->fp32 ? c->q32.count : c->q.count; }
 
 /* stage launchers dispatching on the form */
-void enq_h_half(pic_ctx *c) {
-    if (c->fp32) launch_h_half32(c->g, c->f32, c->stream);
-    else launch_h_half(c->g, c->f, c->stream);
+/* begin_step: the status of a new step starts clear */
+void enq_h_half(pic_ctx *c, bool begin_step) {
+    DevStatus *reset = begin_step ? c->d_st : nullptr;
+    if (c->fp32) launch_h_half32(c->g, c->f32, reset, c->stream);
+    else launch_h_half(c->g, c->f, reset, c->stream);
 }
 void enq_push(pic_ctx *c) {
     if (c->fp32) {
@@ -514,15 +516,17 @@ void enq_push(pic_ctx *c) {
                                 c->d_st, nullptr, c->stream);
     }
 }
-void enq_arrive(pic_ctx *c, hipStream_t st) {
+/* the arrivals of the push, the periodic fold of the current, or both in one
+ * launch (PIC_ARRIVE, PIC_FOLD) */
+void enq_arrive_fold(pic_ctx *c, int what) {
     if (c->fp32) {
         /* the push placed the arrivals; the counts take them in */
-        launch_arrivals_done32(c->g, c->t, c->p32, c->lay32, c->d_st, st);
-        c->arrival_pending = true;
+        launch_arrive_fold_f32(c->g, c->t, c->p32, c->lay32, c->d_st, c->f32, what, c->stream);
+        if (what & PIC_ARRIVE) c->arrival_pending = true;
+    } else {
+        launch_arrive_fold_f64(c->g, c->t, c->p, c->q, c->d_st, c->f, what, c->stream);
     }
-    else launch_arrive_f64(c->g, c->t, c->p, c->q, c->d_st, st);
 }
-void enq_arrive(pic_ctx *c) { enq_arrive(c, c->stream); }
 void enq_fold(pic_ctx *c) {
     if (c->fp32) launch_fold_j32(c->g, c->f32, c->stream);
     else launch_fold_j(c->g, c->f, c->stream);
@@ -539,22 +543,24 @@ void enq_e_periodic(pic_ctx *c) {
     if (c->fp32) launch_e_periodic32(c->g, c->f32, c->stream);
     else launch_e_periodic(c->g, c->f, c->stream);
 }
-/* the step's field update after the push in one pass: current fold, H
- * second half, E update and periodic E ghosts (equal to enq_fold, enq_h2,
- * enq_e, enq_e_periodic bit for bit), H^{n+1} landing in the second H
- * arrays, which then become the live ones */
-void enq_fold_h2_e(pic_ctx *c) {
+/* the step's field update after the current fold in one pass: H second half,
+ * E update and periodic E ghosts (equal to enq_h2, enq_e, enq_e_periodic bit
+ * for bit), H^{n+1} landing in the second H arrays, which then become the
+ * live ones */
+void enq_h2_e(pic_ctx *c) {
     if (c->fp32) {
-        launch_fold_h2_e32(c->g, c->f32, c->h_alt32, c->stream);
+        launch_h2_e32(c->g, c->f32, c->h_alt32, c->stream);
         for (int k = 0; k < 3; k++) std::swap(c->f32.H[k], c->h_alt32[k]);
     } else {
-        launch_fold_h2_e(c->g, c->f, c->h_alt, c->stream);
+        launch_h2_e(c->g, c->f, c->h_alt, c->stream);
         for (int k = 0; k < 3; k++) std::swap(c->f.f[PIC_HX + k], c->h_alt[k]);
     }
 }
-void enq_energy(pic_ctx *c) {
-    if (c->fp32) launch_energy32(c->g, c->f32, c->d_part, c->npart, c->d_red, c->stream);
-    else launch_energy(c->g, c->f, c->d_part, c->npart, c->d_red, c->stream);
+/* the energy into h_red[0], with_status: and the step's status into h_st */
+void enq_energy(pic_ctx *c, bool with_status) {
+    const EnergyOut o{c->d_part, c->d_done, c->h_red, with_status ? c->d_st : nullptr, c->h_st};
+    if (c->fp32) launch_energy32(c->g, c->f32, o, c->npart, c->stream);
+    else launch_energy(c->g, c->f, o, c->npart, c->stream);
 }
 
 int check_ready(pic_ctx *c) {
@@ -590,41 +596,35 @@ void accumulate_profile(pic_ctx *c) {
 }
 
 /* one whole step enqueued on the context stream (Plasma::Step,
- * gpu_plasma.h:605-620); the energy lands in h_red[0] after the sync */
+ * gpu_plasma.h:605-620) in five launches; the energy and the status land in
+ * h_red[0] and h_st by the time the stream is done */
 int enq_step(pic_ctx *c) {
-    launch_reset_status(c->d_st, c->stream);
     mark(c, PIC_STAGE_H_HALF);
-    enq_h_half(c);
+    enq_h_half(c, true);
     mark(c, PIC_STAGE_PUSH_DEPOSIT);
     enq_push(c);
     mark(c, PIC_STAGE_MIGRATE);
-    /* the arrival (particles only) beside the field stages (fields only);
-     * with stage timing on, one after the other so that each stage's events
-     * bracket its own kernels */
-    const bool overlap = c->side && !c->prof;
-    if (overlap) {
-        HIPCHK(hipEventRecord(c->ev_dep, c->stream));
-        HIPCHK(hipStreamWaitEvent(c->side, c->ev_dep, 0));
-        enq_arrive(c, c->side);
-        HIPCHK(hipEventRecord(c->ev_join, c->side));
-    } else {
-        enq_arrive(c, c->stream);
-    }
-    /* current fold, H second half, E update and the periodic E ghosts in
-     * one pass: its time is the E stage's (FOLD_J, H2, E_PERIODIC: 0) */
+    /* with stage timing on, the arrival and the fold are launched apart, so
+     * that each stage's events bracket its own kernels; the fold, H second
+     * half, E update and periodic E ghosts are the E stage's (FOLD_J, H2,
+     * E_PERIODIC: 0) */
+    enq_arrive_fold(c, c->prof ? PIC_ARRIVE : PIC_ARRIVE | PIC_FOLD);
     mark(c, PIC_STAGE_E);
-    enq_fold_h2_e(c);
+    if (c->prof) enq_arrive_fold(c, PIC_FOLD);
+    enq_h2_e(c);
     mark(c, PIC_STAGE_ENERGY);
-    enq_energy(c);
+    enq_energy(c, true);
     mark(c, PIC_NSTAGES);
-    if (overlap) HIPCHK(hipStreamWaitEvent(c->stream, c->ev_join, 0));
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(c->h_red, c->d_red, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     return PIC_SUCCESS;
 }
 
-int finish_step(pic_ctx *c) {
-    HIPCHK(hipMemcpyAsync(c->h_st, c->d_st, sizeof(DevStatus), hipMemcpyDeviceToHost, c->stream));
+/* waits for the stream and examines the status of what ran; have_status: a
+ * whole step left it in h_st */
+int finish_step(pic_ctx *c, bool have_status) {
+    if (!have_status)
+        HIPCHK(hipMemcpyAsync(c->h_st, c->d_st, sizeof(DevStatus), hipMemcpyDeviceToHost,
+                              c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     const DevStatus st = *c->h_st;
     const bool arrived = c->arrival_pending;
@@ -777,13 +777,6 @@ int pic_create(const pic_params *prm, pic_ctx **out) {
     };
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
     if (e != hipSuccess) return fail(record_hip(e, "hipStreamCreate"));
-    /* both streams at the default priority */
-    e = hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking);
-    if (e != hipSuccess) return fail(record_hip(e, "hipStreamCreate"));
-    e = hipEventCreateWithFlags(&c->ev_dep, hipEventDisableTiming);
-    if (e != hipSuccess) return fail(record_hip(e, "hipEventCreate"));
-    e = hipEventCreate(&c->ev_join);
-    if (e != hipSuccess) return fail(record_hip(e, "hipEventCreate"));
     c->fp32 = prm->precision == PIC_FP32;
     for (int k = 0; k < PIC_NFIELDS; k++) {
         void **ptr;
@@ -822,6 +815,10 @@ int pic_create(const pic_params *prm, pic_ctx **out) {
     if ((e = hipMemset(c->d_st, 0, sizeof(DevStatus))) != hipSuccess) return fail(record_hip(e, "status"));
     if ((e = hipHostMalloc(&c->h_st, sizeof(DevStatus))) != hipSuccess) return fail(record_hip(e, "status"));
     if ((e = hipMalloc(&c->d_part, (size_t)c->npart * 27 * sizeof(double))) != hipSuccess)
+        return fail(record_hip(e, "partials"));
+    if ((e = hipMalloc(&c->d_done, sizeof(unsigned))) != hipSuccess)
+        return fail(record_hip(e, "partials"));
+    if ((e = hipMemset(c->d_done, 0, sizeof(unsigned))) != hipSuccess)
         return fail(record_hip(e, "partials"));
     if ((e = hipMalloc(&c->d_red, 64 * sizeof(double))) != hipSuccess) return fail(record_hip(e, "red"));
     if ((e = hipHostMalloc(&c->h_red, 64 * sizeof(double))) != hipSuccess) return fail(record_hip(e, "red"));
@@ -864,15 +861,13 @@ int pic_destroy(pic_ctx *c) {
     if (c->d_st) hipFree(c->d_st);
     if (c->h_st) hipHostFree(c->h_st);
     if (c->d_part) hipFree(c->d_part);
+    if (c->d_done) hipFree(c->d_done);
     if (c->d_red) hipFree(c->d_red);
     if (c->h_red) hipHostFree(c->h_red);
     if (c->d_slot_sort) hipFree(c->d_slot_sort);
     if (c->d_tape) hipFree(c->d_tape);
     for (int k = 0; k <= PIC_NSTAGES; k++)
         if (c->ev[k]) hipEventDestroy(c->ev[k]);
-    if (c->ev_dep) hipEventDestroy(c->ev_dep);
-    if (c->ev_join) hipEventDestroy(c->ev_join);
-    if (c->side) hipStreamDestroy(c->side);
     if (c->stream) hipStreamDestroy(c->stream);
     delete c;
     return PIC_SUCCESS;
@@ -1080,8 +1075,7 @@ int pic_get_field(pic_ctx *c, int which, double *host) {
 int pic_yee_h_half(pic_ctx *c) {
     int rc = check_ready(c);
     if (rc) return rc;
-    launch_reset_status(c->d_st, c->stream);
-    enq_h_half(c);
+    enq_h_half(c, true);
     HIPCHK(hipGetLastError());
     return PIC_SUCCESS;
 }
@@ -1100,7 +1094,7 @@ int pic_push_deposit(pic_ctx *c) {
 int pic_migrate(pic_ctx *c) {
     int rc = check_ready(c);
     if (rc) return rc;
-    enq_arrive(c);
+    enq_arrive_fold(c, PIC_ARRIVE);
     HIPCHK(hipGetLastError());
     return PIC_SUCCESS;
 }
@@ -1135,9 +1129,8 @@ int pic_e_periodic(pic_ctx *c) {
 
 int pic_energy(pic_ctx *c, double *energy) {
     if (!c) return PIC_ERR_INVALID;
-    enq_energy(c);
+    enq_energy(c, false);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(c->h_red, c->d_red, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     if (energy) *energy = c->h_red[0];
     return PIC_SUCCESS;
@@ -1157,7 +1150,7 @@ int pic_step(pic_ctx *c, int nt, double *energy) {
     if (c->arrival_pending && (rc = finish_step(c))) return rc;
     rc = enq_step(c);
     if (rc) return rc;
-    rc = finish_step(c);
+    rc = finish_step(c, true);
     accumulate_profile(c);
     if (energy) *energy = c->h_red[0];
     return rc;

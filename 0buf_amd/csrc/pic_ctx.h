@@ -32,12 +32,6 @@ struct pic_ctx {
     long NC = 0;
     int dev = 0;
     hipStream_t stream = nullptr;
-    /* a step runs the arrival on `side` while the field stages run on
-     * `stream` (the two touch disjoint data); ev_dep orders it after the
-     * push, ev_join joins it before the step's end.  With stage timing on,
-     * the step stays on `stream` alone. */
-    hipStream_t side = nullptr;
-    hipEvent_t ev_dep = nullptr, ev_join = nullptr;
     bool fp32 = false;
     FieldPtrs f{};          /* FP64 plain form */
     PartPtrs p{};
@@ -82,6 +76,7 @@ struct pic_ctx {
     DevStatus *h_st = nullptr;
     double *d_part = nullptr;
     int npart = 1024;
+    unsigned *d_done = nullptr;   /* workgroups done with the energy reduction */
     double *d_red = nullptr;
     double *h_red = nullptr;
     Staged staged;
@@ -107,7 +102,7 @@ int record_hip(hipError_t e, const char *where);
 int commit(pic_ctx *c);
 int check_ready(pic_ctx *c);
 int enq_step(pic_ctx *c);
-int finish_step(pic_ctx *c);
+int finish_step(pic_ctx *c, bool have_status = false);
 /* FP32 form: put every particle into the bucket arrays (unpack the packed
  * set with its pending arrivals) before anything other than the push reads
  * the buckets (no-op otherwise); examines a pending arrival's status first */

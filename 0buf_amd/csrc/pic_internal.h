@@ -378,29 +378,34 @@ inline int push_threads(long ntiles) {
 }
 
 /* kernel launchers (k_fields.hip) */
-/* the step's fused pass after the push: the current fold, H^{n+1} into
- * h_out (the second H arrays; the caller swaps them with the live ones), the
- * E update and the periodic E ghosts, equal to launch_fold_j, launch_h2,
- * launch_e, launch_e_periodic bit for bit */
-void launch_fold_h2_e(const Grid &g, FieldPtrs f, double *const h_out[3], hipStream_t s);
-void launch_fold_h2_e32(const Grid &g, FieldPtrs32 f, float *const h_out[3], hipStream_t s);
-/* sum of nblocks partials into *out (deterministic tree) */
-void launch_reduce_final(const double *partials, int nblocks, double *out, hipStream_t s);
-void launch_h_half(const Grid &g, FieldPtrs f, hipStream_t s);
+/* the step's field update after the current fold: H^{n+1} into h_out (the
+ * second H arrays; the caller swaps them with the live ones), the E update
+ * and the periodic E ghosts, equal to launch_h2, launch_e,
+ * launch_e_periodic bit for bit */
+void launch_h2_e(const Grid &g, FieldPtrs f, double *const h_out[3], hipStream_t s);
+void launch_h2_e32(const Grid &g, FieldPtrs32 f, float *const h_out[3], hipStream_t s);
+/* where an energy reduction leaves its result */
+struct EnergyOut {
+    double *partials;        /* one per workgroup */
+    unsigned *done;          /* workgroups done, 0 between launches */
+    double *h_energy;        /* pinned host memory */
+    const DevStatus *st;     /* the step's status, copied to h_st (null: not) */
+    DevStatus *h_st;         /* pinned host memory */
+};
+/* reset (may be null): the status to clear for the step that begins */
+void launch_h_half(const Grid &g, FieldPtrs f, DevStatus *reset, hipStream_t s);
 void launch_h2(const Grid &g, FieldPtrs f, hipStream_t s);
 void launch_e(const Grid &g, FieldPtrs f, hipStream_t s);
 void launch_e_periodic(const Grid &g, FieldPtrs f, hipStream_t s);
 void launch_fold_j(const Grid &g, FieldPtrs f, hipStream_t s);
-void launch_energy(const Grid &g, FieldPtrs f, double *partials, int nblocks, double *out,
-                   hipStream_t s);
+void launch_energy(const Grid &g, FieldPtrs f, const EnergyOut &o, int nblocks, hipStream_t s);
 void launch_reset_status(DevStatus *st, hipStream_t s);
-void launch_h_half32(const Grid &g, FieldPtrs32 f, hipStream_t s);
+void launch_h_half32(const Grid &g, FieldPtrs32 f, DevStatus *reset, hipStream_t s);
 void launch_h2_32(const Grid &g, FieldPtrs32 f, hipStream_t s);
 void launch_e32(const Grid &g, FieldPtrs32 f, hipStream_t s);
 void launch_e_periodic32(const Grid &g, FieldPtrs32 f, hipStream_t s);
 void launch_fold_j32(const Grid &g, FieldPtrs32 f, hipStream_t s);
-void launch_energy32(const Grid &g, FieldPtrs32 f, double *partials, int nblocks, double *out,
-                     hipStream_t s);
+void launch_energy32(const Grid &g, FieldPtrs32 f, const EnergyOut &o, int nblocks, hipStream_t s);
 TileGeom make_tile_geom(int Nx, int Ny, int Nz);
 
 /* Differentiable form of the FP64 step: the push deposits J as int64 fixed
@@ -433,8 +438,11 @@ void launch_jfix_to_f64(const Grid &g, FieldPtrs f, DiffArgs d, hipStream_t s);
 void launch_copy6(void *const dst[6], const void *const src[6], size_t bytes, hipStream_t s);
 void launch_record_offsets(const Grid &g, const TileGeom &t, const int *count, int cap,
                            long *tile_sum, long *off, long room, DevStatus *st, hipStream_t s);
-void launch_arrive_f64(const Grid &g, const TileGeom &t, PartPtrs p, QueuePtrs q, DevStatus *st,
-                       hipStream_t s);
+/* the arrivals of a push and the periodic fold of the current, in one launch,
+ * or one of the two */
+enum { PIC_ARRIVE = 1, PIC_FOLD = 2 };
+void launch_arrive_fold_f64(const Grid &g, const TileGeom &t, PartPtrs p, QueuePtrs q,
+                            DevStatus *st, FieldPtrs f, int what, hipStream_t s);
 void launch_scatter_load(const long *offsets, long ncell, const double *src[6],
                          const unsigned char *srcsp, PartPtrs p, hipStream_t s);
 void launch_repack(long ncell, PartPtrs from, PartPtrs to, hipStream_t s);
@@ -455,9 +463,10 @@ void launch_push_deposit_f32(const Grid &g, const TileGeom &t, FieldPtrs32 f, Pa
                              int dep_cap, DevStatus *st, const PartPtrs32 *diff,
                              const long *snap_off, long snap_room, hipStream_t s);
 /* after the push, per tile: count = bcount + arrivals (PIC_F_BUCKET_OVERFLOW
- * past cap) and the spill records sorted by cell */
-void launch_arrivals_done32(const Grid &g, const TileGeom &t, PartPtrs32 p, Layout32 L,
-                            DevStatus *st, hipStream_t s);
+ * past cap) and the spill records sorted by cell; and the periodic fold of
+ * the current, in one launch, or one of the two (PIC_ARRIVE, PIC_FOLD) */
+void launch_arrive_fold_f32(const Grid &g, const TileGeom &t, PartPtrs32 p, Layout32 L,
+                            DevStatus *st, FieldPtrs32 f, int what, hipStream_t s);
 /* the packed live set p, its inbox records and its arrivals past the inbox
  * (from the spill lists, or from the departure queues of the last push when
  * from_queue is set: the repair after a full spill list) into buckets of
