@@ -4,16 +4,17 @@
  * Cell::Insert, kernels.cu:316-370), where each leaver joins the bucket of
  * the cell that accepts it.
  *
- * One workgroup per source tile.  Its queue entries carry the destination
- * cell twice: as a bulk cell index (dest) and as an index into the tile's
- * halo box of (TX+2) x (TY+2) x (TZ+2) cells (halo).  Entries bound for the
- * same cell are counted in LDS first, so each destination cell costs one
- * global atomic per source tile instead of one per particle (the beam axis of
- * a skewed workload sends tens of particles per step into the same cells);
- * then every entry takes base + rank as its slot.  A slot past the bucket
- * capacity is kept in q.slot for the regrow path and raises
- * PIC_F_BUCKET_OVERFLOW.  An entry whose halo index or destination cell lies
- * out of range is not placed (slot -1) and raises PIC_F_QUEUE_CORRUPT.
+ * One workgroup per source tile, a leaver per thread, in rounds of PIC_BLOCK.
+ * A record carries the destination cell twice: as a bulk cell index (dest)
+ * and as an index into the tile's halo box of (TX+2) x (TY+2) x (TZ+2) cells.
+ * Leavers bound for the same cell are counted in LDS first, so each
+ * destination cell costs one global atomic per round instead of one per
+ * particle (the beam axis of a skewed workload sends tens of particles per
+ * step into the same cells); then every leaver takes base + rank as its slot.
+ * A slot past the bucket capacity is kept in the record for the regrow path
+ * and raises PIC_F_BUCKET_OVERFLOW.  A record whose halo index or destination
+ * cell lies out of range is not placed and raises PIC_F_QUEUE_CORRUPT.  Bound
+ * by its scattered writes, seven arrays per arrival.
  */
 #ifndef K_ARRIVE_H
 #define K_ARRIVE_H
@@ -24,10 +25,10 @@
 
 /* workgroups [0, tiles): the arrivals of one tile each (tiles: all, or 0);
  * those behind them: the periodic fold of the current */
-template <int TX, int TY, int TZ, class P, class Q, class JT>
-__global__ __launch_bounds__(PIC_BLOCK) void k_arrive_fold(Grid g, TileGeom t, P p, Q q,
-                                                           DevStatus *st, FoldJ<JT> f,
-                                                           unsigned tiles) {
+template <int TX, int TY, int TZ, class JT>
+__global__ __launch_bounds__(PIC_BLOCK) void k_arrive_fold(Grid g, TileGeom t, PartPtrs p,
+                                                           QueuePtrs q, DevStatus *st,
+                                                           FoldJ<JT> f, unsigned tiles) {
     if (blockIdx.x >= tiles) {
         fold_class(g, f, (blockIdx.x - tiles) * PIC_BLOCK + threadIdx.x);
         return;
@@ -42,49 +43,58 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_arrive_fold(Grid g, TileGeom t, P
     const int tx = (int)(tile / ((long)t.ntz * t.nty));
     int n = q.count[tile];
     n = n < q.qcap ? n : q.qcap;
-    const long qb = tile * (long)q.qcap;
-    for (int h = tid; h < NH; h += PIC_BLOCK) hcnt[h] = 0;
-    __syncthreads();
-    /* rank of each entry among the tile's entries for the same cell; an
-     * entry whose halo index or cell lies out of range is refused (slot -1) */
+    Leaver64 *const Q = q.e + tile * (long)q.qcap;
     const long ncell = (long)g.Nx * g.Ny * g.Nz;
-    bool bad = false;
-    for (int j = tid; j < n; j += PIC_BLOCK) {
-        const int h = q.halo[qb + j];
-        if (!arrival_entry_ok(h, NH, (long)q.dest[qb + j], ncell)) {
-            q.slot[qb + j] = -1;
-            bad = true;
-            continue;
+    bool bad = false, over = false;
+    for (int j0 = 0; j0 < n; j0 += PIC_BLOCK) {
+        const int j = j0 + tid;
+        Leaver64 r;
+        int h = -1, rank = 0;
+        if (j < n) r = Q[j];
+        for (int k = tid; k < NH; k += PIC_BLOCK) hcnt[k] = 0;
+        __syncthreads();
+        /* rank of each leaver among the round's leavers for the same cell; a
+         * record whose halo index or cell lies out of range is refused */
+        if (j < n) {
+            h = r.where >> 8;
+            if (arrival_entry_ok(h, NH, (long)r.dest, ncell)) {
+                rank = atomicAdd(&hcnt[h], 1);
+            } else {
+                h = -1;
+                bad = true;
+            }
         }
-        q.slot[qb + j] = atomicAdd(&hcnt[h], 1);
-    }
-    __syncthreads();
-    /* one claim per destination cell on its bucket count */
-    for (int h = tid; h < NH; h += PIC_BLOCK) {
-        const int c = hcnt[h];
-        if (c == 0) continue;
-        int gx = tx * TX - 1 + h / (BY * BZ), gy = ty * TY - 1 + (h / BZ) % BY,
-            gz = tz * TZ - 1 + h % BZ;
-        if (gx < 0) gx += g.Nx; else if (gx >= g.Nx) gx -= g.Nx;
-        if (gy < 0) gy += g.Ny; else if (gy >= g.Ny) gy -= g.Ny;
-        if (gz < 0) gz += g.Nz; else if (gz >= g.Nz) gz -= g.Nz;
-        hbase[h] = atomicAdd(&p.count[((long)gx * g.Ny + gy) * g.Nz + gz], c);
-    }
-    __syncthreads();
-    bool over = false;
-    for (int j = tid; j < n; j += PIC_BLOCK) {
-        const long e = qb + j;
-        if (q.slot[e] < 0) continue;
-        const int slot = hbase[q.halo[e]] + q.slot[e];
-        q.slot[e] = slot;
-        if (slot >= p.cap) {
-            over = true;
-            continue;
+        __syncthreads();
+        /* one claim per destination cell on its bucket count */
+        for (int k = tid; k < NH; k += PIC_BLOCK) {
+            const int c = hcnt[k];
+            if (c == 0) continue;
+            int gx = tx * TX - 1 + k / (BY * BZ), gy = ty * TY - 1 + (k / BZ) % BY,
+                gz = tz * TZ - 1 + k % BZ;
+            if (gx < 0) gx += g.Nx; else if (gx >= g.Nx) gx -= g.Nx;
+            if (gy < 0) gy += g.Ny; else if (gy >= g.Ny) gy -= g.Ny;
+            if (gz < 0) gz += g.Nz; else if (gz >= g.Nz) gz -= g.Nz;
+            hbase[k] = atomicAdd(&p.count[((long)gx * g.Ny + gy) * g.Nz + gz], c);
         }
-        const long to = (long)q.dest[e] * p.cap + slot;
-        for (int k = 0; k < 6; k++) p.p[k][to] = q.q[k][e];
-        p.sp[to] = q.sp[e];
-        if (p.id) p.id[to] = q.id[e];
+        __syncthreads();
+        if (h >= 0) {
+            const int slot = hbase[h] + rank;
+            if (slot >= p.cap) {
+                Q[j].slot = slot;
+                over = true;
+            } else {
+                const long to = (long)r.dest * p.cap + slot;
+                p.p[0][to] = r.xy.x;
+                p.p[1][to] = r.xy.y;
+                p.p[2][to] = r.zu.x;
+                p.p[3][to] = r.zu.y;
+                p.p[4][to] = r.vw.x;
+                p.p[5][to] = r.vw.y;
+                p.sp[to] = (unsigned char)(r.where & 255);
+                if (p.id) p.id[to] = r.id;
+            }
+        }
+        __syncthreads();   /* the counts and claims are read above */
     }
     if (over) atomicOr(&st->flags, (unsigned)PIC_F_BUCKET_OVERFLOW);
     if (bad) atomicOr(&st->flags, (unsigned)PIC_F_QUEUE_CORRUPT);

@@ -226,6 +226,7 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
                   *const P4 = a.p.p[4] + pbase, *const P5 = a.p.p[5] + pbase;
     unsigned char *const SP = a.p.sp + pbase;
     int *const ID = DIFF ? a.p.id + pbase : nullptr;
+    Leaver64 *const QT = a.q.e + tile * (long)a.q.qcap;   /* the tile's departure queue */
 
     const double hx = g.hx, hy = g.hy, hz = g.hz, tau = g.tau;
     unsigned bad = 0;
@@ -458,37 +459,38 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
                 if (ncopy == 0) atomicAdd(&sDrop, 1ull);
                 if (ncopy > 1) atomicAdd(&sDup, (unsigned long long)(ncopy - 1));
                 if (ncopy > 0) {
-                    int slot = atomicAdd(&sQ, ncopy);
-                    const long qb = tile * (long)a.q.qcap;
-                    int kq = 0;
-                    /* receivers in the reference's scan order (x, then y, then z) */
-                    for (int ax = 0; ax < 3; ax++) {
-                        if (!((bx >> ax) & 1u)) continue;
-                        int rx = gi + ax - 1;
+                    const int first = atomicAdd(&sQ, ncopy);
+                    /* the record of receiver (ax, ay, az): axis offsets 0..2 */
+                    auto queue = [&](int ax, int ay, int az, int idx) {
+                        if (idx >= a.q.qcap) return;
+                        int rx = gi + ax - 1, ry = gl + ay - 1, rz = gk + az - 1;
                         if (rx >= g.Nx) rx -= g.Nx; else if (rx < 0) rx += g.Nx;
-                        for (int ay = 0; ay < 3; ay++) {
-                            if (!((by >> ay) & 1u)) continue;
-                            int ry = gl + ay - 1;
-                            if (ry >= g.Ny) ry -= g.Ny; else if (ry < 0) ry += g.Ny;
-                            for (int az = 0; az < 3; az++) {
-                                if (!((bz >> az) & 1u)) continue;
-                                int rz = gk + az - 1;
-                                if (rz >= g.Nz) rz -= g.Nz; else if (rz < 0) rz += g.Nz;
-                                const int idx = slot + kq++;
-                                if (idx >= a.q.qcap) continue;
-                                const long e = qb + idx;
-                                a.q.q[0][e] = xn;
-                                a.q.q[1][e] = yn;
-                                a.q.q[2][e] = zn;
-                                a.q.q[3][e] = pu;
-                                a.q.q[4][e] = pv;
-                                a.q.q[5][e] = pw;
-                                a.q.sp[e] = s;
-                                if (DIFF) a.q.id[e] = pid;
-                                a.q.dest[e] = (int)(((long)rx * g.Ny + ry) * g.Nz + rz);
-                                a.q.halo[e] = (unsigned char)(((G.ca + ax) * BY + (G.cb + ay)) * BZ +
-                                                              (G.cc + az));
-                            }
+                        if (ry >= g.Ny) ry -= g.Ny; else if (ry < 0) ry += g.Ny;
+                        if (rz >= g.Nz) rz -= g.Nz; else if (rz < 0) rz += g.Nz;
+                        const int h = ((G.ca + ax) * BY + (G.cb + ay)) * BZ + (G.cc + az);
+                        Leaver64 &e = slot(QT, (unsigned)idx);
+                        e.xy = make_double2(xn, yn);
+                        e.zu = make_double2(zn, pu);
+                        e.vw = make_double2(pv, pw);
+                        *(int4 *)&e.dest =
+                            make_int4((rx * g.Ny + ry) * g.Nz + rz, (int)s | h << 8, pid, -1);
+                    };
+                    /* nearly every leaver has one receiver: the lanes write
+                     * theirs together.  (As a loop over the 27 neighbours,
+                     * unrolled, the wavefront ran the stores once for every
+                     * neighbour some lane goes to.) */
+                    const int ax0 = __ffs(bx) - 1, ay0 = __ffs(by) - 1, az0 = __ffs(bz) - 1;
+                    queue(ax0, ay0, az0, first);
+                    if (ncopy > 1) {
+                        /* a one-ulp overlap of cells: the others, in the
+                         * reference's scan order (x, then y, then z) */
+                        int kq = 0;
+#pragma unroll 1
+                        for (int k = 0; k < 27; k++) {
+                            const int ax = k / 9, ay = (k / 3) % 3, az = k % 3;
+                            if (!((bx >> ax) & (by >> ay) & (bz >> az) & 1u)) continue;
+                            if (kq > 0) queue(ax, ay, az, first + kq);
+                            kq++;
                         }
                     }
                 }
@@ -651,15 +653,20 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_scatter_ids(const long *off, long
 __global__ __launch_bounds__(PIC_BLOCK) void k_fix_arrivals(QueuePtrs q, int oldcap, PartPtrs to) {
     const long tile = blockIdx.x;
     const int n = q.count[tile];
-    const long qb = tile * (long)q.qcap;
+    const Leaver64 *const Q = q.e + tile * (long)q.qcap;
     for (int j = threadIdx.x; j < n; j += PIC_BLOCK) {
-        const long e = qb + j;
-        const int slot = q.slot[e];
+        const int slot = Q[j].slot;
         if (slot < oldcap || slot >= to.cap) continue;
-        const long dst = (long)q.dest[e] * to.cap + slot;
-        for (int k = 0; k < 6; k++) to.p[k][dst] = q.q[k][e];
-        to.sp[dst] = q.sp[e];
-        if (to.id) to.id[dst] = q.id[e];
+        const Leaver64 r = Q[j];
+        const long dst = (long)r.dest * to.cap + slot;
+        to.p[0][dst] = r.xy.x;
+        to.p[1][dst] = r.xy.y;
+        to.p[2][dst] = r.zu.x;
+        to.p[3][dst] = r.zu.y;
+        to.p[4][dst] = r.vw.x;
+        to.p[5][dst] = r.vw.y;
+        to.sp[dst] = (unsigned char)(r.where & 255);
+        if (to.id) to.id[dst] = r.id;
     }
 }
 
@@ -731,7 +738,7 @@ void launch_arrive_fold_f64(const Grid &g, const TileGeom &t, PartPtrs p, QueueP
     const unsigned tiles = what & PIC_ARRIVE ? (unsigned)t.ntiles : 0;
     const unsigned blocks = tiles + (what & PIC_FOLD ? fold_blocks(g) : 0);
     const FoldJ<double> J{{f.f[PIC_JX], f.f[PIC_JY], f.f[PIC_JZ]}};
-    hipLaunchKernelGGL((k_arrive_fold<TXC, TYC, TZC, PartPtrs, QueuePtrs, double>), dim3(blocks),
+    hipLaunchKernelGGL((k_arrive_fold<TXC, TYC, TZC, double>), dim3(blocks),
                        dim3(PIC_BLOCK), 0, s, g, t, p, q, st, J, tiles);
 }
 

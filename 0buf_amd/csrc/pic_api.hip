@@ -160,33 +160,18 @@ void swap_sets32(pic_ctx *c) {
     std::swap(c->p32.id, c->alt32.id);
 }
 
-template <class Q>
-void free_queue(Q &q) {
-    for (int k = 0; k < 6; k++)
-        if (q.q[k]) (void)hipFree(q.q[k]);
-    if (q.sp) (void)hipFree(q.sp);
-    if (q.dest) (void)hipFree(q.dest);
-    if (q.slot) (void)hipFree(q.slot);
+void free_queue(QueuePtrs &q) {
+    if (q.e) (void)hipFree(q.e);
     if (q.count) (void)hipFree(q.count);
-    if (q.id) (void)hipFree(q.id);
-    if (q.halo) (void)hipFree(q.halo);
-    q = Q{};
+    q = QueuePtrs{};
 }
 
-template <class Q>
-int alloc_queue(Q &q, const TileGeom &t, int qcap, bool with_id) {
-    using T = std::remove_pointer_t<std::remove_reference_t<decltype(q.q[0])>>;
-    q = Q{};
+int alloc_queue(QueuePtrs &q, const TileGeom &t, int qcap) {
+    q = QueuePtrs{};
     q.qcap = qcap;
-    size_t n = (size_t)t.ntiles * qcap;
-    for (int k = 0; k < 6; k++) HIPCHK(hipMalloc(&q.q[k], n * sizeof(T)));
-    HIPCHK(hipMalloc(&q.sp, n));
-    HIPCHK(hipMalloc(&q.dest, n * sizeof(int)));
-    HIPCHK(hipMalloc(&q.slot, n * sizeof(int)));
+    HIPCHK(hipMalloc(&q.e, (size_t)t.ntiles * qcap * sizeof(Leaver64)));
     HIPCHK(hipMalloc(&q.count, t.ntiles * sizeof(int)));
     HIPCHK(hipMemset(q.count, 0, t.ntiles * sizeof(int)));
-    if (with_id) HIPCHK(hipMalloc(&q.id, n * sizeof(int)));
-    HIPCHK(hipMalloc(&q.halo, n));
     return PIC_SUCCESS;
 }
 
@@ -197,7 +182,7 @@ void free_queue(QueuePtrs32 &q) {
     q = QueuePtrs32{};
 }
 
-int alloc_queue(QueuePtrs32 &q, const TileGeom &t, int qcap, bool) {
+int alloc_queue(QueuePtrs32 &q, const TileGeom &t, int qcap) {
     q = QueuePtrs32{};
     q.qcap = qcap;
     const size_t n = (size_t)t.ntiles * qcap;
@@ -283,7 +268,7 @@ int commit_into(pic_ctx *c, P &parts, Q &queue, int cap, const std::vector<long>
     if constexpr (std::is_same<P, PartPtrs32>::value) rc = alloc_live32(c, cap);
     else rc = alloc_parts(parts, NC, cap, true, c->diff);
     if (rc) return rc;
-    rc = alloc_queue(queue, c->t, queue_capacity(c->t, cap), c->diff);
+    rc = alloc_queue(queue, c->t, queue_capacity(c->t, cap));
     if (rc) return rc;
     long *d_off = nullptr;
     T *d_src[6] = {nullptr};
@@ -391,7 +376,7 @@ int regrow_parts(pic_ctx *c, P &parts, Q &queue) {
     free_parts(parts);
     parts = np;
     Q nq;
-    rc = alloc_queue(nq, c->t, queue_capacity(c->t, cap), c->diff);
+    rc = alloc_queue(nq, c->t, queue_capacity(c->t, cap));
     if (rc) return rc;
     free_queue(queue);
     queue = nq;
@@ -435,7 +420,7 @@ int regrow32(pic_ctx *c, bool from_queue) {
     c->lay32.tcap = (long)c->t.TX * c->t.TY * c->t.TZ * cap;
     c->lay32.packed = 0;
     QueuePtrs32 nq;
-    if ((rc = alloc_queue(nq, c->t, queue_capacity(c->t, cap), c->diff))) return rc;
+    if ((rc = alloc_queue(nq, c->t, queue_capacity(c->t, cap)))) return rc;
     free_queue(c->q32);
     c->q32 = nq;
     c->regrows++;
@@ -963,8 +948,8 @@ int pic_generate_device(pic_ctx *c, const pic_species_spec *specs, int nspec,
     HIPCHK(hipSetDevice(c->dev));
     int rc = c->fp32 ? alloc_live32(c, cap) : alloc_parts(c->p, NC, cap, true, c->diff);
     if (rc) return rc;
-    rc = c->fp32 ? alloc_queue(c->q32, c->t, queue_capacity(c->t, cap), c->diff)
-                 : alloc_queue(c->q, c->t, queue_capacity(c->t, cap), c->diff);
+    rc = c->fp32 ? alloc_queue(c->q32, c->t, queue_capacity(c->t, cap))
+                 : alloc_queue(c->q, c->t, queue_capacity(c->t, cap));
     if (rc) return rc;
     HIPCHK(hipMemsetAsync(count_ptr(c), 0, NC * sizeof(int), c->stream));
     int *d_cnt = nullptr, *d_start = nullptr, *d_fail = nullptr;

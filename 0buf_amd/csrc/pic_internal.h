@@ -150,15 +150,21 @@ struct QueuePtrs32 {
     int qcap;                /* entries per tile */
 };
 
+/* FP64 departure queue: one 64-byte record (half a line) per leaver, four
+ * 16-byte stores in the push and four loads in the arrival */
+struct __align__(16) Leaver64 {
+    double2 xy, zu, vw;      /* x y, z pu, pv pw */
+    int dest;                /* destination bulk cell */
+    int where;               /* species | destination in the source tile's
+                                (TX+2)(TY+2)(TZ+2) halo box << 8 */
+    int id;                  /* differentiable form only */
+    int slot;                /* -1; the slot the arrival claimed where that lies
+                                past the bucket capacity */
+};
 struct QueuePtrs {
-    double *q[6];
-    unsigned char *sp;
-    int *dest;               /* destination bulk cell */
-    int *slot;               /* slot claimed by the arrival kernel */
+    Leaver64 *e;
     int *count;              /* per tile */
     int qcap;                /* entries per tile */
-    int *id;                 /* differentiable form only */
-    unsigned char *halo;     /* destination in the source tile's (TX+2)(TY+2)(TZ+2) halo box */
 };
 
 struct TileGeom {
