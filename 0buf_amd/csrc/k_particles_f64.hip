@@ -321,8 +321,8 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
                     const int ii[6] = {W.ix, W.i1x, W.iy, W.i1y, W.iz, W.i1z};
                     for (int q = 0; q < 6; q++) tape_put(tout, TAPE_GIDX + q, 1, ii[q], 2);
                     for (int d = 0; d < 3; d++) {
-                        tape_put(tout, TAPE_FLOOR + 4 * d, 2, W.f1[d] - gc[d], 0);
-                        tape_put(tout, TAPE_FLOOR + 4 * d + 2, 2, W.f15[d] - gc[d], 0);
+                        tape_put(tout, TAPE_FLOOR + 4 * d, 2, (int)W.f1[d] - gc[d], 0);
+                        tape_put(tout, TAPE_FLOOR + 4 * d + 2, 2, (int)W.f15[d] - gc[d], 0);
                     }
                 }
                 const double s1 = W.s1, s2 = W.s2, s3 = W.s3, s4 = W.s4, s5 = W.s5, s6 = W.s6;
