@@ -374,29 +374,33 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_fold_j(Grid g, FV<T, JT> f, int d
  * one-address atomics.  The workgroup that finishes last adds up the
  * partials and puts the energy, and the step's status where asked for, into
  * pinned host memory: as a launch and two copies of their own these took
- * about 15 us of a small step. */
-__device__ __forceinline__ double block_tree(double *red, double s) {
-    red[threadIdx.x] = s;
+ * about 15 us of a small step.  Each workgroup's release and acquire at
+ * device scope passes through the L2s, so they are few (one per CU) and
+ * large: 1024 workgroups of 256 took 33 us at 256x64x64 cells, 12 more than
+ * the same without the last step. */
+constexpr int ENERGY_T = 1024, ENERGY_BLOCKS = 256;
+
+__device__ __forceinline__ double block_sum(double *red, double s) {
+    for (int d = 32; d > 0; d >>= 1) s += __shfl_xor(s, d);
+    if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = s;
     __syncthreads();
-    for (int w = PIC_BLOCK / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    return red[0];
+    s = 0.0;
+    for (int w = 0; w < ENERGY_T / 64; w++) s += red[w];
+    return s;
 }
 
 template <typename T, typename JT>
-__global__ __launch_bounds__(PIC_BLOCK) void k_energy(Grid g, FV<T, JT> f, EnergyOut o) {
-    __shared__ double red[PIC_BLOCK];
+__global__ __launch_bounds__(ENERGY_T) void k_energy(Grid g, FV<T, JT> f, EnergyOut o) {
+    __shared__ double red[2][ENERGY_T / 64];
     __shared__ bool last;
     const T *ex = f.E[0], *ey = f.E[1], *ez = f.E[2];
     double s = 0.0;
-    for (long n = (long)blockIdx.x * PIC_BLOCK + threadIdx.x; n < g.G;
-         n += (long)gridDim.x * PIC_BLOCK) {
+    for (long n = (long)blockIdx.x * ENERGY_T + threadIdx.x; n < g.G;
+         n += (long)gridDim.x * ENERGY_T) {
         double a = (double)ex[n], b = (double)ey[n], c = (double)ez[n];
         s += a * a + b * b + c * c;
     }
-    const double part = block_tree(red, s);
+    const double part = block_sum(red[0], s);
     if (threadIdx.x == 0) {
         __hip_atomic_store(&o.partials[blockIdx.x], part, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
@@ -406,10 +410,11 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_energy(Grid g, FV<T, JT> f, Energ
     }
     __syncthreads();
     if (!last) return;
-    s = 0.0;
-    for (int j = threadIdx.x; j < (int)gridDim.x; j += PIC_BLOCK)
-        s += __hip_atomic_load(&o.partials[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const double total = block_tree(red, s);
+    static_assert(ENERGY_BLOCKS <= ENERGY_T, "one partial per thread");
+    s = threadIdx.x < gridDim.x ? __hip_atomic_load(&o.partials[threadIdx.x], __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT)
+                                : 0.0;
+    const double total = block_sum(red[1], s);
     if (threadIdx.x == 0) {
         *o.done = 0;
         *o.h_energy = total;
@@ -464,10 +469,9 @@ void fold_j(const Grid &g, FV<T, JT> f, hipStream_t s) {
                            g, f, dir);
 }
 template <typename T, typename JT>
-void energy(const Grid &g, FV<T, JT> f, const EnergyOut &o, int nblocks, hipStream_t s) {
-    /* (workgroups past the nodes would add exact zeros) */
-    const unsigned nb = std::min((unsigned)nblocks, blocks_for(g.G));
-    hipLaunchKernelGGL((k_energy<T, JT>), dim3(nb), dim3(PIC_BLOCK), 0, s, g, f, o);
+void energy(const Grid &g, FV<T, JT> f, const EnergyOut &o, hipStream_t s) {
+    const unsigned nb = (unsigned)std::min((g.G + ENERGY_T - 1) / ENERGY_T, (long)ENERGY_BLOCKS);
+    hipLaunchKernelGGL((k_energy<T, JT>), dim3(nb), dim3(ENERGY_T), 0, s, g, f, o);
 }
 
 }  // namespace
@@ -479,8 +483,8 @@ void launch_h2(const Grid &g, FieldPtrs f, hipStream_t s) { h2(g, view(f), s); }
 void launch_e(const Grid &g, FieldPtrs f, hipStream_t s) { e_update(g, view(f), s); }
 void launch_e_periodic(const Grid &g, FieldPtrs f, hipStream_t s) { e_periodic(g, view(f), s); }
 void launch_fold_j(const Grid &g, FieldPtrs f, hipStream_t s) { fold_j(g, view(f), s); }
-void launch_energy(const Grid &g, FieldPtrs f, const EnergyOut &o, int nblocks, hipStream_t s) {
-    energy(g, view(f), o, nblocks, s);
+void launch_energy(const Grid &g, FieldPtrs f, const EnergyOut &o, hipStream_t s) {
+    energy(g, view(f), o, s);
 }
 
 void launch_h_half32(const Grid &g, FieldPtrs32 f, DevStatus *reset, hipStream_t s) {
@@ -492,8 +496,8 @@ void launch_e_periodic32(const Grid &g, FieldPtrs32 f, hipStream_t s) {
     e_periodic(g, view(f), s);
 }
 void launch_fold_j32(const Grid &g, FieldPtrs32 f, hipStream_t s) { fold_j(g, view(f), s); }
-void launch_energy32(const Grid &g, FieldPtrs32 f, const EnergyOut &o, int nblocks, hipStream_t s) {
-    energy(g, view(f), o, nblocks, s);
+void launch_energy32(const Grid &g, FieldPtrs32 f, const EnergyOut &o, hipStream_t s) {
+    energy(g, view(f), o, s);
 }
 
 void launch_h2_e(const Grid &g, FieldPtrs f, double *const h_out[3], hipStream_t s) {

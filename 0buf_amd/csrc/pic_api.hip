@@ -544,8 +544,8 @@ void enq_h2_e(pic_ctx *c) {
 /* the energy into h_red[0], with_status: and the step's status into h_st */
 void enq_energy(pic_ctx *c, bool with_status) {
     const EnergyOut o{c->d_part, c->d_done, c->h_red, with_status ? c->d_st : nullptr, c->h_st};
-    if (c->fp32) launch_energy32(c->g, c->f32, o, c->npart, c->stream);
-    else launch_energy(c->g, c->f, o, c->npart, c->stream);
+    if (c->fp32) launch_energy32(c->g, c->f32, o, c->stream);
+    else launch_energy(c->g, c->f, o, c->stream);
 }
 
 int check_ready(pic_ctx *c) {

@@ -392,7 +392,7 @@ void launch_h2_e(const Grid &g, FieldPtrs f, double *const h_out[3], hipStream_t
 void launch_h2_e32(const Grid &g, FieldPtrs32 f, float *const h_out[3], hipStream_t s);
 /* where an energy reduction leaves its result */
 struct EnergyOut {
-    double *partials;        /* one per workgroup */
+    double *partials;        /* one per workgroup, at most 256 */
     unsigned *done;          /* workgroups done, 0 between launches */
     double *h_energy;        /* pinned host memory */
     const DevStatus *st;     /* the step's status, copied to h_st (null: not) */
@@ -404,14 +404,14 @@ void launch_h2(const Grid &g, FieldPtrs f, hipStream_t s);
 void launch_e(const Grid &g, FieldPtrs f, hipStream_t s);
 void launch_e_periodic(const Grid &g, FieldPtrs f, hipStream_t s);
 void launch_fold_j(const Grid &g, FieldPtrs f, hipStream_t s);
-void launch_energy(const Grid &g, FieldPtrs f, const EnergyOut &o, int nblocks, hipStream_t s);
+void launch_energy(const Grid &g, FieldPtrs f, const EnergyOut &o, hipStream_t s);
 void launch_reset_status(DevStatus *st, hipStream_t s);
 void launch_h_half32(const Grid &g, FieldPtrs32 f, DevStatus *reset, hipStream_t s);
 void launch_h2_32(const Grid &g, FieldPtrs32 f, hipStream_t s);
 void launch_e32(const Grid &g, FieldPtrs32 f, hipStream_t s);
 void launch_e_periodic32(const Grid &g, FieldPtrs32 f, hipStream_t s);
 void launch_fold_j32(const Grid &g, FieldPtrs32 f, hipStream_t s);
-void launch_energy32(const Grid &g, FieldPtrs32 f, const EnergyOut &o, int nblocks, hipStream_t s);
+void launch_energy32(const Grid &g, FieldPtrs32 f, const EnergyOut &o, hipStream_t s);
 TileGeom make_tile_geom(int Nx, int Ny, int Nz);
 
 /* Differentiable form of the FP64 step: the push deposits J as int64 fixed
