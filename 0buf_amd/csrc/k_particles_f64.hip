@@ -22,6 +22,7 @@
 #include "k_arrive.h"
 #include "k_tape.h"
 #include "k_push_math.h"
+#include "k_receiver.h"
 
 #pragma clang fp contract(off)
 
@@ -93,18 +94,20 @@ __device__ __forceinline__ void pqr_lds(double *sJ, const Geo &c, const DivConst
     const int u = c.ca + ix - 2, v = c.cb + iy - 2, w = c.cc + iz - 2;
     const int n = (u * BY + v) * BZ + w;
     double *Jx = sJ, *Jy = sJ + NB, *Jz = sJ + 2 * NB;
-    jadd<DIFF>(Jx, n, su * (dy1 * dz1 + s1), bad);
-    jadd<DIFF>(Jx, n + 1, su * (dy1 * dz - s1), bad);
-    jadd<DIFF>(Jx, n + BZ, su * (dy * dz1 - s1), bad);
-    jadd<DIFF>(Jx, n + BZ + 1, su * (dy * dz + s1), bad);
-    jadd<DIFF>(Jy, n, sv * (dx1 * dz1 + s2), bad);
-    jadd<DIFF>(Jy, n + 1, sv * (dx1 * dz - s2), bad);
-    jadd<DIFF>(Jy, n + BY * BZ, sv * (dx * dz1 - s2), bad);
-    jadd<DIFF>(Jy, n + BY * BZ + 1, sv * (dx * dz + s2), bad);
-    jadd<DIFF>(Jz, n, sw * (dx1 * dy1 + s3), bad);
-    jadd<DIFF>(Jz, n + BZ, sw * (dx1 * dy - s3), bad);
-    jadd<DIFF>(Jz, n + BY * BZ, sw * (dx * dy1 - s3), bad);
-    jadd<DIFF>(Jz, n + BY * BZ + BZ, sw * (dx * dy + s3), bad);
+    /* (one rounding less per weight than the reference's product and sum: the
+     * order of the atomic sums moves J by more) */
+    jadd<DIFF>(Jx, n, su * fma(dy1, dz1, s1), bad);
+    jadd<DIFF>(Jx, n + 1, su * fma(dy1, dz, -s1), bad);
+    jadd<DIFF>(Jx, n + BZ, su * fma(dy, dz1, -s1), bad);
+    jadd<DIFF>(Jx, n + BZ + 1, su * fma(dy, dz, s1), bad);
+    jadd<DIFF>(Jy, n, sv * fma(dx1, dz1, s2), bad);
+    jadd<DIFF>(Jy, n + 1, sv * fma(dx1, dz, -s2), bad);
+    jadd<DIFF>(Jy, n + BY * BZ, sv * fma(dx, dz1, -s2), bad);
+    jadd<DIFF>(Jy, n + BY * BZ + 1, sv * fma(dx, dz, s2), bad);
+    jadd<DIFF>(Jz, n, sw * fma(dx1, dy1, s3), bad);
+    jadd<DIFF>(Jz, n + BZ, sw * fma(dx1, dy, -s3), bad);
+    jadd<DIFF>(Jz, n + BY * BZ, sw * fma(dx, dy1, -s3), bad);
+    jadd<DIFF>(Jz, n + BY * BZ + BZ, sw * fma(dx, dy, s3), bad);
 }
 
 /* 4 waves per SIMD (at most 128 VGPRs): the FP64 chains of the push are
@@ -373,6 +376,9 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
                 const double e1x = m ? R.x2x : x1, e1y = m ? R.x2y : y1, e1z = m ? R.x2z : z1;
                 pqr_lds<BY, BZ, NB, DIFF>(myJ, G, a.dc, R.i1x, R.i1y, R.i1z, x, y, z, e1x, e1y, e1z,
                                           mass, bad, true);
+                /* (kept waiting in registers until a lane has a second one, as
+                 * the FP32 push does, they spill at 128 VGPRs: 2.47 against
+                 * 2.38 ms at 67M particles) */
                 pqr_lds<BY, BZ, NB, DIFF>(myJ, G, a.dc, R.i2x, R.i2y, R.i2z, R.x2x, R.x2y, R.x2z, x1,
                                           y1, z1, mass, bad, m != 0);
             }
@@ -423,21 +429,16 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
                  * 27-neighbourhood (getWrapCellNumber) whose isPointInCell
                  * (cell.h:717) holds receives a copy; per axis the test is
                  * separable, so the receivers are a product of per-axis sets. */
-                /* per axis, bit d+1 set when neighbour d in {-1,0,1} accepts */
-                unsigned bx = 0, by = 0, bz = 0;
-                for (int d = -1; d <= 1; d++) {
-                    int r = gi + d;
-                    if (r >= g.Nx) r -= g.Nx; else if (r < 0) r += g.Nx;
-                    double r0 = (double)r * hx;
-                    if (r0 <= xn && xn < r0 + hx) bx |= 1u << (d + 1);
-                    r = gl + d;
-                    if (r >= g.Ny) r -= g.Ny; else if (r < 0) r += g.Ny;
-                    r0 = (double)r * hy;
-                    if (r0 <= yn && yn < r0 + hy) by |= 1u << (d + 1);
-                    r = gk + d;
-                    if (r >= g.Nz) r -= g.Nz; else if (r < 0) r += g.Nz;
-                    r0 = (double)r * hz;
-                    if (r0 <= zn && zn < r0 + hz) bz |= 1u << (d + 1);
+                /* per axis, bit d+1 set when neighbour d in {-1,0,1} accepts;
+                 * the test of all three only where some lane lies near a face */
+                bool near = false;
+                unsigned bx = receiver(xn, a.dc.rhx, gi, g.Nx, near),
+                         by = receiver(yn, a.dc.rhy, gl, g.Ny, near),
+                         bz = receiver(zn, a.dc.rhz, gk, g.Nz, near);
+                if (near) {
+                    bx = receivers(xn, hx, gi, g.Nx);
+                    by = receivers(yn, hy, gl, g.Ny);
+                    bz = receivers(zn, hz, gk, g.Nz);
                 }
                 if (trec) {
                     const unsigned bb[3] = {bx, by, bz};
