@@ -34,14 +34,13 @@ namespace {
 
 constexpr int TXC = 2, TYC = 4, TZC = 8;
 
-/* copies of the LDS adjoint box the gather adjoint scatters into: lane l adds
- * into copy l % ACOPIES, dividing the same-address conflicts of the FP64 LDS
- * atomics (the particles of one cell scatter to the same nodes); the copies
- * are summed before the global add */
-#ifndef PIC_ACOPIES64
-#define PIC_ACOPIES64 3
-#endif
-constexpr int ACOPIES = PIC_ACOPIES64;
+/* Copies of the LDS adjoint box the gather adjoint scatters into, lane l
+ * adding into copy l % ACOPIES, copies 9 mod 16 doubles apart (the reasons
+ * stand at the FP32 adjoint's).  Measured, one step at 24.6M particles,
+ * 128x64x64 cells, before the changes below: 2.54 ms with 5 copies, 2.61 with
+ * 4, 2.83 with 3; 3.71 with 3 copies on the same banks. */
+constexpr int ACOPIES = 6;
+constexpr int copy_stride(int n) { return (n + 6) / 16 * 16 + 9; }   /* >= n, 9 mod 16 */
 
 inline unsigned blocks_for(long n) { return (unsigned)((n + PIC_BLOCK - 1) / PIC_BLOCK); }
 
@@ -239,27 +238,27 @@ struct AdjArgs {
 /* adjoint of one pqr segment (cell.h:1511-1693): gradient of
  * sum_nodes lamJ[node] * contribution(A -> B) with respect to the segment
  * ends A and B; lamJ is read from the LDS box at the forward's nodes */
-template <int BY, int BZ, int NB>
+template <int BY, int BZ, int JY0, int JZ0>
 __device__ __forceinline__ void pqr_adj(const double *sL, const Geo &c, const DivConst &dc, int ix,
                                         int iy, int iz, double ax, double ay, double az, double bx,
                                         double by, double bz, double q, double gA[3],
                                         double gB[3]) {
+#pragma clang fp contract(fast)   /* no decision depends on the reverse sweep */
     const double dx = (0.50 * (ax + bx) - c.hx * ((double)ix - 2.50) - c.x0);
     const double dy = (0.50 * (ay + by) - c.hy * ((double)iy - 2.50) - c.y0);
     const double dz = (0.50 * (az + bz) - c.hz * ((double)iz - 2.50) - c.z0);
     const double dx1 = c.hx - dx, dy1 = c.hy - dy, dz1 = c.hz - dz;
     const double Dx = bx - ax, Dy = by - ay, Dz = bz - az;
     const double s1 = Dy * Dz * dc.r12, s2 = Dx * Dz * dc.r12, s3 = Dx * Dy * dc.r12;
-    const double kx = q * dc.rDx, ky = q * dc.rDy, kz = q * dc.rDz;
+    /* the forward deposits nothing outside the tile stencil (and flags it):
+     * weight 0, at a node inside the box.  (An early return would put gA and
+     * gB in scratch memory.) */
+    const bool in = ix >= 2 && ix <= 3 && iy >= 2 && iy <= 3 && iz >= 2 && iz <= 3;
+    const double qi = in ? q : 0.0;
+    const double kx = qi * dc.rDx, ky = qi * dc.rDy, kz = qi * dc.rDz;
     const double SU = Dx * kx, SV = Dy * ky, SW = Dz * kz;
-    const int u = c.ca + ix - 2, v = c.cb + iy - 2, w = c.cc + iz - 2;
-    const int n = (u * BY + v) * BZ + w;
-    /* the forward deposits nothing outside the tile stencil (and flags it) */
-    if (ix < 2 || ix > 3 || iy < 2 || iy > 3 || iz < 2 || iz > 3) {
-        for (int d = 0; d < 3; d++) gA[d] = gB[d] = 0.0;
-        return;
-    }
-    const double *Lx = sL, *Ly = sL + NB, *Lz = sL + 2 * NB;
+    const int n = in ? ((c.ca + ix - 2) * BY + c.cb + iy - 2) * BZ + c.cc + iz - 2 : 0;
+    const double *Lx = sL, *Ly = sL + JY0, *Lz = sL + JZ0;
     const double a0 = Lx[n], a1 = Lx[n + 1], a2 = Lx[n + BZ], a3 = Lx[n + BZ + 1];
     const double b0 = Ly[n], b1 = Ly[n + 1], b2 = Ly[n + BY * BZ], b3 = Ly[n + BY * BZ + 1];
     const double c0 = Lz[n], c1 = Lz[n + BZ], c2 = Lz[n + BY * BZ], c3 = Lz[n + BY * BZ + BZ];
@@ -293,28 +292,36 @@ __device__ __forceinline__ void pqr_adj(const double *sL, const Geo &c, const Di
     gB[2] = 0.5 * gdz + gDz;
 }
 
-/* adjoint of Interpolate3D: scatter lam * weight into the LDS adjoint box and
- * return d(lam * value)/d(sx, sy, sz), the weights of the near planes
- * (the far-plane weights are 1 - s) */
+/* Interpolate3D with the forward's rounding sequence (interp, k_push_math.h),
+ * and the derivatives of the value with respect to sx, sy, sz, the weights of
+ * the near planes (the far-plane weights are 1 - s), from the same eight
+ * nodes: the reverse part needs no node again */
 template <int BY, int BZ>
-__device__ __forceinline__ void interp_adj(const double *F, double *A, int u, int v, int w,
-                                           double sx, double sy, double sz, double lam,
-                                           double &dsx, double &dsy, double &dsz) {
-    const double sx1 = 1. - sx, sy1 = 1. - sy, sz1 = 1. - sz;
-    const int o = (u * BY + v) * BZ + w;
+__device__ __forceinline__ double interp_grad(const double *F, int o, double sx, double sx1,
+                                              double sy, double sy1, double sz, double sz1,
+                                              double g[3]) {
     const double f000 = F[o], f001 = F[o + 1], f010 = F[o + BZ], f011 = F[o + BZ + 1];
     const double f100 = F[o + BY * BZ], f101 = F[o + BY * BZ + 1];
     const double f110 = F[o + BY * BZ + BZ], f111 = F[o + BY * BZ + BZ + 1];
+    const double z00 = sz * f000 + sz1 * f001, z01 = sz * f010 + sz1 * f011;
+    const double z10 = sz * f100 + sz1 * f101, z11 = sz * f110 + sz1 * f111;
+    const double y0 = sy * z00 + sy1 * z01, y1 = sy * z10 + sy1 * z11;
+    {
+#pragma clang fp contract(fast)
+        g[0] = y0 - y1;
+        g[1] = sx * (z00 - z01) + sx1 * (z10 - z11);
+        g[2] = sx * (sy * (f000 - f001) + sy1 * (f010 - f011)) +
+               sx1 * (sy * (f100 - f101) + sy1 * (f110 - f111));
+    }
+    const double t1 = sx * y0, t2 = sx1 * y1;
+    return t2 + t1;
+}
+
+/* its adjoint: lam * weight into the eight nodes of the LDS adjoint box */
+template <int BY, int BZ>
+__device__ __forceinline__ void interp_scatter(double *A, int o, double sx, double sx1, double sy,
+                                               double sy1, double sz, double sz1, double lam) {
     const double yz00 = sy * sz, yz01 = sy * sz1, yz10 = sy1 * sz, yz11 = sy1 * sz1;
-    const double p0 = yz00 * f000 + yz01 * f001 + yz10 * f010 + yz11 * f011;
-    const double p1 = yz00 * f100 + yz01 * f101 + yz10 * f110 + yz11 * f111;
-    dsx += lam * (p0 - p1);
-    const double ly0 = sx * (sz * f000 + sz1 * f001) + sx1 * (sz * f100 + sz1 * f101);
-    const double ly1 = sx * (sz * f010 + sz1 * f011) + sx1 * (sz * f110 + sz1 * f111);
-    dsy += lam * (ly0 - ly1);
-    const double lz0 = sx * (sy * f000 + sy1 * f010) + sx1 * (sy * f100 + sy1 * f110);
-    const double lz1 = sx * (sy * f001 + sy1 * f011) + sx1 * (sy * f101 + sy1 * f111);
-    dsz += lam * (lz0 - lz1);
     const double lx0 = lam * sx, lx1 = lam * sx1;
     atomicAdd(&A[o], lx0 * yz00);
     atomicAdd(&A[o + 1], lx0 * yz01);
@@ -327,11 +334,13 @@ __device__ __forceinline__ void interp_adj(const double *F, double *A, int u, in
 }
 
 __device__ __forceinline__ void cross(const double a[3], const double b[3], double r[3]) {
+#pragma clang fp contract(fast)
     r[0] = a[1] * b[2] - a[2] * b[1];
     r[1] = a[2] * b[0] - a[0] * b[2];
     r[2] = a[0] * b[1] - a[1] * b[0];
 }
 __device__ __forceinline__ double dot3(const double a[3], const double b[3]) {
+#pragma clang fp contract(fast)
     return a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
 }
 
@@ -339,10 +348,18 @@ template <int TX, int TY, int TZ, int NT>
 __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
     constexpr int C = TX * TY * TZ;
     constexpr int BX = TX + 2, BY = TY + 2, BZ = TZ + 2, NB = BX * BY * BZ;
-    __shared__ double sF[6 * NB];    /* E, H' of the forward step */
-    __shared__ double sL[3 * NB];    /* lamJ */
-    __shared__ double sA[ACOPIES * 6 * NB];   /* lamE, lamH' accumulated by the gather adjoint */
-    double *const myA = sA + (threadIdx.x % ACOPIES) * (6 * NB);
+    /* Ex, Hy, Hz and Jx (node-type, or dual, along x) take x planes 0..TX only
+     * (NBX nodes), the others all BX planes, as in the FP32 form's boxes */
+    constexpr int NBX = (TX + 1) * BY * BZ;
+    constexpr int FB[6] = {0, NBX, NBX + NB, NBX + 2 * NB, NBX + 3 * NB, 2 * NBX + 3 * NB};
+    constexpr int FN[6] = {NBX, NB, NB, NB, NBX, NBX};   /* nodes in each box */
+    constexpr int NF = 3 * NBX + 3 * NB, NJ = NBX + 2 * NB, JY0 = FB[1], JZ0 = FB[2];
+    constexpr int AS = copy_stride(NF);
+    static_assert(AS >= NF && AS % 16 == 9, "");
+    __shared__ double sF[NF];        /* E, H' of the forward step */
+    __shared__ double sL[NJ];        /* lamJ */
+    __shared__ double sA[ACOPIES * AS];   /* lamE, lamH' accumulated by the gather adjoint */
+    double *const myA = sA + (threadIdx.x % ACOPIES) * AS;
     __shared__ int sOff[C + 1];
     __shared__ int sCnt[C];
     __shared__ unsigned sFlags;
@@ -391,13 +408,15 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
         }
         if (tid < NB) {
 #pragma unroll
-            for (int q = 0; q < 6; q++) sF[q * NB + tid] = fv[q];
-#pragma unroll
-            for (int q = 0; q < 3; q++) sL[q * NB + tid] = lj[q];
+            for (int q = 0; q < 6; q++) {
+                if (tid >= FN[q]) continue;
+                sF[FB[q] + tid] = fv[q];
+                if (q < 3) sL[FB[q] + tid] = lj[q];
+            }
         }
         if (tid < C) sCnt[tid] = cnt;
     }
-    for (int e = tid; e < ACOPIES * 6 * NB; e += NT) sA[e] = 0.0;
+    for (int e = tid; e < ACOPIES * AS; e += NT) sA[e] = 0.0;
     if (tid == 0) sFlags = 0;
     __syncthreads();
     if (tid == 0) {
@@ -443,6 +462,8 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
         const double fry = divc(y - G.y0, hy, a.dc.rhy);
         const double frz = divc(z - G.z0, hz, a.dc.rhz);
         double Ef[3] = {0, 0, 0}, Hf[3] = {0, 0, 0};
+        int o[6] = {0, 0, 0, 0, 0, 0};
+        double gw[6][3] = {};   /* d(field component) / d(near weights) */
         const bool live = !(x < 0 || y < 0 || z < 0);
         GatherIdx W{};
         if (live) {
@@ -453,13 +474,22 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
                 const double s1 = W.s1, s2 = W.s2, s3 = W.s3, s4 = W.s4, s5 = W.s5, s6 = W.s6;
                 const double s11 = 1. - s1, s21 = 1. - s2, s31 = 1. - s3, s41 = 1. - s4,
                              s51 = 1. - s5, s61 = 1. - s6;
-                const int ua = G.ca - 2, va = G.cb - 2, wa = G.cc - 2;
-                Ef[0] = interp<BY, BZ>(sF + 0 * NB, ua + W.ix, va + W.i1y, wa + W.i1z, s1, s11, s4, s41, s6, s61);
-                Ef[1] = interp<BY, BZ>(sF + 1 * NB, ua + W.i1x, va + W.iy, wa + W.i1z, s2, s21, s3, s31, s6, s61);
-                Ef[2] = interp<BY, BZ>(sF + 2 * NB, ua + W.i1x, va + W.i1y, wa + W.iz, s2, s21, s4, s41, s5, s51);
-                Hf[0] = interp<BY, BZ>(sF + 3 * NB, ua + W.i1x, va + W.iy, wa + W.iz, s2, s21, s3, s31, s5, s51);
-                Hf[1] = interp<BY, BZ>(sF + 4 * NB, ua + W.ix, va + W.i1y, wa + W.iz, s1, s11, s4, s41, s5, s51);
-                Hf[2] = interp<BY, BZ>(sF + 5 * NB, ua + W.ix, va + W.iy, wa + W.i1z, s1, s11, s3, s31, s6, s61);
+                /* node of the component's near corner in its box */
+                const int n0 = ((G.ca - 2) * BY + (G.cb - 2)) * BZ + (G.cc - 2);
+                const int bx = W.ix * (BY * BZ), bx1 = W.i1x * (BY * BZ), by = W.iy * BZ,
+                          by1 = W.i1y * BZ, bz = W.iz, bz1 = W.i1z;
+                o[0] = n0 + bx + by1 + bz1;
+                Ef[0] = interp_grad<BY, BZ>(sF + FB[0], o[0], s1, s11, s4, s41, s6, s61, gw[0]);
+                o[1] = n0 + bx1 + by + bz1;
+                Ef[1] = interp_grad<BY, BZ>(sF + FB[1], o[1], s2, s21, s3, s31, s6, s61, gw[1]);
+                o[2] = n0 + bx1 + by1 + bz;
+                Ef[2] = interp_grad<BY, BZ>(sF + FB[2], o[2], s2, s21, s4, s41, s5, s51, gw[2]);
+                o[3] = n0 + bx1 + by + bz;
+                Hf[0] = interp_grad<BY, BZ>(sF + FB[3], o[3], s2, s21, s3, s31, s5, s51, gw[3]);
+                o[4] = n0 + bx + by1 + bz;
+                Hf[1] = interp_grad<BY, BZ>(sF + FB[4], o[4], s1, s11, s4, s41, s5, s51, gw[4]);
+                o[5] = n0 + bx + by + bz1;
+                Hf[2] = interp_grad<BY, BZ>(sF + FB[5], o[5], s1, s11, s3, s31, s6, s61, gw[5]);
             }
         }
         const Boris B = boris_move(pu, pv, pw, Ef[0], Ef[1], Ef[2], Hf[0], Hf[1], Hf[2], tau1);
@@ -469,7 +499,7 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
         const Relay R = relay_point(x, y, z, x1, y1, z1, frx, fry, frz, G, a.dc);
         const int m = R.m;
 
-        /* ---- reverse ---- */
+        /* ---- reverse (contracted: no decision depends on it) ---- */
         double2 *const lq = (double2 *)(a.lp.v + (long)pid * PIC_LSTRIDE);
         const double2 q0 = lq[0], q1 = lq[1], q2 = lq[2];
         double lx1[3] = {q0.x, q0.y, q1.x};
@@ -478,9 +508,10 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
         const double X0[3] = {x, y, z}, X1[3] = {x1, y1, z1};
         /* deposit: J = pqr(i1; x -> e1) + [m != 0] pqr(i2; x2 -> x1) */
         {
+#pragma clang fp contract(fast)
             double gA[3], gB[3];
             const double e1x = m ? R.x2x : x1, e1y = m ? R.x2y : y1, e1z = m ? R.x2z : z1;
-            pqr_adj<BY, BZ, NB>(sL, G, a.dc, R.i1x, R.i1y, R.i1z, x, y, z, e1x, e1y, e1z, mass,
+            pqr_adj<BY, BZ, JY0, JZ0>(sL, G, a.dc, R.i1x, R.i1y, R.i1z, x, y, z, e1x, e1y, e1z, mass,
                                 gA, gB);
             lx[0] = gA[0];
             lx[1] = gA[1];
@@ -491,7 +522,7 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
                 lx1[2] += gB[2];
             } else {
                 double hA[3], hB[3];
-                pqr_adj<BY, BZ, NB>(sL, G, a.dc, R.i2x, R.i2y, R.i2z, R.x2x, R.x2y, R.x2z, x1, y1,
+                pqr_adj<BY, BZ, JY0, JZ0>(sL, G, a.dc, R.i2x, R.i2y, R.i2z, R.x2x, R.x2y, R.x2z, x1, y1,
                                     z1, mass, hA, hB);
                 lx1[0] += hB[0];
                 lx1[1] += hB[1];
@@ -502,34 +533,33 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
                 const bool cr[3] = {(m & 4) != 0, (m & 2) != 0, (m & 1) != 0};
                 const double F[3] = {R.fx, R.fy, R.fz};
                 double lsr = 0.0;
+#pragma unroll
                 for (int d = 0; d < 3; d++) {
-                    if (cr[d]) continue;
-                    lsr += lx2[d] * (X1[d] - X0[d]);
-                    lx[d] += lx2[d] * (1.0 - R.sr);
-                    lx1[d] += lx2[d] * R.sr;
+                    const double v = cr[d] ? 0.0 : lx2[d];
+                    lsr += v * (X1[d] - X0[d]);
+                    lx[d] += v * (1.0 - R.sr);
+                    lx1[d] += v * R.sr;
                 }
+                /* sr = num/den: one crossed face num = f_d - x_d, den = D_d;
+                 * two num = sum (f_d - x_d) D_d, den = sum D_d^2.  (Selected,
+                 * not branched around: a branch per axis became a computed
+                 * index, which put the arrays in scratch memory.) */
                 const int nc = (int)cr[0] + (int)cr[1] + (int)cr[2];
-                if (nc == 1) {
-                    const int d = cr[0] ? 0 : (cr[1] ? 1 : 2);
-                    const double D = X1[d] - X0[d];
-                    lx[d] += lsr * (R.sr - 1.0) / D;
-                    lx1[d] += lsr * (-R.sr / D);
-                } else if (nc == 2) {
-                    for (int d = 0; d < 3; d++) {
-                        if (!cr[d]) continue;
-                        const double D = X1[d] - X0[d], f = F[d] - X0[d];
-                        /* num = sum (f_d - x_d) D_d, den = sum D_d^2 */
-                        const double dnum_x = -D - f, dnum_x1 = f;
-                        const double dden_x = -2.0 * D, dden_x1 = 2.0 * D;
-                        lx[d] += lsr * (dnum_x - R.sr * dden_x) / R.den;
-                        lx1[d] += lsr * (dnum_x1 - R.sr * dden_x1) / R.den;
-                    }
+                const double w = nc == 1 || nc == 2 ? lsr / R.den : 0.0;
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    const double D = X1[d] - X0[d], f = F[d] - X0[d];
+                    const double gx = nc == 1 ? R.sr - 1.0 : 2.0 * R.sr * D - D - f;
+                    const double gx1 = nc == 1 ? -R.sr : f - 2.0 * R.sr * D;
+                    lx[d] += cr[d] ? w * gx : 0.0;
+                    lx1[d] += cr[d] ? w * gx1 : 0.0;
                 }
             }
         }
         /* x1 = x + tau g2 p1 */
         for (int d = 0; d < 3; d++) lx[d] += lx1[d];
         {
+#pragma clang fp contract(fast)
             const double lu[3] = {tau * lx1[0], tau * lx1[1], tau * lx1[2]};
             const double g2 = B.g2, g23 = g2 * g2 * g2;
             const double pl = dot3(B.p1, lu);
@@ -538,6 +568,7 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
         /* p1 = pp + tau1 E;  pp = (s + (b.s) b + s x b) / (1 + b.b) */
         double lE[3], lH[3], lpm[3];
         {
+#pragma clang fp contract(fast)
             for (int d = 0; d < 3; d++) lE[d] = tau1 * lp1[d];
             const double *b = B.b, *sv = B.s;
             const double rD = 1.0 / B.sden;
@@ -579,17 +610,25 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
         /* gather: scatter into the adjoint box, position derivative through
          * the weights (every s has ds/dx = -1/h) */
         if (live && W.ok) {
-            const int ua = G.ca - 2, va = G.cb - 2, wa = G.cc - 2;
-            double dsx = 0, dsy = 0, dsz = 0;
-            interp_adj<BY, BZ>(sF + 0 * NB, myA + 0 * NB, ua + W.ix, va + W.i1y, wa + W.i1z, W.s1, W.s4, W.s6, lE[0], dsx, dsy, dsz);
-            interp_adj<BY, BZ>(sF + 1 * NB, myA + 1 * NB, ua + W.i1x, va + W.iy, wa + W.i1z, W.s2, W.s3, W.s6, lE[1], dsx, dsy, dsz);
-            interp_adj<BY, BZ>(sF + 2 * NB, myA + 2 * NB, ua + W.i1x, va + W.i1y, wa + W.iz, W.s2, W.s4, W.s5, lE[2], dsx, dsy, dsz);
-            interp_adj<BY, BZ>(sF + 3 * NB, myA + 3 * NB, ua + W.i1x, va + W.iy, wa + W.iz, W.s2, W.s3, W.s5, lH[0], dsx, dsy, dsz);
-            interp_adj<BY, BZ>(sF + 4 * NB, myA + 4 * NB, ua + W.ix, va + W.i1y, wa + W.iz, W.s1, W.s4, W.s5, lH[1], dsx, dsy, dsz);
-            interp_adj<BY, BZ>(sF + 5 * NB, myA + 5 * NB, ua + W.ix, va + W.iy, wa + W.i1z, W.s1, W.s3, W.s6, lH[2], dsx, dsy, dsz);
-            lx[0] -= dsx * a.dc.rhx;
-            lx[1] -= dsy * a.dc.rhy;
-            lx[2] -= dsz * a.dc.rhz;
+            interp_scatter<BY, BZ>(myA + FB[0], o[0], W.s1, 1. - W.s1, W.s4, 1. - W.s4, W.s6,
+                                   1. - W.s6, lE[0]);
+            interp_scatter<BY, BZ>(myA + FB[1], o[1], W.s2, 1. - W.s2, W.s3, 1. - W.s3, W.s6,
+                                   1. - W.s6, lE[1]);
+            interp_scatter<BY, BZ>(myA + FB[2], o[2], W.s2, 1. - W.s2, W.s4, 1. - W.s4, W.s5,
+                                   1. - W.s5, lE[2]);
+            interp_scatter<BY, BZ>(myA + FB[3], o[3], W.s2, 1. - W.s2, W.s3, 1. - W.s3, W.s5,
+                                   1. - W.s5, lH[0]);
+            interp_scatter<BY, BZ>(myA + FB[4], o[4], W.s1, 1. - W.s1, W.s4, 1. - W.s4, W.s5,
+                                   1. - W.s5, lH[1]);
+            interp_scatter<BY, BZ>(myA + FB[5], o[5], W.s1, 1. - W.s1, W.s3, 1. - W.s3, W.s6,
+                                   1. - W.s6, lH[2]);
+            const double rh[3] = {a.dc.rhx, a.dc.rhy, a.dc.rhz};
+            for (int d = 0; d < 3; d++) {
+#pragma clang fp contract(fast)
+                const double ds = lE[0] * gw[0][d] + lE[1] * gw[1][d] + lE[2] * gw[2][d] +
+                                  lH[0] * gw[3][d] + lH[1] * gw[4][d] + lH[2] * gw[5][d];
+                lx[d] -= ds * rh[d];
+            }
         }
         lq[0] = make_double2(lx[0], lx[1]);
         lq[1] = make_double2(lx[2], lpm[0]);
@@ -600,9 +639,10 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
     if (tid < NB) {   /* thread n adds box node n of the six adjoint boxes */
 #pragma unroll
         for (int q = 0; q < 6; q++) {
-            const int e = q * NB + tid;
+            if (tid >= FN[q]) continue;
+            const int e = FB[q] + tid;
             double val = sA[e];
-            for (int r = 1; r < ACOPIES; r++) val += sA[r * 6 * NB + e];
+            for (int r = 1; r < ACOPIES; r++) val += sA[r * AS + e];
             if (val != 0.0 && node_in)
                 atomicAdd(q < 3 ? &a.lam.E[q][noff] : &a.lam.H[q - 3][noff], val);
         }

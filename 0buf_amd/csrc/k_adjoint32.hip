@@ -22,14 +22,19 @@ namespace {
 constexpr int TXC = 2, TYC = 4, TZC = 8;
 constexpr int ADJ_NT = 512;   /* threads of a workgroup (launch_adj_particles_f32) */
 
-/* copies of the LDS adjoint box the gather adjoint scatters into: lane l adds
- * into copy l % ACOPIES, dividing the same-address conflicts of the FP64 LDS
- * atomics (the particles of one cell scatter to the same nodes); the copies
- * are summed before the global add */
-#ifndef PIC_ACOPIES32
-#define PIC_ACOPIES32 4
-#endif
-constexpr int ACOPIES = PIC_ACOPIES32;
+/* Copies of the LDS adjoint box the gather adjoint scatters into: lane l adds
+ * into copy l % ACOPIES (the particles of one cell scatter to the same nodes);
+ * the copies are summed before the global add.  The LDS takes the FP64 adds of
+ * 16 lanes at a time, on 16 banks of doubles: adds to one bank, equal
+ * addresses or not, wait for each other.  The 8 corners that the lanes of one
+ * cell differ by lie on 8 banks (strides 1, 10, 60), and copies 9 mod 16
+ * doubles apart spread the lanes best: about 2.9 turns per add with 6 copies
+ * and 3.3 with 4; with 4 copies 12 mod 16 apart 3.8, 8 mod 16 4.8, 0 mod 16
+ * 7.9.  Measured, one step at 50M particles, 256x64x64 cells: 3.07 ms with 6
+ * copies 9 apart, 3.25 with 5, 3.44 with 4; 3.57 with 4 copies 12 apart, 4.16
+ * 8 apart, 5.7 0 apart.  7 copies leave one workgroup per CU (3.51). */
+constexpr int ACOPIES = 6;
+constexpr int copy_stride(int n) { return (n + 6) / 16 * 16 + 9; }   /* >= n, 9 mod 16 */
 
 struct AdjArgs32 {
     Grid g;
@@ -146,8 +151,10 @@ __global__ __launch_bounds__(NT) void k_adj_particles32(AdjArgs32 a) {
     constexpr int JY0 = FB[1], JZ0 = FB[2];
     __shared__ float sF[NF];
     __shared__ float sL[NJ];
-    __shared__ double sA[ACOPIES * NF];
-    double *const myA = sA + (threadIdx.x % ACOPIES) * NF;
+    constexpr int AS = copy_stride(NF);
+    static_assert(AS >= NF && AS % 16 == 9, "");
+    __shared__ double sA[ACOPIES * AS];
+    double *const myA = sA + (threadIdx.x % ACOPIES) * AS;
     __shared__ int sOff[C + 1];
     __shared__ int sCnt[C];
 
@@ -204,7 +211,7 @@ __global__ __launch_bounds__(NT) void k_adj_particles32(AdjArgs32 a) {
         }
         if (tid < C) sCnt[tid] = cnt;
     }
-    for (int e = tid; e < ACOPIES * NF; e += NT) sA[e] = 0.0;
+    for (int e = tid; e < ACOPIES * AS; e += NT) sA[e] = 0.0;
     __syncthreads();
     if (tid == 0) {
         int s = 0;
@@ -373,7 +380,7 @@ __global__ __launch_bounds__(NT) void k_adj_particles32(AdjArgs32 a) {
             if (tid >= FN[q]) continue;
             const int e = FB[q] + tid;
             double val = sA[e];
-            for (int r = 1; r < ACOPIES; r++) val += sA[r * NF + e];
+            for (int r = 1; r < ACOPIES; r++) val += sA[r * AS + e];
             if (val != 0.0 && node_in)
                 atomicAdd(q < 3 ? &a.lam.E[q][noff] : &a.lam.H[q - 3][noff], val);
         }

@@ -378,46 +378,56 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_fold_j(Grid g, FV<T, JT> f, int d
  * device scope passes through the L2s, so they are few (one per CU) and
  * large: 1024 workgroups of 256 took 33 us at 256x64x64 cells, 12 more than
  * the same without the last step. */
-constexpr int ENERGY_T = 1024, ENERGY_BLOCKS = 256;
+constexpr int ENERGY_T = 1024, ENERGY_PARTS = 1024, SUB = ENERGY_T / PIC_BLOCK;
 
-__device__ __forceinline__ double block_sum(double *red, double s) {
-    for (int d = 32; d > 0; d >>= 1) s += __shfl_xor(s, d);
-    if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = s;
+/* The sum over PIC_BLOCK consecutive threads, SUB sums in a workgroup: the
+ * pairs t, t + 128, then t, t + 64, ... in turn.  Thread 0 of each holds it. */
+__device__ __forceinline__ double sub_tree(double (*red)[PIC_BLOCK], double s) {
+    const int sub = threadIdx.x / PIC_BLOCK, t = threadIdx.x % PIC_BLOCK;
+    red[sub][t] = s;
     __syncthreads();
-    s = 0.0;
-    for (int w = 0; w < ENERGY_T / 64; w++) s += red[w];
+    if (t < 64) {
+        const double *r = red[sub] + t;
+        s = (r[0] + r[128]) + (r[64] + r[192]);
+        for (int d = 32; d > 0; d >>= 1) s += __shfl_down(s, d);
+    }
+    __syncthreads();
     return s;
 }
 
 template <typename T, typename JT>
 __global__ __launch_bounds__(ENERGY_T) void k_energy(Grid g, FV<T, JT> f, EnergyOut o) {
-    __shared__ double red[2][ENERGY_T / 64];
+    __shared__ double red[SUB][PIC_BLOCK];
     __shared__ bool last;
     const T *ex = f.E[0], *ey = f.E[1], *ez = f.E[2];
+    /* ENERGY_PARTS partials, each the sum of PIC_BLOCK threads that stride
+     * over the nodes, whatever the launch */
+    const int part = blockIdx.x * SUB + threadIdx.x / PIC_BLOCK;
     double s = 0.0;
-    for (long n = (long)blockIdx.x * ENERGY_T + threadIdx.x; n < g.G;
-         n += (long)gridDim.x * ENERGY_T) {
+    for (long n = (long)part * PIC_BLOCK + threadIdx.x % PIC_BLOCK; n < g.G;
+         n += (long)ENERGY_PARTS * PIC_BLOCK) {
         double a = (double)ex[n], b = (double)ey[n], c = (double)ez[n];
         s += a * a + b * b + c * c;
     }
-    const double part = block_sum(red[0], s);
-    if (threadIdx.x == 0) {
-        __hip_atomic_store(&o.partials[blockIdx.x], part, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-        /* the partial is released with the count and acquired by the last */
+    s = sub_tree(red, s);
+    if (threadIdx.x % PIC_BLOCK == 0)
+        __hip_atomic_store(&o.partials[part], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    /* the workgroup's partials are released with the count and acquired by
+     * the last */
+    if (threadIdx.x == 0)
         last = __hip_atomic_fetch_add(o.done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
                gridDim.x - 1;
-    }
     __syncthreads();
     if (!last) return;
-    static_assert(ENERGY_BLOCKS <= ENERGY_T, "one partial per thread");
-    s = threadIdx.x < gridDim.x ? __hip_atomic_load(&o.partials[threadIdx.x], __ATOMIC_RELAXED,
-                                                    __HIP_MEMORY_SCOPE_AGENT)
-                                : 0.0;
-    const double total = block_sum(red[1], s);
+    s = 0.0;
+    if (threadIdx.x < PIC_BLOCK)
+        for (unsigned j = threadIdx.x; j < gridDim.x * SUB; j += PIC_BLOCK)
+            s += __hip_atomic_load(&o.partials[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s = sub_tree(red, s);
     if (threadIdx.x == 0) {
         *o.done = 0;
-        *o.h_energy = total;
+        *o.h_energy = s;
         if (o.st) *o.h_st = *o.st;
     }
 }
@@ -470,7 +480,9 @@ void fold_j(const Grid &g, FV<T, JT> f, hipStream_t s) {
 }
 template <typename T, typename JT>
 void energy(const Grid &g, FV<T, JT> f, const EnergyOut &o, hipStream_t s) {
-    const unsigned nb = (unsigned)std::min((g.G + ENERGY_T - 1) / ENERGY_T, (long)ENERGY_BLOCKS);
+    /* (partials past the nodes would add exact zeros) */
+    const unsigned nb =
+        (unsigned)std::min((g.G + ENERGY_T - 1) / ENERGY_T, (long)ENERGY_PARTS / SUB);
     hipLaunchKernelGGL((k_energy<T, JT>), dim3(nb), dim3(ENERGY_T), 0, s, g, f, o);
 }
 

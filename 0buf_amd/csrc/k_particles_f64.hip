@@ -94,20 +94,22 @@ __device__ __forceinline__ void pqr_lds(double *sJ, const Geo &c, const DivConst
     const int u = c.ca + ix - 2, v = c.cb + iy - 2, w = c.cc + iz - 2;
     const int n = (u * BY + v) * BZ + w;
     double *Jx = sJ, *Jy = sJ + NB, *Jz = sJ + 2 * NB;
-    /* (one rounding less per weight than the reference's product and sum: the
-     * order of the atomic sums moves J by more) */
-    jadd<DIFF>(Jx, n, su * fma(dy1, dz1, s1), bad);
-    jadd<DIFF>(Jx, n + 1, su * fma(dy1, dz, -s1), bad);
-    jadd<DIFF>(Jx, n + BZ, su * fma(dy, dz1, -s1), bad);
-    jadd<DIFF>(Jx, n + BZ + 1, su * fma(dy, dz, s1), bad);
-    jadd<DIFF>(Jy, n, sv * fma(dx1, dz1, s2), bad);
-    jadd<DIFF>(Jy, n + 1, sv * fma(dx1, dz, -s2), bad);
-    jadd<DIFF>(Jy, n + BY * BZ, sv * fma(dx, dz1, -s2), bad);
-    jadd<DIFF>(Jy, n + BY * BZ + 1, sv * fma(dx, dz, s2), bad);
-    jadd<DIFF>(Jz, n, sw * fma(dx1, dy1, s3), bad);
-    jadd<DIFF>(Jz, n + BZ, sw * fma(dx1, dy, -s3), bad);
-    jadd<DIFF>(Jz, n + BY * BZ, sw * fma(dx, dy1, -s3), bad);
-    jadd<DIFF>(Jz, n + BY * BZ + BZ, sw * fma(dx, dy, s3), bad);
+    /* plain form: one rounding less per weight than the reference's product
+     * and sum (the order of the atomic sums moves J by more); the
+     * differentiable form, whose sums have no order, keeps both */
+    auto weight = [](double a, double b, double s) { return DIFF ? a * b + s : fma(a, b, s); };
+    jadd<DIFF>(Jx, n, su * weight(dy1, dz1, s1), bad);
+    jadd<DIFF>(Jx, n + 1, su * weight(dy1, dz, -s1), bad);
+    jadd<DIFF>(Jx, n + BZ, su * weight(dy, dz1, -s1), bad);
+    jadd<DIFF>(Jx, n + BZ + 1, su * weight(dy, dz, s1), bad);
+    jadd<DIFF>(Jy, n, sv * weight(dx1, dz1, s2), bad);
+    jadd<DIFF>(Jy, n + 1, sv * weight(dx1, dz, -s2), bad);
+    jadd<DIFF>(Jy, n + BY * BZ, sv * weight(dx, dz1, -s2), bad);
+    jadd<DIFF>(Jy, n + BY * BZ + 1, sv * weight(dx, dz, s2), bad);
+    jadd<DIFF>(Jz, n, sw * weight(dx1, dy1, s3), bad);
+    jadd<DIFF>(Jz, n + BZ, sw * weight(dx1, dy, -s3), bad);
+    jadd<DIFF>(Jz, n + BY * BZ, sw * weight(dx, dy1, -s3), bad);
+    jadd<DIFF>(Jz, n + BY * BZ + BZ, sw * weight(dx, dy, s3), bad);
 }
 
 /* 4 waves per SIMD (at most 128 VGPRs): the FP64 chains of the push are

@@ -392,7 +392,7 @@ void launch_h2_e(const Grid &g, FieldPtrs f, double *const h_out[3], hipStream_t
 void launch_h2_e32(const Grid &g, FieldPtrs32 f, float *const h_out[3], hipStream_t s);
 /* where an energy reduction leaves its result */
 struct EnergyOut {
-    double *partials;        /* one per workgroup, at most 256 */
+    double *partials;        /* 1024 */
     unsigned *done;          /* workgroups done, 0 between launches */
     double *h_energy;        /* pinned host memory */
     const DevStatus *st;     /* the step's status, copied to h_st (null: not) */
