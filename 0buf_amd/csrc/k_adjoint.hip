@@ -13,7 +13,7 @@
  *     W_t = sum E'^2
  * The reverse step takes (lamE, lamH, lamP) at s_t to s_{t-1}:
  *   1. lamE += 2 w_t E_t                                (k_adj_seed_energy)
- *   2. lamE <- P^T lamE                                 (k_adj_e_periodic_*)
+ *   2. lamE <- P^T lamE                                 (k_adj_e_periodic)
  *   3. lamH += Ce^T lamE|R ; lamQ := lamH|RQ ;
  *      lamJ := -tau lamE|R                              (k_adj_curl_e)
  *   4. lamJ <- Fold^T lamJ                              (k_adj_fold_j)
@@ -26,6 +26,7 @@
  * particle stage accumulates lamE, lamH in an LDS box per tile with FP64
  * atomics and adds the box to the global arrays with FP64 atomics.
  */
+#include "k_fold.h"
 #include "k_push_math.h"
 
 #pragma clang fp contract(off)
@@ -61,48 +62,35 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_adj_seed_energy(Grid g, const dou
     l.E[2][n] += w2 * Ez[n];
 }
 
-/* transpose of E[0] = E[N]; E[N+1] = E[1] along one line */
-__device__ __forceinline__ void ghost_copy_T(double *L, long n0, long n1, long nN, long nN1) {
-    L[n1] += L[nN1];
-    L[nN1] = 0.0;
-    L[nN] += L[n0];
-    L[n0] = 0.0;
-}
-
-/* transpose of k_e_periodic_z (Ex over i in [0,Nx], l in [0,Ny+1]; Ey over
- * i in [0,Nx+1], l in [0,Ny]) */
-__global__ __launch_bounds__(PIC_BLOCK) void k_adj_e_periodic_z(Grid g, AdjLam lam) {
-    const long t = (long)blockIdx.x * PIC_BLOCK + threadIdx.x;
-    if (t >= (long)(g.Nx + 2) * (g.Ny + 2)) return;
-    const int i = (int)(t / (g.Ny + 2)), l = (int)(t % (g.Ny + 2));
-    const long base = (long)i * g.sx + (long)l * g.sy;
-    if (l <= g.Ny) ghost_copy_T(lam.E[1], base, base + 1, base + g.Nz, base + g.Nz + 1);
-    if (i <= g.Nx) ghost_copy_T(lam.E[0], base, base + 1, base + g.Nz, base + g.Nz + 1);
-}
-
-/* transpose of k_e_periodic_x (Ey over l in [0,Ny], k in [1,Nz]; Ez over l
- * in [1,Ny], k in [0,Nz]) */
-__global__ __launch_bounds__(PIC_BLOCK) void k_adj_e_periodic_x(Grid g, AdjLam lam) {
-    const long t = (long)blockIdx.x * PIC_BLOCK + threadIdx.x;
-    if (t >= (long)(g.Ny + 2) * g.sy) return;
-    const int l = (int)(t / g.sy), k = (int)(t % g.sy);
-    const long base = (long)l * g.sy + k;
-    const long n0 = base, n1 = (long)g.sx + base, nN = (long)g.Nx * g.sx + base,
-               nN1 = (long)(g.Nx + 1) * g.sx + base;
-    if (l >= 1 && l <= g.Ny && k <= g.Nz) ghost_copy_T(lam.E[2], n0, n1, nN, nN1);
-    if (l <= g.Ny && k >= 1 && k <= g.Nz) ghost_copy_T(lam.E[1], n0, n1, nN, nN1);
-}
-
-/* transpose of k_e_periodic_y (ghost_mode 1: Ex and Ez along y) */
-__global__ __launch_bounds__(PIC_BLOCK) void k_adj_e_periodic_y(Grid g, AdjLam lam) {
-    const long t = (long)blockIdx.x * PIC_BLOCK + threadIdx.x;
-    if (t >= (long)(g.Nx + 2) * g.sy) return;
-    const int i = (int)(t / g.sy), k = (int)(t % g.sy);
-    const long base = (long)i * g.sx + k;
-    const long n0 = base, n1 = base + g.sy, nN = base + (long)g.Ny * g.sy,
-               nN1 = base + (long)(g.Ny + 1) * g.sy;
-    ghost_copy_T(lam.E[2], n0, n1, nN, nN1);
-    ghost_copy_T(lam.E[0], n0, n1, nN, nN1);
+/* transposes of the periodic E ghost copies, the forward's x, z and (in
+ * ghost_mode 1) y copies last to first, E[0] = E[N]; E[N+1] = E[1] along a line
+ * becoming L[N] += L[0], L[0] = 0; L[1] += L[N+1], L[N+1] = 0.  One thread per
+ * class of nodes the copies combine (k_fold.h), one launch: three of their
+ * own took 15 us of a small step.
+ *   z: Ex over i in [0,Nx], l in [0,Ny+1]; Ey over i in [0,Nx+1], l in [0,Ny]
+ *   x: Ey over l in [0,Ny], k in [1,Nz]; Ez over l in [1,Ny], k in [0,Nz]
+ *   y (ghost_mode 1): Ex and Ez */
+__global__ __launch_bounds__(PIC_BLOCK) void k_adj_e_periodic(Grid g, AdjLam lam) {
+    const unsigned t = blockIdx.x * PIC_BLOCK + threadIdx.x;
+    if (t >= shell_count(g)) return;
+    const NodeClass c = node_class(g, t);
+    for (int cc = 0; cc < 3; cc++)
+        on_class(c, lam.E[cc], [&](double (&v)[8]) {
+            auto back = [&](int d, auto in_range) {
+                class_pairs(c, v, d, [&](double &r, double &p, int s) {
+                    if (!in_range(s)) return;
+                    r += p;
+                    p = 0.0;
+                });
+            };
+            if (g.ghost_mode == 1 && cc != 1) back(1, [](int) { return true; });
+            if (cc == 0) back(2, [&](int s) { return c.i(s) <= g.Nx; });
+            if (cc == 1) back(2, [&](int s) { return c.l(s) <= g.Ny; });
+            if (cc == 1)
+                back(0, [&](int s) { return c.l(s) <= g.Ny && c.k(s) >= 1 && c.k(s) <= g.Nz; });
+            if (cc == 2)
+                back(0, [&](int s) { return c.l(s) >= 1 && c.l(s) <= g.Ny && c.k(s) <= g.Nz; });
+        });
 }
 
 /* E-update ranges (emeElement, kernels.cu:1162-1181) */
@@ -160,34 +148,29 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_adj_curl_e(Grid g, AdjLam lam) {
     lam.J[2][n] = -tau * ez;
 }
 
-/* transpose of the J fold for one face direction (k_fold_j: per component
- * c: if dir != c: J[1] += J[N-1]; if !(dir == y && c == y): J[N-1] = J[1];
- * J[0] += J[N-2]; J[N-2] = J[0]), operations reversed */
-__global__ __launch_bounds__(PIC_BLOCK) void k_adj_fold_j(Grid g, AdjLam lam, int dir) {
-    const long t = (long)blockIdx.x * PIC_BLOCK + threadIdx.x;
-    int na, nb, N;
-    if (dir == 0) { na = g.Ny + 2; nb = g.Nz + 2; N = g.Nx + 2; }
-    else if (dir == 1) { na = g.Nx + 2; nb = g.Nz + 2; N = g.Ny + 2; }
-    else { na = g.Nx + 2; nb = g.Ny + 2; N = g.Nz + 2; }
-    if (t >= (long)na * nb) return;
-    const int a = (int)(t / nb), b = (int)(t % nb);
-    long base, stride;
-    if (dir == 0) { base = (long)a * g.sy + b; stride = g.sx; }
-    else if (dir == 1) { base = (long)a * g.sx + b; stride = g.sy; }
-    else { base = (long)a * g.sx + (long)b * g.sy; stride = 1; }
-    const long n1 = base + stride, nNm1 = base + (long)(N - 1) * stride;
-    const long nNm2 = base + (long)(N - 2) * stride, n0 = base;
-    for (int c = 2; c >= 0; c--) {
-        double *L = lam.J[c];
-        L[n0] += L[nNm2];
-        L[nNm2] = 0.0;
-        L[nNm2] += L[n0];
-        if (dir != 1 || c != 1) {
-            L[n1] += L[nNm1];
-            L[nNm1] = 0.0;
-        }
-        if (dir != c) L[nNm1] += L[n1];
-    }
+/* transpose of the J fold (k_fold_j, per axis and component: if axis != c:
+ * J[1] += J[N+1]; if !(axis == y && c == y): J[N+1] = J[1]; J[0] += J[N];
+ * J[N] = J[0]), operations reversed, z, y, x; one thread per class of nodes the
+ * fold combines, one launch instead of three */
+__global__ __launch_bounds__(PIC_BLOCK) void k_adj_fold_j(Grid g, AdjLam lam) {
+    const unsigned t = blockIdx.x * PIC_BLOCK + threadIdx.x;
+    if (t >= shell_count(g)) return;
+    const NodeClass c = node_class(g, t);
+    const bool at_n[3] = {c.ri == g.Nx, c.rl == g.Ny, c.rk == g.Nz};
+    for (int cc = 0; cc < 3; cc++)
+        on_class(c, lam.J[cc], [&](double (&v)[8]) {
+#pragma unroll
+            for (int d = 2; d >= 0; d--)
+                class_pairs(c, v, d, [&](double &r, double &p, int) {
+                    if (at_n[d] || d != cc) {          /* both ends take the sum */
+                        r += p;
+                        p = r;
+                    } else if (d != 1) {
+                        r += p;
+                        p = 0.0;
+                    }
+                });
+        });
 }
 
 /* transpose of Q = Ch E:  Qx = 1/2(c1z(Ey[k+1]-Ey) - c1y(Ez[l+1]-Ez)) etc.,
@@ -678,13 +661,7 @@ void launch_adj_seed_energy(const Grid &g, const double *const E[3], double w, A
 }
 
 void launch_adj_e_periodic(const Grid &g, AdjLam l, hipStream_t s) {
-    if (g.ghost_mode == 1)
-        hipLaunchKernelGGL(k_adj_e_periodic_y, dim3(blocks_for((long)(g.Nx + 2) * g.sy)),
-                           dim3(PIC_BLOCK), 0, s, g, l);
-    hipLaunchKernelGGL(k_adj_e_periodic_z, dim3(blocks_for((long)(g.Nx + 2) * (g.Ny + 2))),
-                       dim3(PIC_BLOCK), 0, s, g, l);
-    hipLaunchKernelGGL(k_adj_e_periodic_x, dim3(blocks_for((long)(g.Ny + 2) * g.sy)),
-                       dim3(PIC_BLOCK), 0, s, g, l);
+    hipLaunchKernelGGL(k_adj_e_periodic, dim3(fold_blocks(g)), dim3(PIC_BLOCK), 0, s, g, l);
 }
 
 void launch_adj_curl_e(const Grid &g, AdjLam l, hipStream_t s) {
@@ -692,11 +669,7 @@ void launch_adj_curl_e(const Grid &g, AdjLam l, hipStream_t s) {
 }
 
 void launch_adj_fold_j(const Grid &g, AdjLam l, hipStream_t s) {
-    const long faces[3] = {(long)(g.Ny + 2) * (g.Nz + 2), (long)(g.Nx + 2) * (g.Nz + 2),
-                           (long)(g.Nx + 2) * (g.Ny + 2)};
-    for (int dir = 2; dir >= 0; dir--)
-        hipLaunchKernelGGL(k_adj_fold_j, dim3(blocks_for(faces[dir])), dim3(PIC_BLOCK), 0, s, g,
-                           l, dir);
+    hipLaunchKernelGGL(k_adj_fold_j, dim3(fold_blocks(g)), dim3(PIC_BLOCK), 0, s, g, l);
 }
 
 void launch_adj_particles_f64(const Grid &g, const TileGeom &t, AdjFwd fwd, PartPtrs snap,

@@ -48,69 +48,90 @@ __host__ __device__ __forceinline__ unsigned shell_count(const Grid &g) {
            2u * (unsigned)(g.Nx - 2) * (g.Ny - 2);
 }
 
+/* class t: its representative (ri, rl, rk), the partner coordinate along each
+ * axis (-1: none) and the node of member s (bit d of s: the partner's
+ * coordinate along d) */
+struct NodeClass {
+    int ri, rl, rk, px, py, pz;
+    unsigned m[8];
+    __device__ __forceinline__ bool member(int s) const {
+        return ((s & 1) == 0 || px >= 0) && ((s & 2) == 0 || py >= 0) && ((s & 4) == 0 || pz >= 0);
+    }
+    __device__ __forceinline__ int i(int s) const { return s & 1 ? px : ri; }
+    __device__ __forceinline__ int l(int s) const { return s & 2 ? py : rl; }
+    __device__ __forceinline__ int k(int s) const { return s & 4 ? pz : rk; }
+};
+
+__device__ __forceinline__ NodeClass node_class(const Grid &g, unsigned t) {
+    const int Nx = g.Nx, Ny = g.Ny, Nz = g.Nz;
+    NodeClass c;
+    const unsigned fx = 2u * Ny * Nz, fy = 2u * (unsigned)(Nx - 2) * Nz;
+    if (t < fx) {                                    /* ri in {1, Nx} */
+        const unsigned a = t / ((unsigned)Ny * Nz), r = t - a * ((unsigned)Ny * Nz);
+        c.ri = a ? Nx : 1;
+        c.rl = (int)(r / Nz) + 1;
+        c.rk = (int)(r % Nz) + 1;
+    } else if ((t -= fx) < fy) {                     /* rl in {1, Ny} */
+        const unsigned a = t / ((unsigned)(Nx - 2) * Nz), r = t - a * ((unsigned)(Nx - 2) * Nz);
+        c.rl = a ? Ny : 1;
+        c.ri = (int)(r / Nz) + 2;
+        c.rk = (int)(r % Nz) + 1;
+    } else {                                         /* rk in {1, Nz} */
+        t -= fy;
+        const unsigned a = t / ((unsigned)(Nx - 2) * (Ny - 2)),
+                       r = t - a * ((unsigned)(Nx - 2) * (Ny - 2));
+        c.rk = a ? Nz : 1;
+        c.ri = (int)(r / (Ny - 2)) + 2;
+        c.rl = (int)(r % (Ny - 2)) + 2;
+    }
+    c.px = c.ri == Nx ? 0 : c.ri == 1 ? Nx + 1 : -1;
+    c.py = c.rl == Ny ? 0 : c.rl == 1 ? Ny + 1 : -1;
+    c.pz = c.rk == Nz ? 0 : c.rk == 1 ? Nz + 1 : -1;
+#pragma unroll
+    for (int s = 0; s < 8; s++)
+        c.m[s] = (unsigned)c.i(s) * (unsigned)g.sx + (unsigned)c.l(s) * (unsigned)g.sy +
+                 (unsigned)c.k(s);
+    return c;
+}
+
+/* the values of one component at the class's nodes, op on them, and back:
+ * op(v) works on v[8] in registers */
+template <typename JT, class Op>
+__device__ __forceinline__ void on_class(const NodeClass &c, JT *J, Op op) {
+    JT v[8];
+#pragma unroll
+    for (int s = 0; s < 8; s++) v[s] = c.member(s) ? J[c.m[s]] : (JT)0;
+    op(v);
+#pragma unroll
+    for (int s = 0; s < 8; s++)
+        if (c.member(s)) J[c.m[s]] = v[s];
+}
+
+/* pair(v at the representative's side, v at the partner's, member s) over the
+ * class's pairs along axis d (no pair: none) */
+template <typename JT, class Pair>
+__device__ __forceinline__ void class_pairs(const NodeClass &c, JT (&v)[8], int d, Pair pair) {
+    if ((d == 0 ? c.px : d == 1 ? c.py : c.pz) < 0) return;
+#pragma unroll
+    for (int s = 0; s < 8; s++)
+        if (!(s & (1 << d)) && c.member(s)) pair(v[s], v[s | (1 << d)], s);
+}
+
 /* the three k_fold_j launches x, y, z in one: thread t takes one class of
  * more than one node, folds its current in registers (x pairs, then y, then
  * z, as the launches run, with the same additions) and writes it back */
 template <typename JT>
 __device__ __forceinline__ void fold_class(const Grid &g, const FoldJ<JT> &f, unsigned t) {
     if (t >= shell_count(g)) return;
-    const int Nx = g.Nx, Ny = g.Ny, Nz = g.Nz;
-    int ri, rl, rk;
-    const unsigned fx = 2u * Ny * Nz, fy = 2u * (unsigned)(Nx - 2) * Nz;
-    if (t < fx) {                                    /* ri in {1, Nx} */
-        const unsigned a = t / ((unsigned)Ny * Nz), r = t - a * ((unsigned)Ny * Nz);
-        ri = a ? Nx : 1;
-        rl = (int)(r / Nz) + 1;
-        rk = (int)(r % Nz) + 1;
-    } else if ((t -= fx) < fy) {                     /* rl in {1, Ny} */
-        const unsigned a = t / ((unsigned)(Nx - 2) * Nz), r = t - a * ((unsigned)(Nx - 2) * Nz);
-        rl = a ? Ny : 1;
-        ri = (int)(r / Nz) + 2;
-        rk = (int)(r % Nz) + 1;
-    } else {                                         /* rk in {1, Nz} */
-        t -= fy;
-        const unsigned a = t / ((unsigned)(Nx - 2) * (Ny - 2)),
-                       r = t - a * ((unsigned)(Nx - 2) * (Ny - 2));
-        rk = a ? Nz : 1;
-        ri = (int)(r / (Ny - 2)) + 2;
-        rl = (int)(r % (Ny - 2)) + 2;
-    }
-    const unsigned sy = (unsigned)g.sy, sx = (unsigned)g.sx;
-    const int px = ri == Nx ? 0 : ri == 1 ? Nx + 1 : -1;
-    const int py = rl == Ny ? 0 : rl == 1 ? Ny + 1 : -1;
-    const int pz = rk == Nz ? 0 : rk == 1 ? Nz + 1 : -1;
-    const int X[2] = {ri, px}, Y[2] = {rl, py}, Z[2] = {rk, pz};
-    auto member = [&](int s) {
-        return ((s & 1) == 0 || px >= 0) && ((s & 2) == 0 || py >= 0) && ((s & 4) == 0 || pz >= 0);
-    };
-    unsigned m[8];
+    const NodeClass c = node_class(g, t);
+    const bool at_n[3] = {c.ri == g.Nx, c.rl == g.Ny, c.rk == g.Nz};
+    for (int cc = 0; cc < 3; cc++)
+        on_class(c, f.J[cc], [&](JT (&v)[8]) {
 #pragma unroll
-    for (int s = 0; s < 8; s++)
-        m[s] = (unsigned)X[s & 1] * sx + (unsigned)Y[(s >> 1) & 1] * sy + (unsigned)Z[s >> 2];
-    for (int cc = 0; cc < 3; cc++) {
-        JT *J = f.J[cc];
-        JT v[8];
-#pragma unroll
-        for (int s = 0; s < 8; s++) v[s] = member(s) ? J[m[s]] : (JT)0;
-        if (px >= 0) {
-#pragma unroll
-            for (int s = 0; s < 8; s += 2)
-                if (member(s)) fold_pair(v[s], v[s | 1], 0, cc, ri == Nx);
-        }
-        if (py >= 0) {
-#pragma unroll
-            for (int s = 0; s < 8; s++)
-                if (!(s & 2) && member(s)) fold_pair(v[s], v[s | 2], 1, cc, rl == Ny);
-        }
-        if (pz >= 0) {
-#pragma unroll
-            for (int s = 0; s < 4; s++)
-                if (member(s)) fold_pair(v[s], v[s | 4], 2, cc, rk == Nz);
-        }
-#pragma unroll
-        for (int s = 0; s < 8; s++)
-            if (member(s)) J[m[s]] = v[s];
-    }
+            for (int d = 0; d < 3; d++)
+                class_pairs(c, v, d,
+                            [&](JT &r, JT &p, int) { fold_pair(r, p, d, cc, at_n[d]); });
+        });
 }
 
 /* workgroups of PIC_BLOCK threads that fold every class */

@@ -217,8 +217,8 @@ int recorded_step(pic_ctx *c, AdjointStore *s, int r) {
     const void *src[6];
     for (int k = 0; k < 6; k++) src[k] = live_field(c, k);
     launch_copy6(f.f, src, bytes, c->stream);
-    launch_record_offsets(c->g, c->t, live_count(c), live_cap(c), s->tile_sum, s->recoff[r],
-                          s->room, c->d_st, c->stream);
+    launch_record_offsets(c->g, c->t, live_count(c), live_cap(c), s->tile_sum, c->d_done,
+                          s->recoff[r], s->room, c->d_st, c->stream);
     if (c->fp32) c->rec_snap32 = s->rec32[r];
     else c->rec_snap = s->rec[r];
     c->rec_off = s->recoff[r];

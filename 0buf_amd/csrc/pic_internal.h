@@ -438,12 +438,14 @@ void launch_push_deposit_f64(const Grid &g, const TileGeom &t, FieldPtrs f, Part
                              const DiffArgs *diff, hipStream_t s);
 void launch_jfix_to_f64(const Grid &g, FieldPtrs f, DiffArgs d, hipStream_t s);
 /* compact record offsets (k_records.hip): off[t] = particles of the tiles
- * before t (counts capped at cap), off[ntiles] the total; a total beyond
+ * before t (counts capped at cap), off[ntiles] the total (tile_sum: one entry
+ * per tile, done: 0 between launches); a total beyond
  * `room` raises PIC_F_RECORD (the push writes no record entry past room) */
 /* six device arrays of `bytes` (a multiple of 4) each, in one launch */
 void launch_copy6(void *const dst[6], const void *const src[6], size_t bytes, hipStream_t s);
 void launch_record_offsets(const Grid &g, const TileGeom &t, const int *count, int cap,
-                           long *tile_sum, long *off, long room, DevStatus *st, hipStream_t s);
+                           long *tile_sum, unsigned *done, long *off, long room, DevStatus *st,
+                           hipStream_t s);
 /* the arrivals of a push and the periodic fold of the current, in one launch,
  * or one of the two */
 enum { PIC_ARRIVE = 1, PIC_FOLD = 2 };
