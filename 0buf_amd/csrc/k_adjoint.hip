@@ -227,20 +227,20 @@ __device__ __forceinline__ void pqr_adj(const double *sL, const Geo &c, const Di
                                         double by, double bz, double q, double gA[3],
                                         double gB[3]) {
 #pragma clang fp contract(fast)   /* no decision depends on the reverse sweep */
-    const double dx = (0.50 * (ax + bx) - c.hx * ((double)ix - 2.50) - c.x0);
-    const double dy = (0.50 * (ay + by) - c.hy * ((double)iy - 2.50) - c.y0);
-    const double dz = (0.50 * (az + bz) - c.hz * ((double)iz - 2.50) - c.z0);
+    const double dx = 0.50 * (ax + bx) - c.hx * ((double)ix - 2.50);
+    const double dy = 0.50 * (ay + by) - c.hy * ((double)iy - 2.50);
+    const double dz = 0.50 * (az + bz) - c.hz * ((double)iz - 2.50);
     const double dx1 = c.hx - dx, dy1 = c.hy - dy, dz1 = c.hz - dz;
     const double Dx = bx - ax, Dy = by - ay, Dz = bz - az;
     const double s1 = Dy * Dz * dc.r12, s2 = Dx * Dz * dc.r12, s3 = Dx * Dy * dc.r12;
     /* the forward deposits nothing outside the tile stencil (and flags it):
      * weight 0, at a node inside the box.  (An early return would put gA and
      * gB in scratch memory.) */
-    const bool in = ix >= 2 && ix <= 3 && iy >= 2 && iy <= 3 && iz >= 2 && iz <= 3;
+    const bool in = (unsigned)((ix - 2) | (iy - 2) | (iz - 2)) <= 1u;
     const double qi = in ? q : 0.0;
     const double kx = qi * dc.rDx, ky = qi * dc.rDy, kz = qi * dc.rDz;
     const double SU = Dx * kx, SV = Dy * ky, SW = Dz * kz;
-    const int n = in ? ((c.ca + ix - 2) * BY + c.cb + iy - 2) * BZ + c.cc + iz - 2 : 0;
+    const int n = in ? c.n0 + (ix != 2 ? BY * BZ : 0) + (iy != 2 ? BZ : 0) + iz - 2 : 0;
     const double *Lx = sL, *Ly = sL + JY0, *Lz = sL + JZ0;
     const double a0 = Lx[n], a1 = Lx[n + 1], a2 = Lx[n + BZ], a3 = Lx[n + BZ + 1];
     const double b0 = Ly[n], b1 = Ly[n + 1], b2 = Ly[n + BY * BZ], b3 = Ly[n + BY * BZ + 1];
@@ -276,28 +276,24 @@ __device__ __forceinline__ void pqr_adj(const double *sL, const Geo &c, const Di
 }
 
 /* Interpolate3D with the forward's rounding sequence (interp, k_push_math.h),
- * and the derivatives of the value with respect to sx, sy, sz, the weights of
- * the near planes (the far-plane weights are 1 - s), from the same eight
- * nodes: the reverse part needs no node again */
+ * and the derivatives of the value with respect to the far-plane weights sx1,
+ * sy1, sz1 (the near ones are 1 minus them), from the same eight nodes: the
+ * reverse part needs no node again */
 template <int BY, int BZ>
-__device__ __forceinline__ double interp_grad(const double *F, int o, double sx, double sx1,
-                                              double sy, double sy1, double sz, double sz1,
-                                              double g[3]) {
-    const double f000 = F[o], f001 = F[o + 1], f010 = F[o + BZ], f011 = F[o + BZ + 1];
-    const double f100 = F[o + BY * BZ], f101 = F[o + BY * BZ + 1];
-    const double f110 = F[o + BY * BZ + BZ], f111 = F[o + BY * BZ + BZ + 1];
-    const double z00 = sz * f000 + sz1 * f001, z01 = sz * f010 + sz1 * f011;
-    const double z10 = sz * f100 + sz1 * f101, z11 = sz * f110 + sz1 * f111;
-    const double y0 = sy * z00 + sy1 * z01, y1 = sy * z10 + sy1 * z11;
-    {
-#pragma clang fp contract(fast)
-        g[0] = y0 - y1;
-        g[1] = sx * (z00 - z01) + sx1 * (z10 - z11);
-        g[2] = sx * (sy * (f000 - f001) + sy1 * (f010 - f011)) +
-               sx1 * (sy * (f100 - f101) + sy1 * (f110 - f111));
-    }
-    const double t1 = sx * y0, t2 = sx1 * y1;
-    return t2 + t1;
+__device__ __forceinline__ double interp_grad(const double *F, int o, double sx1, double sy1,
+                                              double sz1, double g[3]) {
+    const double f00 = F[o], f01 = F[o + BZ], f10 = F[o + BY * BZ], f11 = F[o + BY * BZ + BZ];
+    const double d00 = F[o + 1] - f00, d01 = F[o + BZ + 1] - f01;
+    const double d10 = F[o + BY * BZ + 1] - f10, d11 = F[o + BY * BZ + BZ + 1] - f11;
+    const double z00 = fma(sz1, d00, f00), z01 = fma(sz1, d01, f01);
+    const double z10 = fma(sz1, d10, f10), z11 = fma(sz1, d11, f11);
+    const double e0 = z01 - z00, e1 = z11 - z10;
+    const double y0 = fma(sy1, e0, z00), y1 = fma(sy1, e1, z10);
+    const double dy0 = fma(sy1, d01 - d00, d00), dy1 = fma(sy1, d11 - d10, d10);
+    g[0] = y1 - y0;
+    g[1] = fma(sx1, e1 - e0, e0);
+    g[2] = fma(sx1, dy1 - dy0, dy0);
+    return fma(sx1, g[0], y0);
 }
 
 /* its adjoint: lam * weight into the eight nodes of the LDS adjoint box */
@@ -422,16 +418,13 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
             if (sOff[mid] <= fidx) lo = mid; else hi = mid;
         }
         const int c = lo;
-        Geo G;
-        G.ca = c / (TY * TZ);
-        G.cb = (c / TZ) % TY;
-        G.cc = c % TZ;
-        const int gi = I0 + G.ca, gl = L0 + G.cb, gk = K0 + G.cc;
+        const int ca = c / (TY * TZ), cb = (c / TZ) % TY, cc = c % TZ;
+        const int gi = I0 + ca, gl = L0 + cb, gk = K0 + cc;
         const long pidx = a.snap_off[tile] + fidx;    /* compact record */
-        G.hx = hx; G.hy = hy; G.hz = hz; G.tau = tau;
-        G.x0 = (double)gi * hx;
-        G.y0 = (double)gl * hy;
-        G.z0 = (double)gk * hz;
+        Geo G;
+        G.n0 = (ca * BY + cb) * BZ + cc;
+        G.hx = hx; G.hy = hy; G.hz = hz;
+        const double x0 = (double)gi * hx, y0 = (double)gl * hy, z0 = (double)gk * hz;
 
         const double x = a.p.p[0][pidx], y = a.p.p[1][pidx], z = a.p.p[2][pidx];
         const double pu = a.p.p[3][pidx], pv = a.p.p[4][pidx], pw = a.p.p[5][pidx];
@@ -441,12 +434,13 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
         const double tau1 = q_m * tau * 0.5;
 
         /* ---- forward recompute, the push kernel's arithmetic ---- */
-        const double frx = divc(x - G.x0, hx, a.dc.rhx);
-        const double fry = divc(y - G.y0, hy, a.dc.rhy);
-        const double frz = divc(z - G.z0, hz, a.dc.rhz);
+        const double xl = x - x0, yl = y - y0, zl = z - z0;
+        const double frx = divc(xl, hx, a.dc.rhx);
+        const double fry = divc(yl, hy, a.dc.rhy);
+        const double frz = divc(zl, hz, a.dc.rhz);
         double Ef[3] = {0, 0, 0}, Hf[3] = {0, 0, 0};
         int o[6] = {0, 0, 0, 0, 0, 0};
-        double gw[6][3] = {};   /* d(field component) / d(near weights) */
+        double gw[6][3] = {};   /* d(field component) / d(far weights) */
         const bool live = !(x < 0 || y < 0 || z < 0);
         GatherIdx W{};
         if (live) {
@@ -454,32 +448,34 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
             if (!W.ok) {
                 bad = 1;
             } else {
-                const double s1 = W.s1, s2 = W.s2, s3 = W.s3, s4 = W.s4, s5 = W.s5, s6 = W.s6;
-                const double s11 = 1. - s1, s21 = 1. - s2, s31 = 1. - s3, s41 = 1. - s4,
-                             s51 = 1. - s5, s61 = 1. - s6;
+                const double s11 = 1. - W.s1, s21 = 1. - W.s2, s31 = 1. - W.s3, s41 = 1. - W.s4,
+                             s51 = 1. - W.s5, s61 = 1. - W.s6;
                 /* node of the component's near corner in its box */
-                const int n0 = ((G.ca - 2) * BY + (G.cb - 2)) * BZ + (G.cc - 2);
-                const int bx = W.ix * (BY * BZ), bx1 = W.i1x * (BY * BZ), by = W.iy * BZ,
-                          by1 = W.i1y * BZ, bz = W.iz, bz1 = W.i1z;
-                o[0] = n0 + bx + by1 + bz1;
-                Ef[0] = interp_grad<BY, BZ>(sF + FB[0], o[0], s1, s11, s4, s41, s6, s61, gw[0]);
-                o[1] = n0 + bx1 + by + bz1;
-                Ef[1] = interp_grad<BY, BZ>(sF + FB[1], o[1], s2, s21, s3, s31, s6, s61, gw[1]);
-                o[2] = n0 + bx1 + by1 + bz;
-                Ef[2] = interp_grad<BY, BZ>(sF + FB[2], o[2], s2, s21, s4, s41, s5, s51, gw[2]);
-                o[3] = n0 + bx1 + by + bz;
-                Hf[0] = interp_grad<BY, BZ>(sF + FB[3], o[3], s2, s21, s3, s31, s5, s51, gw[3]);
-                o[4] = n0 + bx + by1 + bz;
-                Hf[1] = interp_grad<BY, BZ>(sF + FB[4], o[4], s1, s11, s4, s41, s5, s51, gw[4]);
-                o[5] = n0 + bx + by + bz1;
-                Hf[2] = interp_grad<BY, BZ>(sF + FB[5], o[5], s1, s11, s3, s31, s6, s61, gw[5]);
+                const int X = G.n0 + (W.ix != 2 ? BY * BZ : 0),
+                          X1 = G.n0 + (W.i1x != 2 ? BY * BZ : 0),
+                          Y = W.iy != 2 ? BZ : 0, Y1 = W.i1y != 2 ? BZ : 0, Z = W.iz - 2,
+                          Z1 = W.i1z - 2;
+                o[0] = X + Y1 + Z1;
+                Ef[0] = interp_grad<BY, BZ>(sF + FB[0], o[0], s11, s41, s61, gw[0]);
+                o[1] = X1 + Y + Z1;
+                Ef[1] = interp_grad<BY, BZ>(sF + FB[1], o[1], s21, s31, s61, gw[1]);
+                o[2] = X1 + Y1 + Z;
+                Ef[2] = interp_grad<BY, BZ>(sF + FB[2], o[2], s21, s41, s51, gw[2]);
+                o[3] = X1 + Y + Z;
+                Hf[0] = interp_grad<BY, BZ>(sF + FB[3], o[3], s21, s31, s51, gw[3]);
+                o[4] = X + Y1 + Z;
+                Hf[1] = interp_grad<BY, BZ>(sF + FB[4], o[4], s11, s41, s51, gw[4]);
+                o[5] = X + Y + Z1;
+                Hf[2] = interp_grad<BY, BZ>(sF + FB[5], o[5], s11, s31, s61, gw[5]);
             }
         }
-        const Boris B = boris_move(pu, pv, pw, Ef[0], Ef[1], Ef[2], Hf[0], Hf[1], Hf[2], tau1);
-        const double x1 = x + tau * (B.g2 * B.p1[0]);
-        const double y1 = y + tau * (B.g2 * B.p1[1]);
-        const double z1 = z + tau * (B.g2 * B.p1[2]);
-        const Relay R = relay_point(x, y, z, x1, y1, z1, frx, fry, frz, G, a.dc);
+        const Boris B = boris_move<true>(pu, pv, pw, Ef[0], Ef[1], Ef[2], Hf[0], Hf[1], Hf[2], tau1);
+        const double x1 = advance<true>(x, tau, B.g2, B.p1[0]) - x0,
+                     y1 = advance<true>(y, tau, B.g2, B.p1[1]) - y0,
+                     z1 = advance<true>(z, tau, B.g2, B.p1[2]) - z0;
+        const Relay R = relay_point(xl, yl, zl, x1, y1, z1, frx, fry, frz,
+                                    divc(x1, hx, a.dc.rhx), divc(y1, hy, a.dc.rhy),
+                                    divc(z1, hz, a.dc.rhz), G);
         const int m = R.m;
 
         /* ---- reverse (contracted: no decision depends on it) ---- */
@@ -488,13 +484,13 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
         double lx1[3] = {q0.x, q0.y, q1.x};
         double lp1[3] = {q1.y, q2.x, q2.y};
         double lx[3];
-        const double X0[3] = {x, y, z}, X1[3] = {x1, y1, z1};
+        const double X0[3] = {xl, yl, zl}, X1[3] = {x1, y1, z1};
         /* deposit: J = pqr(i1; x -> e1) + [m != 0] pqr(i2; x2 -> x1) */
         {
 #pragma clang fp contract(fast)
             double gA[3], gB[3];
             const double e1x = m ? R.x2x : x1, e1y = m ? R.x2y : y1, e1z = m ? R.x2z : z1;
-            pqr_adj<BY, BZ, JY0, JZ0>(sL, G, a.dc, R.i1x, R.i1y, R.i1z, x, y, z, e1x, e1y, e1z, mass,
+            pqr_adj<BY, BZ, JY0, JZ0>(sL, G, a.dc, R.i1x, R.i1y, R.i1z, xl, yl, zl, e1x, e1y, e1z, mass,
                                 gA, gB);
             lx[0] = gA[0];
             lx[1] = gA[1];
@@ -523,17 +519,15 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
                     lx[d] += v * (1.0 - R.sr);
                     lx1[d] += v * R.sr;
                 }
-                /* sr = num/den: one crossed face num = f_d - x_d, den = D_d;
-                 * two num = sum (f_d - x_d) D_d, den = sum D_d^2.  (Selected,
-                 * not branched around: a branch per axis became a computed
-                 * index, which put the arrays in scratch memory.) */
-                const int nc = (int)cr[0] + (int)cr[1] + (int)cr[2];
-                const double w = nc == 1 || nc == 2 ? lsr / R.den : 0.0;
+                /* sr = num/den over the one or two crossed faces, num = sum
+                 * (f_d - x_d) D_d, den = sum D_d^2.  (Selected, not branched
+                 * around: a branch per axis became a computed index, which
+                 * put the arrays in scratch memory.) */
+                const double w = m != 7 ? lsr / R.den : 0.0;
 #pragma unroll
                 for (int d = 0; d < 3; d++) {
                     const double D = X1[d] - X0[d], f = F[d] - X0[d];
-                    const double gx = nc == 1 ? R.sr - 1.0 : 2.0 * R.sr * D - D - f;
-                    const double gx1 = nc == 1 ? -R.sr : f - 2.0 * R.sr * D;
+                    const double gx = 2.0 * R.sr * D - D - f, gx1 = f - 2.0 * R.sr * D;
                     lx[d] += cr[d] ? w * gx : 0.0;
                     lx1[d] += cr[d] ? w * gx1 : 0.0;
                 }
@@ -591,7 +585,7 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
             for (int d = 0; d < 3; d++) lE[d] += tau1 * lpm[d];
         }
         /* gather: scatter into the adjoint box, position derivative through
-         * the weights (every s has ds/dx = -1/h) */
+         * the weights (every far weight has d/dx = 1/h) */
         if (live && W.ok) {
             interp_scatter<BY, BZ>(myA + FB[0], o[0], W.s1, 1. - W.s1, W.s4, 1. - W.s4, W.s6,
                                    1. - W.s6, lE[0]);
@@ -610,7 +604,7 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
 #pragma clang fp contract(fast)
                 const double ds = lE[0] * gw[0][d] + lE[1] * gw[1][d] + lE[2] * gw[2][d] +
                                   lH[0] * gw[3][d] + lH[1] * gw[4][d] + lH[2] * gw[5][d];
-                lx[d] -= ds * rh[d];
+                lx[d] += ds * rh[d];
             }
         }
         lq[0] = make_double2(lx[0], lx[1]);

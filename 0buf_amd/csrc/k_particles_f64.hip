@@ -14,8 +14,16 @@
  *      computed with the reference predicates; leavers go to the tile's
  *      departure region, stayers are compacted in place in flat order;
  *   4. the J box is added to the global arrays with FP64 atomics.
- * The arithmetic mirrors cell.h / particle.h in the reference's evaluation
- * order and is built with -ffp-contract=off.
+ * Decisions (cells, directions, receivers) mirror cell.h / particle.h in the
+ * reference's evaluation order; the file is built with -ffp-contract=off and
+ * writes the multiply-adds it wants fused as fma.
+ *
+ * Bound by vector issue (four fifths of its cycles), so what pays is fewer
+ * instructions a particle: coordinates relative to the owner cell, one weight
+ * factor per axis, fused segment weights, and every face test replaced by the
+ * cell that the end lies in (k_receiver.h) took 20 steps at 256x64x64 cells,
+ * 67M particles, from 68.0 to 60.6 ms, a step at 45x27x19 cells from 131 to
+ * 118 us.
  */
 #include <type_traits>
 
@@ -54,72 +62,110 @@ struct PushArgs {
     int snap_on;
 };
 
-/* one node contribution to the LDS J box: FP64 atomic add, or in the
- * differentiable form the contribution v 2^48 rounded to an integer with the
- * 1.5 2^52 shifter (exact for |v| < 8, flagged otherwise) and added as int64 */
+/* one node contribution a b to the LDS J box: FP64 atomic add, or in the
+ * differentiable form the contribution (a scaled by 2^48) rounded to an integer
+ * with the 1.5 2^52 shifter (exact for |a b| < 2^51) and added as int64 */
 template <bool DIFF>
-__device__ __forceinline__ void jadd(double *sJ, int n, double v, unsigned &bad) {
+__device__ __forceinline__ void jadd(double *sJ, int n, double a, double b) {
     if constexpr (DIFF) {
-        const double t = fma(v, PIC_J_SCALE64, 6755399441055744.0);
+        const double t = fma(a, b, 6755399441055744.0);
         const long long q = __double_as_longlong(t) - 0x4338000000000000LL;
-        if (!(fabs(v) < 8.0)) bad = 1;
         atomicAdd(reinterpret_cast<unsigned long long *>(sJ) + n, (unsigned long long)q);
     } else {
-        atomicAdd(&sJ[n], v);
+        atomicAdd(&sJ[n], a * b);
     }
 }
 
-/* cell.h:1511-1693 pqr: 12 node contributions of one straight segment,
- * accumulated into the LDS J box at local node (owner + tile index - 2). */
-template <int BY, int BZ, int NB, bool DIFF>
+/* cell.h:1511-1693 pqr: 12 node contributions of one straight segment a -> b
+ * inside dual cell (ix, iy, iz), accumulated into the LDS J box at local node
+ * (owner + tile index - 2).  Coordinates are relative to the owner cell's corner
+ * (the reference's 1/2 (a + b) - h (i - 2.5) - x0 with x0 = 0); k = weight over
+ * the face area and tau per axis, one factor where the reference multiplies by
+ * the weight and divides by the product. */
+template <int BY, int BZ, int JY0, int JZ0, bool DIFF>
 __device__ __forceinline__ void pqr_lds(double *sJ, const Geo &c, const DivConst &dc, int ix,
-                                        int iy, int iz, double xx, double xy, double xz,
-                                        double x1x, double x1y, double x1z, double a,
-                                        unsigned &bad, bool active) {
+                                        int iy, int iz, double ax, double ay, double az,
+                                        double bx, double by, double bz, double kx, double ky,
+                                        double kz, unsigned &bad, bool active) {
     if (!active) return;
-    if (ix < 2 || ix > 3 || iy < 2 || iy > 3 || iz < 2 || iz > 3) {
+    const int u = ix - 2, v = iy - 2, w = iz - 2;
+    if ((unsigned)(u | v | w) > 1u) {
         bad = 1;
         return;
     }
-    double dx = (0.50 * (xx + x1x) - c.hx * ((double)ix - 2.50) - c.x0);
-    double dy = (0.50 * (xy + x1y) - c.hy * ((double)iy - 2.50) - c.y0);
-    double dz = (0.50 * (xz + x1z) - c.hz * ((double)iz - 2.50) - c.z0);
-    double dx1 = c.hx - dx, dy1 = c.hy - dy, dz1 = c.hz - dz;
-    double su = x1x - xx, sv = x1y - xy, sw = x1z - xz;
-    double s1 = divc(sv * sw, 12.0, dc.r12), s2 = divc(su * sw, 12.0, dc.r12),
-           s3 = divc(su * sv, 12.0, dc.r12);
-    su = divc(su * a, dc.Dx, dc.rDx);
-    sv = divc(sv * a, dc.Dy, dc.rDy);
-    sw = divc(sw * a, dc.Dz, dc.rDz);
-    const int u = c.ca + ix - 2, v = c.cb + iy - 2, w = c.cc + iz - 2;
-    const int n = (u * BY + v) * BZ + w;
-    double *Jx = sJ, *Jy = sJ + NB, *Jz = sJ + 2 * NB;
-    /* plain form: one rounding less per weight than the reference's product
-     * and sum (the order of the atomic sums moves J by more); the
-     * differentiable form, whose sums have no order, keeps both */
-    auto weight = [](double a, double b, double s) { return DIFF ? a * b + s : fma(a, b, s); };
-    jadd<DIFF>(Jx, n, su * weight(dy1, dz1, s1), bad);
-    jadd<DIFF>(Jx, n + 1, su * weight(dy1, dz, -s1), bad);
-    jadd<DIFF>(Jx, n + BZ, su * weight(dy, dz1, -s1), bad);
-    jadd<DIFF>(Jx, n + BZ + 1, su * weight(dy, dz, s1), bad);
-    jadd<DIFF>(Jy, n, sv * weight(dx1, dz1, s2), bad);
-    jadd<DIFF>(Jy, n + 1, sv * weight(dx1, dz, -s2), bad);
-    jadd<DIFF>(Jy, n + BY * BZ, sv * weight(dx, dz1, -s2), bad);
-    jadd<DIFF>(Jy, n + BY * BZ + 1, sv * weight(dx, dz, s2), bad);
-    jadd<DIFF>(Jz, n, sw * weight(dx1, dy1, s3), bad);
-    jadd<DIFF>(Jz, n + BZ, sw * weight(dx1, dy, -s3), bad);
-    jadd<DIFF>(Jz, n + BY * BZ, sw * weight(dx, dy1, -s3), bad);
-    jadd<DIFF>(Jz, n + BY * BZ + BZ, sw * weight(dx, dy, s3), bad);
+    const double dx = fma(0.5, ax + bx, u ? -0.5 * c.hx : 0.5 * c.hx);
+    const double dy = fma(0.5, ay + by, v ? -0.5 * c.hy : 0.5 * c.hy);
+    const double dz = fma(0.5, az + bz, w ? -0.5 * c.hz : 0.5 * c.hz);
+    const double dx1 = c.hx - dx, dy1 = c.hy - dy, dz1 = c.hz - dz;
+    double su = bx - ax, sv = by - ay, sw = bz - az;
+    const double su12 = su * dc.r12;
+    const double s1 = (sv * dc.r12) * sw, s2 = su12 * sw, s3 = su12 * sv;
+    su *= kx;
+    sv *= ky;
+    sw *= kz;
+    const int n = c.n0 + (u ? BY * BZ : 0) + (v ? BZ : 0) + w;
+    double *Jx = sJ, *Jy = sJ + JY0, *Jz = sJ + JZ0;
+    const double wx0 = fma(dy1, dz1, s1), wx1 = fma(dy1, dz, -s1), wx2 = fma(dy, dz1, -s1),
+                 wx3 = fma(dy, dz, s1);
+    const double wy0 = fma(dx1, dz1, s2), wy1 = fma(dx1, dz, -s2), wy2 = fma(dx, dz1, -s2),
+                 wy3 = fma(dx, dz, s2);
+    const double wz0 = fma(dx1, dy1, s3), wz1 = fma(dx1, dy, -s3), wz2 = fma(dx, dy1, -s3),
+                 wz3 = fma(dx, dy, s3);
+    if constexpr (DIFF) {
+        /* every contribution below 8 (2^51 units): a weight inside the dual
+         * cell is at most 13/12 of the face; where that bound does not tell,
+         * the contributions themselves */
+        if (!(fabs(su) * dc.face[0] < 4.0 && fabs(sv) * dc.face[1] < 4.0 &&
+              fabs(sw) * dc.face[2] < 4.0)) {
+            auto over = [](double a, double w0, double w1, double w2, double w3) {
+                return !(fabs(a * w0) < 8.0 && fabs(a * w1) < 8.0 && fabs(a * w2) < 8.0 &&
+                         fabs(a * w3) < 8.0);
+            };
+            if (over(su, wx0, wx1, wx2, wx3) || over(sv, wy0, wy1, wy2, wy3) ||
+                over(sw, wz0, wz1, wz2, wz3))
+                bad = 1;
+        }
+        su *= PIC_J_SCALE64;
+        sv *= PIC_J_SCALE64;
+        sw *= PIC_J_SCALE64;
+    }
+    jadd<DIFF>(Jx, n, su, wx0);
+    jadd<DIFF>(Jx, n + 1, su, wx1);
+    jadd<DIFF>(Jx, n + BZ, su, wx2);
+    jadd<DIFF>(Jx, n + BZ + 1, su, wx3);
+    jadd<DIFF>(Jy, n, sv, wy0);
+    jadd<DIFF>(Jy, n + 1, sv, wy1);
+    jadd<DIFF>(Jy, n + BY * BZ, sv, wy2);
+    jadd<DIFF>(Jy, n + BY * BZ + 1, sv, wy3);
+    jadd<DIFF>(Jz, n, sw, wz0);
+    jadd<DIFF>(Jz, n + BZ, sw, wz1);
+    jadd<DIFF>(Jz, n + BY * BZ, sw, wz2);
+    jadd<DIFF>(Jz, n + BY * BZ + BZ, sw, wz3);
+}
+
+/* flyDirection (cell.h:694-701) along one axis: 0, 1, 2 */
+__device__ __forceinline__ int flies(double v, double v0, double h, int i, int n, double L) {
+    return ((v > v0 + h) && (v < v0 + 2 * h)) || ((v < h) && (i == n - 1))
+               ? 2
+               : ((v < v0) || ((v > L - h) && (i == 0)) ? 0 : 1);
 }
 
 /* 4 waves per SIMD (at most 128 VGPRs): the FP64 chains of the push are
  * latency-bound at 3 */
-template <int TX, int TY, int TZ, bool DIFF, int NT>
+template <int TX, int TY, int TZ, bool DIFF, bool TAPE, int NT>
 __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
     constexpr int C = TX * TY * TZ;
     constexpr int BX = TX + 2, BY = TY + 2, BZ = TZ + 2, NB = BX * BY * BZ;
-    __shared__ double sF[6 * NB];
-    __shared__ double sJ[JCOPIES * 3 * NB];
+    /* the current box: Jx (dual along x) takes x planes 0..TX only, Jy and Jz
+     * all of them; copies JS apart, 8 mod 16 doubles, so that the two copies'
+     * nodes of a cell lie on other banks */
+    constexpr int NBX = (TX + 1) * BY * BZ;
+    constexpr int JY0 = NBX, JZ0 = NBX + NB, NJ = NBX + 2 * NB, JS = (NJ + 15) / 16 * 16 + 8;
+    /* field boxes; the differentiable form keeps (value, difference to the
+     * next node along z) */
+    using Node = std::conditional_t<DIFF, double2, double>;
+    __shared__ Node sF[6 * NB];
+    __shared__ double sJ[JCOPIES * JS];
     __shared__ int sOff[C + 1];
     __shared__ int sCnt[C];
     __shared__ int sLeave[C];
@@ -129,9 +175,9 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
     __shared__ int sQ;
     __shared__ unsigned sFlags;
     __shared__ unsigned long long sDrop, sDup;
-    __shared__ double2 sMQ[PIC_MAX_SLOTS];   /* (m, q_m) per species slot */
+    __shared__ double sSpec[PIC_MAX_SLOTS][4];   /* q/m tau/2 and m over Dx, Dy, Dz per species slot */
     extern __shared__ unsigned sGrp[];    /* line groups of the tile */
-    double *const myJ = sJ + (threadIdx.x % JCOPIES) * (3 * NB);
+    double *const myJ = sJ + (threadIdx.x % JCOPIES) * JS;
 
     const Grid &g = a.g;
     const int tid = threadIdx.x;
@@ -165,12 +211,16 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
                          K0 + nw <= g.Nz + 1;
     const unsigned noff = (unsigned)(I0 + nu) * g.sx + (unsigned)(L0 + nv) * g.sy + (K0 + nw);
     {
-        double fv[6];
+        double fv[6], fd[6];   /* node value, next node's value (0 outside the grid) */
 #pragma unroll
-        for (int q = 0; q < 6; q++) fv[q] = 0.0;
+        for (int q = 0; q < 6; q++) fv[q] = fd[q] = 0.0;
         if (node_in) {
 #pragma unroll
             for (int q = 0; q < 6; q++) fv[q] = a.f.f[PIC_EX + q][noff];
+        }
+        if (DIFF && node_in && nw + 1 < BZ && K0 + nw + 1 <= g.Nz + 1) {
+#pragma unroll
+            for (int q = 0; q < 6; q++) fd[q] = a.f.f[PIC_EX + q][noff + 1];
         }
         const int ca = tid / (TY * TZ), cb = (tid / TZ) % TY, cc = tid % TZ;
         const int gi = I0 + ca, gl = L0 + cb, gk = K0 + cc;
@@ -183,7 +233,10 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
         }
         if (tid < NB) {
 #pragma unroll
-            for (int q = 0; q < 6; q++) sF[q * NB + tid] = fv[q];
+            for (int q = 0; q < 6; q++) {
+                if constexpr (DIFF) sF[q * NB + tid] = make_double2(fv[q], fd[q] - fv[q]);
+                else sF[q * NB + tid] = fv[q];
+            }
         }
         if (tid < C) {
             sCnt[tid] = cnt;
@@ -192,11 +245,16 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
             sBase[tid] = ((ca * g.Ny + cb) * g.Nz + cc) * cap;
         }
     }
-    for (int e = tid; e < JCOPIES * 3 * NB; e += NT) sJ[e] = 0.0;
-    /* weight and q/m per species slot: a kernel-argument table indexed by a
+    for (int e = tid; e < JCOPIES * JS; e += NT) sJ[e] = 0.0;
+    /* the factors of each species slot: a kernel-argument table indexed by a
      * per-particle value would be a vector memory load in the loop, whose
      * wait would also wait for the particle loads in flight */
-    if (tid < PIC_MAX_SLOTS) sMQ[tid] = make_double2(a.sp.m[tid], a.sp.q_m[tid]);
+    if (tid < PIC_MAX_SLOTS) {
+        sSpec[tid][0] = a.sp.q_m[tid] * g.tau * 0.5;
+        sSpec[tid][1] = a.sp.m[tid] / a.dc.Dx;
+        sSpec[tid][2] = a.sp.m[tid] / a.dc.Dy;
+        sSpec[tid][3] = a.sp.m[tid] / a.dc.Dz;
+    }
     if (tid == 0) {
         sQ = 0;
         sFlags = 0;
@@ -262,15 +320,12 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
             c = group_cell(ge);
             j = group_start(ge) + (lane - (63 - __clzll(msk))) + (gidx == 0 ? o0 : 0);
             const unsigned rel = (unsigned)(sBase[c] + j);
+            const int ca = c / (TY * TZ), cb = (c / TZ) % TY, cc = c % TZ;
+            const int gi = I0 + ca, gl = L0 + cb, gk = K0 + cc;
             Geo G;
-            G.ca = c / (TY * TZ);
-            G.cb = (c / TZ) % TY;
-            G.cc = c % TZ;
-            const int gi = I0 + G.ca, gl = L0 + G.cb, gk = K0 + G.cc;
-            G.hx = hx; G.hy = hy; G.hz = hz; G.tau = tau;
-            G.x0 = (double)gi * hx;
-            G.y0 = (double)gl * hy;
-            G.z0 = (double)gk * hz;
+            G.n0 = (int)__umul24(__umul24((unsigned)ca, BY) + (unsigned)cb, BZ) + cc;
+            G.hx = hx; G.hy = hy; G.hz = hz;
+            const double x0 = (double)gi * hx, y0 = (double)gl * hy, z0 = (double)gk * hz;
 
             const double x = slot(P0, rel), y = slot(P1, rel), z = slot(P2, rel);
             pu = slot(P3, rel);
@@ -278,12 +333,10 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
             pw = slot(P5, rel);
             s = slot(SP, rel);
             pid = DIFF ? slot(ID, rel) : 0;
-            const double2 mq = sMQ[s];
-            const double mass = mq.x, q_m = mq.y;
             /* decision tape (differentiable form): record this step's
              * decisions, or replay a recorded run's */
-            const bool trec = DIFF && a.d.tape_mode == PIC_TAPE_RECORD;
-            bool trep = DIFF && a.d.tape_mode == PIC_TAPE_REPLAY;
+            const bool trec = TAPE && a.d.tape_mode == PIC_TAPE_RECORD;
+            const bool trep = TAPE && a.d.tape_mode == PIC_TAPE_REPLAY;
             const bool tin = (trec || trep) && pid >= 0 && pid < a.d.tape_n;
             tape_word tw = 0;
             if (trep) {
@@ -302,9 +355,11 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
                 a.d.snap.id[r] = pid;
             }
 
-            const double frx = divc(x - G.x0, hx, a.dc.rhx);
-            const double fry = divc(y - G.y0, hy, a.dc.rhy);
-            const double frz = divc(z - G.z0, hz, a.dc.rhz);
+            /* relative to the owner cell's corner */
+            const double xl = x - x0, yl = y - y0, zl = z - z0;
+            const double frx = divc(xl, hx, a.dc.rhx);
+            const double fry = divc(yl, hy, a.dc.rhy);
+            const double frz = divc(zl, hz, a.dc.rhz);
             double Ex = 0, Ey = 0, Ez = 0, Hx = 0, Hy = 0, Hz = 0;
             const bool neg = trep ? (tw & 1ull) != 0 : (x < 0 || y < 0 || z < 0);
             if (trec && neg) tout |= 1ull;
@@ -331,41 +386,46 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
                     }
                 }
                 const double s1 = W.s1, s2 = W.s2, s3 = W.s3, s4 = W.s4, s5 = W.s5, s6 = W.s6;
-                const double s11 = 1. - s1, s21 = 1. - s2, s31 = 1. - s3, s41 = 1. - s4,
-                             s51 = 1. - s5, s61 = 1. - s6;
+                const double s11 = 1. - W.s1, s21 = 1. - W.s2, s31 = 1. - W.s3, s41 = 1. - W.s4,
+                             s51 = 1. - W.s5, s61 = 1. - W.s6;
                 if (!W.ok) {
                     bad = 1;
                 } else {
-                    const int ua = G.ca - 2, va = G.cb - 2, wa = G.cc - 2;
-                    Ex = interp<BY, BZ>(sF + 0 * NB, ua + W.ix, va + W.i1y, wa + W.i1z, s1, s11, s4, s41, s6, s61);
-                    Ey = interp<BY, BZ>(sF + 1 * NB, ua + W.i1x, va + W.iy, wa + W.i1z, s2, s21, s3, s31, s6, s61);
-                    Ez = interp<BY, BZ>(sF + 2 * NB, ua + W.i1x, va + W.i1y, wa + W.iz, s2, s21, s4, s41, s5, s51);
-                    Hx = interp<BY, BZ>(sF + 3 * NB, ua + W.i1x, va + W.iy, wa + W.iz, s2, s21, s3, s31, s5, s51);
-                    Hy = interp<BY, BZ>(sF + 4 * NB, ua + W.ix, va + W.i1y, wa + W.iz, s1, s11, s4, s41, s5, s51);
-                    Hz = interp<BY, BZ>(sF + 5 * NB, ua + W.ix, va + W.iy, wa + W.i1z, s1, s11, s3, s31, s6, s61);
+                    const int X = G.n0 + (W.ix != 2 ? BY * BZ : 0),
+                              X1 = G.n0 + (W.i1x != 2 ? BY * BZ : 0),
+                              Y = W.iy != 2 ? BZ : 0, Y1 = W.i1y != 2 ? BZ : 0, Z = W.iz - 2,
+                              Z1 = W.i1z - 2;
+                    Ex = interp<BY, BZ>(sF + 0 * NB, X + Y1 + Z1, s11, s41, s61, s1, s4, s6);
+                    Ey = interp<BY, BZ>(sF + 1 * NB, X1 + Y + Z1, s21, s31, s61, s2, s3, s6);
+                    Ez = interp<BY, BZ>(sF + 2 * NB, X1 + Y1 + Z, s21, s41, s51, s2, s4, s5);
+                    Hx = interp<BY, BZ>(sF + 3 * NB, X1 + Y + Z, s21, s31, s51, s2, s3, s5);
+                    Hy = interp<BY, BZ>(sF + 4 * NB, X + Y1 + Z, s11, s41, s51, s1, s4, s5);
+                    Hz = interp<BY, BZ>(sF + 5 * NB, X + Y + Z1, s11, s31, s61, s1, s3, s6);
                 }
             }
 
             /* Particle::Move (particle.h:160-202) */
-            const Boris B = boris_move(pu, pv, pw, Ex, Ey, Ez, Hx, Hy, Hz, q_m * tau * 0.5);
+            const Boris B = boris_move<DIFF>(pu, pv, pw, Ex, Ey, Ez, Hx, Hy, Hz, sSpec[s][0]);
             pu = B.p1[0];
             pv = B.p1[1];
             pw = B.p1[2];
-            const double x1 = x + tau * (B.g2 * pu);
-            const double y1 = y + tau * (B.g2 * pv);
-            const double z1 = z + tau * (B.g2 * pw);
+            const double x1 = advance<DIFF>(x, tau, B.g2, pu), y1 = advance<DIFF>(y, tau, B.g2, pv),
+                         z1 = advance<DIFF>(z, tau, B.g2, pw);
+            const double x1l = x1 - x0, y1l = y1 - y0, z1l = z1 - z0;
+            const double t1x = divc(x1l, hx, a.dc.rhx), t1y = divc(y1l, hy, a.dc.rhy),
+                         t1z = divc(z1l, hz, a.dc.rhz);
 
             /* CurrentToMesh (cell.h:1306-1422): one code path for every lane;
              * without a crossing the first segment is the whole path (x2 = x1)
              * and the second is skipped */
             {
                 const Relay R =
-                    trep ? relay_from(x, y, z, x1, y1, z1, G, tape_get(tw, TAPE_RI1, 1, 2),
+                    trep ? relay_from(xl, yl, zl, x1l, y1l, z1l, G, tape_get(tw, TAPE_RI1, 1, 2),
                                       tape_get(tw, TAPE_RI1 + 1, 1, 2),
                                       tape_get(tw, TAPE_RI1 + 2, 1, 2),
                                       tape_get(tw, TAPE_RI2, 2, 1), tape_get(tw, TAPE_RI2 + 2, 2, 1),
                                       tape_get(tw, TAPE_RI2 + 4, 2, 1))
-                         : relay_point(x, y, z, x1, y1, z1, frx, fry, frz, G, a.dc);
+                         : relay_point(xl, yl, zl, x1l, y1l, z1l, frx, fry, frz, t1x, t1y, t1z, G);
                 if (trec) {
                     tape_put(tout, TAPE_RI1, 1, R.i1x, 2);
                     tape_put(tout, TAPE_RI1 + 1, 1, R.i1y, 2);
@@ -375,51 +435,67 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
                     tape_put(tout, TAPE_RI2 + 4, 2, R.i2z, 1);
                 }
                 const int m = R.m;
-                const double e1x = m ? R.x2x : x1, e1y = m ? R.x2y : y1, e1z = m ? R.x2z : z1;
-                pqr_lds<BY, BZ, NB, DIFF>(myJ, G, a.dc, R.i1x, R.i1y, R.i1z, x, y, z, e1x, e1y, e1z,
-                                          mass, bad, true);
+                const double e1x = m ? R.x2x : x1l, e1y = m ? R.x2y : y1l, e1z = m ? R.x2z : z1l;
+                const double kx = sSpec[s][1], ky = sSpec[s][2], kz = sSpec[s][3];
+                pqr_lds<BY, BZ, JY0, JZ0, DIFF>(myJ, G, a.dc, R.i1x, R.i1y, R.i1z, xl, yl, zl, e1x,
+                                                e1y, e1z, kx, ky, kz, bad, true);
                 /* (kept waiting in registers until a lane has a second one, as
                  * the FP32 push does, they spill at 128 VGPRs: 2.47 against
                  * 2.38 ms at 67M particles) */
-                pqr_lds<BY, BZ, NB, DIFF>(myJ, G, a.dc, R.i2x, R.i2y, R.i2z, R.x2x, R.x2y, R.x2z, x1,
-                                          y1, z1, mass, bad, m != 0);
+                pqr_lds<BY, BZ, JY0, JZ0, DIFF>(myJ, G, a.dc, R.i2x, R.i2y, R.i2z, R.x2x, R.x2y,
+                                                R.x2z, x1l, y1l, z1l, kx, ky, kz, bad, m != 0);
             }
 
-            /* x <- x1, Reflect (cell.h:1410-1478) */
-            if (DIFF && (trec || trep)) {
-                const double v1[3] = {x1, y1, z1}, Lm[3] = {g.Lx, g.Ly, g.Lz};
-                double vn[3];
-                for (int d = 0; d < 3; d++) {
-                    const int k = trep ? tape_get(tw, TAPE_REFL + 2 * d, 2, 0)
-                                       : reflect_case(v1[d], Lm[d]);
-                    if (trec) tape_put(tout, TAPE_REFL + 2 * d, 2, k, 0);
-                    vn[d] = reflect_apply(v1[d], Lm[d], k);
+            /* x <- x1, Reflect (cell.h:1410-1478), flyDirection (cell.h:694-701) with
+             * the owner cell's geometry, the test of the own cell, and the
+             * receivers: GPU_ArrangeFlights (kernels.cu:316-370) gives every bulk
+             * cell of the 27-neighbourhood (getWrapCellNumber) whose isPointInCell
+             * (cell.h:717) holds a copy; per axis the test is separable, so the
+             * receivers are a product of per-axis sets, bit d+1 set when
+             * neighbour d in {-1,0,1} accepts.  All follow from the cell that x1
+             * lies in; the tests themselves only where some lane lies near a face
+             * (axis_step), and for the decision tape. */
+            int dx = 0, dy = 0, dz = 0;
+            bool near = TAPE;
+            if (!TAPE) {
+                xn = axis_step(x1, t1x, gi, g.Nx, g.Lx, dx, near);
+                yn = axis_step(y1, t1y, gl, g.Ny, g.Ly, dy, near);
+                zn = axis_step(z1, t1z, gk, g.Nz, g.Lz, dz, near);
+            }
+            stays = (dx | dy | dz) == 0;
+            bool inside = stays;
+            unsigned bx = 1u << (dx + 1), by = 1u << (dy + 1), bz = 1u << (dz + 1);
+            if (near) {
+                if (TAPE && (trec || trep)) {
+                    const double v1[3] = {x1, y1, z1}, Lm[3] = {g.Lx, g.Ly, g.Lz};
+                    double vn[3];
+                    for (int d = 0; d < 3; d++) {
+                        const int k = trep ? tape_get(tw, TAPE_REFL + 2 * d, 2, 0)
+                                           : reflect_case(v1[d], Lm[d]);
+                        if (trec) tape_put(tout, TAPE_REFL + 2 * d, 2, k, 0);
+                        vn[d] = reflect_apply(v1[d], Lm[d], k);
+                    }
+                    xn = vn[0];
+                    yn = vn[1];
+                    zn = vn[2];
+                } else {
+                    xn = reflect1(x1, g.Lx);
+                    yn = reflect1(y1, g.Ly);
+                    zn = reflect1(z1, g.Lz);
                 }
-                xn = vn[0];
-                yn = vn[1];
-                zn = vn[2];
-            } else {
-                xn = reflect1(x1, g.Lx);
-                yn = reflect1(y1, g.Ly);
-                zn = reflect1(z1, g.Lz);
+                stays = flies(xn, x0, hx, gi, g.Nx, g.Lx) == 1 &&
+                        flies(yn, y0, hy, gl, g.Ny, g.Ly) == 1 &&
+                        flies(zn, z0, hz, gk, g.Nz, g.Lz) == 1;
+                inside = (x0 <= xn) && (xn < x0 + hx) && (y0 <= yn) && (yn < y0 + hy) &&
+                         (z0 <= zn) && (zn < z0 + hz);
+                if (!stays || TAPE) {
+                    bx = receivers(xn, hx, gi, g.Nx);
+                    by = receivers(yn, hy, gl, g.Ny);
+                    bz = receivers(zn, hz, gk, g.Nz);
+                }
             }
-
-            /* flyDirection (cell.h:694-701) with the owner cell's geometry */
-            int ddx = (((xn > G.x0 + hx) && (xn < G.x0 + 2 * hx)) || ((xn < hx) && (gi == g.Nx - 1)))
-                          ? 2
-                          : (((xn < G.x0) || ((xn > g.Lx - hx) && (gi == 0))) ? 0 : 1);
-            int ddy = (((yn > G.y0 + hy) && (yn < G.y0 + 2 * hy)) || ((yn < hy) && (gl == g.Ny - 1)))
-                          ? 2
-                          : (((yn < G.y0) || ((yn > g.Ly - hy) && (gl == 0))) ? 0 : 1);
-            int ddz = (((zn > G.z0 + hz) && (zn < G.z0 + 2 * hz)) || ((zn < hz) && (gk == g.Nz - 1)))
-                          ? 2
-                          : (((zn < G.z0) || ((zn > g.Lz - hz) && (gk == 0))) ? 0 : 1);
-            const int dir = ddx * 9 + ddy * 3 + ddz;
-            const bool inside = (G.x0 <= xn) && (xn < G.x0 + hx) && (G.y0 <= yn) &&
-                                (yn < G.y0 + hy) && (G.z0 <= zn) && (zn < G.z0 + hz);
             if (!inside) atomicAdd(&sOut[c], 1);
 
-            stays = dir == 13;
             /* a replayed word that cannot be trusted keeps its particle in
              * place (the step reports PIC_F_RANGE) */
             if (trep) stays = ((tw >> TAPE_STAY) & 1ull) || !tin ||
@@ -427,21 +503,6 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
             if (trec && stays) tout |= 1ull << TAPE_STAY;
             if (!stays) {
                 atomicAdd(&sLeave[c], 1);
-                /* GPU_ArrangeFlights (kernels.cu:316-370): every bulk cell of the
-                 * 27-neighbourhood (getWrapCellNumber) whose isPointInCell
-                 * (cell.h:717) holds receives a copy; per axis the test is
-                 * separable, so the receivers are a product of per-axis sets. */
-                /* per axis, bit d+1 set when neighbour d in {-1,0,1} accepts;
-                 * the test of all three only where some lane lies near a face */
-                bool near = false;
-                unsigned bx = receiver(xn, a.dc.rhx, gi, g.Nx, near),
-                         by = receiver(yn, a.dc.rhy, gl, g.Ny, near),
-                         bz = receiver(zn, a.dc.rhz, gk, g.Nz, near);
-                if (near) {
-                    bx = receivers(xn, hx, gi, g.Nx);
-                    by = receivers(yn, hy, gl, g.Ny);
-                    bz = receivers(zn, hz, gk, g.Nz);
-                }
                 if (trec) {
                     const unsigned bb[3] = {bx, by, bz};
                     for (int d = 0; d < 3; d++) {
@@ -470,7 +531,8 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
                         if (rx >= g.Nx) rx -= g.Nx; else if (rx < 0) rx += g.Nx;
                         if (ry >= g.Ny) ry -= g.Ny; else if (ry < 0) ry += g.Ny;
                         if (rz >= g.Nz) rz -= g.Nz; else if (rz < 0) rz += g.Nz;
-                        const int h = ((G.ca + ax) * BY + (G.cb + ay)) * BZ + (G.cc + az);
+                        const int h = G.n0 + (int)__umul24((unsigned)ax, BY * BZ) +
+                                      (int)__umul24((unsigned)ay, BZ) + az;
                         Leaver64 &e = slot(QT, (unsigned)idx);
                         e.xy = make_double2(xn, yn);
                         e.zu = make_double2(zn, pu);
@@ -500,7 +562,7 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
             }
         }
 
-        if constexpr (DIFF) {
+        if constexpr (TAPE) {
             if (valid && a.d.tape_mode == PIC_TAPE_RECORD && pid >= 0 && pid < a.d.tape_n)
                 a.d.tape_row[pid] = tout | (1ull << TAPE_VALID);
         }
@@ -543,16 +605,18 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
     if (tid < NB) {   /* thread n adds box node n of the three components */
 #pragma unroll
         for (int comp = 0; comp < 3; comp++) {
-            const int e = comp * NB + tid;
+            constexpr int J0[3] = {0, JY0, JZ0};
+            if (comp == 0 && tid >= NBX) continue;
+            const int e = J0[comp] + tid;
             if constexpr (DIFF) {
                 const unsigned long long *u = reinterpret_cast<const unsigned long long *>(sJ);
                 unsigned long long val = u[e];
-                for (int r = 1; r < JCOPIES; r++) val += u[r * 3 * NB + e];
+                for (int r = 1; r < JCOPIES; r++) val += u[r * JS + e];
                 if (val != 0ull && node_in)
                     atomicAdd(reinterpret_cast<unsigned long long *>(a.d.jfix[comp]) + noff, val);
             } else {
                 double val = sJ[e];
-                for (int r = 1; r < JCOPIES; r++) val += sJ[r * 3 * NB + e];
+                for (int r = 1; r < JCOPIES; r++) val += sJ[r * JS + e];
                 if (val != 0.0 && node_in) atomicAdd(&a.f.f[PIC_JX + comp][noff], val);
             }
         }
@@ -718,18 +782,21 @@ void launch_push_deposit_f64(const Grid &g, const TileGeom &t, FieldPtrs f, Part
     /* dynamic LDS: one 4-byte entry per line group */
     const size_t lds = (size_t)4 * TXC * TYC * TZC * ((p.cap + GS64 - 1) / GS64);
     const int nt = push_threads(t.ntiles);
-    auto launch = [&](auto diff_on, auto threads) {
+    const bool tape = diff && diff->tape_mode != PIC_TAPE_OFF;
+    auto launch = [&](auto diff_on, auto tape_on, auto threads) {
         constexpr int NT = decltype(threads)::value;
-        hipLaunchKernelGGL((k_push_deposit<TXC, TYC, TZC, decltype(diff_on)::value, NT>),
+        hipLaunchKernelGGL((k_push_deposit<TXC, TYC, TZC, decltype(diff_on)::value,
+                                           decltype(tape_on)::value, NT>),
                            dim3((unsigned)t.ntiles), dim3(NT), lds, s, a);
     };
-    auto with_threads = [&](auto diff_on) {
-        if (nt == 1024) launch(diff_on, std::integral_constant<int, 1024>());
-        else if (nt == 512) launch(diff_on, std::integral_constant<int, 512>());
-        else launch(diff_on, std::integral_constant<int, PIC_BLOCK>());
+    auto with_threads = [&](auto diff_on, auto tape_on) {
+        if (nt == 1024) launch(diff_on, tape_on, std::integral_constant<int, 1024>());
+        else if (nt == 512) launch(diff_on, tape_on, std::integral_constant<int, 512>());
+        else launch(diff_on, tape_on, std::integral_constant<int, PIC_BLOCK>());
     };
-    if (diff) with_threads(std::true_type());
-    else with_threads(std::false_type());
+    if (tape) with_threads(std::true_type(), std::true_type());
+    else if (diff) with_threads(std::true_type(), std::false_type());
+    else with_threads(std::false_type(), std::false_type());
 }
 
 void launch_jfix_to_f64(const Grid &g, FieldPtrs f, DiffArgs d, hipStream_t s) {

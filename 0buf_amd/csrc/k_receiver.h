@@ -1,5 +1,6 @@
 /*
- * k_receiver.h -- which cells of an axis take a leaver of the FP64 push.
+ * k_receiver.h -- where a particle of the FP64 push ends along an axis, and
+ * which cells take it.
  *
  * The reference offers a leaver to every cell of its neighbourhood, and a
  * cell r takes it when r h <= v < r h + h (isPointInCell, cell.h:717) with
@@ -31,17 +32,19 @@ PIC_RHD unsigned receivers(double v, double h, int i, int n) {
     return b;
 }
 
-/* the same from one product with rh = 1/h: away from the cells' faces only
- * the cell trunc(v/h) takes v.  `near` is set where that cannot be told this
- * way: v within 1e-6 h of a face (far more than the rounding of v rh below
- * 2^31 cells), negative, or in no cell of the neighbourhood.  For n >= 3. */
-PIC_RHD unsigned receiver(double v, double rh, int i, int n, bool &near) {
-    const double t = v * rh, c = trunc(t), f = t - c;
-    const bool inner = f > 1e-6 && f < 1.0 - 1e-6 && t < (double)n;
-    int d = (inner ? (int)c : i) - i;
-    if (d > 1) d -= n; else if (d < -1) d += n;
-    if (!inner || d < -1 || d > 1) near = true;
-    return 1u << ((d + 1) & 3);
+/* One axis of a move that ends well inside a cell: v1 = where the straight path
+ * from cell i (of n >= 3) ends, t = (v1 - i h)/h.  Returns the position wrapped
+ * into [0, L) and d in {-1, 0, 1}, the cell it lies in less i.  Reflect, the fly
+ * direction, the test of the own cell and the receivers all follow from d alone
+ * there.  `near` is set where they may not: v1 within 1e-6 h of a face (far more
+ * than the rounding of i h below 2^31 cells), past the neighbours, or NaN. */
+PIC_RHD double axis_step(double v1, double t, int i, int n, double L, int &d, bool &near) {
+    const double c = floor(t);
+    const bool inner = fabs(t - c - 0.5) < 0.5 - 1e-6 && c >= -1.0 && c <= 1.0;
+    if (!inner) near = true;
+    d = inner ? (int)c : 0;
+    const int r = i + d;
+    return v1 + (r >= n ? -L : r < 0 ? L : 0.0);
 }
 
 #endif

@@ -1,12 +1,13 @@
-"""The short form of the FP64 push's receiver test against the reference's test
-of every neighbour, compiled for the CPU (tests/cpu/receiver_check.cpp)."""
+"""The short form of the FP64 push's move along an axis against the reference's
+tests of cell, direction and receivers, compiled for the CPU
+(tests/cpu/receiver_check.cpp)."""
 import os
 import subprocess
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-def test_receiver_short_form(tmp_path):
+def test_axis_step(tmp_path):
     exe = tmp_path / "receiver_check"
     subprocess.run(["g++", "-std=c++17", "-O2", "-ffp-contract=off", "-Wall", "-Werror", "-I",
                     os.path.join(ROOT, "0buf_amd", "csrc"),
