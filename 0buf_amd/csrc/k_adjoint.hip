@@ -345,15 +345,9 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
 
     const Grid &g = a.g;
     const int tid = threadIdx.x;
-    long tile;
-    {
-        long nt = a.t.ntiles, b = blockIdx.x;
-        long q = nt / 8, r = nt % 8, x = b % 8;
-        tile = x * q + (x < r ? x : r) + b / 8;
-    }
-    const int tz = (int)(tile % a.t.ntz);
-    const int ty = (int)((tile / a.t.ntz) % a.t.nty);
-    const int tx = (int)(tile / ((long)a.t.ntz * a.t.nty));
+    const TileAt at = tile_of_block(a.t, blockIdx.x);
+    const long tile = at.tile;
+    const int tx = at.tx, ty = at.ty, tz = at.tz;
     const int I0 = tx * TX, L0 = ty * TY, K0 = tz * TZ;
     const int cap = a.p.cap;
 
@@ -398,13 +392,11 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
     for (int e = tid; e < ACOPIES * AS; e += NT) sA[e] = 0.0;
     if (tid == 0) sFlags = 0;
     __syncthreads();
-    if (tid == 0) {
-        int s = 0;
-        for (int c = 0; c < C; c++) {
-            sOff[c] = s;
-            s += sCnt[c];
-        }
-        sOff[C] = s;
+    static_assert(C == 64, "one wavefront scans the tile's cells");
+    if (tid < 64) {
+        int total;
+        sOff[tid] = wave_excl_scan(sCnt[tid], total);
+        if (tid == 0) sOff[C] = total;
     }
     __syncthreads();
     const int T = sOff[C];

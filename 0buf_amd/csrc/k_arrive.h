@@ -36,11 +36,10 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_arrive_fold(Grid g, TileGeom t, P
     constexpr int BY = TY + 2, BZ = TZ + 2, NH = (TX + 2) * BY * BZ;
     __shared__ int hcnt[NH];
     __shared__ int hbase[NH];
-    const long tile = blockIdx.x;
+    const TileAt at = tile_of_block(t, blockIdx.x);
+    const long tile = at.tile;
+    const int tx = at.tx, ty = at.ty, tz = at.tz;
     const int tid = threadIdx.x;
-    const int tz = (int)(tile % t.ntz);
-    const int ty = (int)((tile / t.ntz) % t.nty);
-    const int tx = (int)(tile / ((long)t.ntz * t.nty));
     int n = q.count[tile];
     n = n < q.qcap ? n : q.qcap;
     Leaver64 *const Q = q.e + tile * (long)q.qcap;

@@ -76,9 +76,8 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_rho(Grid g, TileGeom t, P p, Spec
     __shared__ unsigned long long box[NB];
     __shared__ double sM[PIC_MAX_SLOTS];
     const int tid = threadIdx.x, lane = tid % CL;
-    const long tile = blockIdx.x;
-    const int tz = (int)(tile % t.ntz), ty = (int)((tile / t.ntz) % t.nty),
-              tx = (int)(tile / ((long)t.ntz * t.nty));
+    const TileAt at = tile_of_block(t, blockIdx.x);
+    const int tx = at.tx, ty = at.ty, tz = at.tz;
     for (int n = tid; n < NB; n += PIC_BLOCK) box[n] = 0;
     if (tid < PIC_MAX_SLOTS) sM[tid] = sp.m[tid];
     __syncthreads();

@@ -226,17 +226,11 @@ __global__ __launch_bounds__(NT, NT == 1024 ? 4 : NT == 512 ? 6 : 7) void k_push
     const int tid = threadIdx.x;
     const bool snap = DIFF && a.snap_on;
     const bool packed = a.L.packed != 0;
-    long tile;
-    {
-        long nt = a.t.ntiles, b = blockIdx.x;
-        long q = nt / 8, r = nt % 8, x = b % 8;
-        tile = x * q + (x < r ? x : r) + b / 8;
-    }
-    const int tz = (int)(tile % a.t.ntz);
-    const int ty = (int)((tile / a.t.ntz) % a.t.nty);
-    const int tx = (int)(tile / ((long)a.t.ntz * a.t.nty));
-    /* workgroup-uniform (the 64-bit divisions above run on the vector
-     * unit; readfirstlane keeps the tile's base addresses scalar) */
+    const TileAt at = tile_of_block(a.t, blockIdx.x);
+    const long tile = at.tile;
+    const int tx = at.tx, ty = at.ty, tz = at.tz;
+    /* workgroup-uniform (the divisions run on the vector unit; readfirstlane
+     * keeps the tile's base addresses scalar) */
     const int I0 = __builtin_amdgcn_readfirstlane(tx * TX);
     const int L0 = __builtin_amdgcn_readfirstlane(ty * TY);
     const int K0 = __builtin_amdgcn_readfirstlane(tz * TZ);
@@ -787,8 +781,9 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_arrive_fold32(Grid g, TileGeom t,
     const long tile = (long)blockIdx.x * (PIC_BLOCK / 64) + threadIdx.x / 64;
     const bool have = tile < t.ntiles;
     if (have) {
-        const int tz = (int)(tile % t.ntz), ty = (int)((tile / t.ntz) % t.nty),
-                  tx = (int)(tile / ((long)t.ntz * t.nty));
+        const unsigned col = (unsigned)tile / (unsigned)t.ntz;   /* 32 bits: tile_of_block */
+        const int tz = (int)((unsigned)tile - col * (unsigned)t.ntz), ty = (int)(col % (unsigned)t.nty),
+                  tx = (int)(col / (unsigned)t.nty);
         int nsp = 0;
         bool over = false;
         if (c < C) {

@@ -183,20 +183,11 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
     const int tid = threadIdx.x;
     const bool snap = DIFF && a.snap_on;
 
-    /* XCD-aware tile order: workgroups are dealt to the 8 XCDs round-robin,
-     * so each XCD gets a contiguous run of neighbouring tiles and their
-     * shared halo nodes stay in that XCD's L2. */
-    long tile;
-    {
-        long nt = a.t.ntiles, b = blockIdx.x;
-        long q = nt / 8, r = nt % 8, x = b % 8;
-        tile = x * q + (x < r ? x : r) + b / 8;
-    }
-    const int tz = (int)(tile % a.t.ntz);
-    const int ty = (int)((tile / a.t.ntz) % a.t.nty);
-    const int tx = (int)(tile / ((long)a.t.ntz * a.t.nty));
-    /* workgroup-uniform (the 64-bit divisions above run on the vector
-     * unit; readfirstlane keeps the tile's base addresses scalar) */
+    const TileAt at = tile_of_block(a.t, blockIdx.x);
+    const long tile = at.tile;
+    const int tx = at.tx, ty = at.ty, tz = at.tz;
+    /* workgroup-uniform (the divisions run on the vector unit; readfirstlane
+     * keeps the tile's base addresses scalar) */
     const int I0 = __builtin_amdgcn_readfirstlane(tx * TX);
     const int L0 = __builtin_amdgcn_readfirstlane(ty * TY);
     const int K0 = __builtin_amdgcn_readfirstlane(tz * TZ);

@@ -173,6 +173,22 @@ struct TileGeom {
     long ntiles;
 };
 
+/* Tile of workgroup b, one workgroup per tile: workgroups are dealt to the 8
+ * XCDs round-robin, so each XCD gets a contiguous run of neighbouring tiles and
+ * what they share (halo nodes, the buckets that arrivals go to) stays in that
+ * XCD's L2.  In 32 bits (fewer than 2^31 tiles): the 64-bit divisions took
+ * about 420 scalar instructions before a workgroup's first load. */
+struct TileAt {
+    int tile, tx, ty, tz;
+};
+__device__ __forceinline__ TileAt tile_of_block(const TileGeom &t, unsigned b) {
+    const unsigned nt = (unsigned)t.ntiles, q = nt >> 3, r = nt & 7u, x = b & 7u;
+    const unsigned tile = x * q + (x < r ? x : r) + (b >> 3);
+    const unsigned a = tile / (unsigned)t.ntz, c = a / (unsigned)t.nty;
+    return TileAt{(int)tile, (int)c, (int)(a - c * (unsigned)t.nty),
+                  (int)(tile - a * (unsigned)t.ntz)};
+}
+
 /* The push kernels number a tile's particles in flat order f = 0..T-1
  * (cell by cell, sOff[c] = first f of local cell c; the step records use
  * this order).  A particle's bucket slot is addressed by a 32-bit byte offset
