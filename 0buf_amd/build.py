@@ -4,7 +4,7 @@ Usage: python 0buf_amd/build.py   (or __graft_entry__.build())
 
 Every HIP file is compiled with hipcc --offload-arch=gfx950; the host-only
 initializer with g++.  Objects go to 0buf_amd/_build/, the library to
-0buf_amd/libpic_amd.so.  No cmake/ninja: the dependency graph is eleven files.
+0buf_amd/libpic_amd.so.  No cmake/ninja: the dependency graph is a dozen files.
 """
 import os
 import subprocess
@@ -41,6 +41,7 @@ HIP_SOURCES = {
     "pic_api.hip": ["-ffp-contract=off"],
     "pic_adjoint.hip": ["-ffp-contract=off"],
     "pic_noalloc.hip": ["-ffp-contract=off"],
+    "pic_readback.hip": ["-ffp-contract=off"],
 }
 CXX_SOURCES = {"pic_init.cpp": ["-O2", "-fPIC", "-std=c++17", "-ffp-contract=off", "-pthread"],
                "pic_io.cpp": ["-O2", "-fPIC", "-std=c++17"]}

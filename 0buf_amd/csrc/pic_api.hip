@@ -739,6 +739,7 @@ int pic_create(const pic_params *prm, pic_ctx **out) {
     HIPCHK(hipSetDevice(prm->device));
     if (int rc0 = noalloc_init(prm->device)) return rc0;
     pic_ctx *c = new pic_ctx();
+    readback_attach();
     c->prm = *prm;
     c->dev = prm->device;
     Grid &g = c->g;
@@ -809,6 +810,9 @@ int pic_create(const pic_params *prm, pic_ctx **out) {
     if ((e = hipHostMalloc(&c->h_red, 64 * sizeof(double))) != hipSuccess) return fail(record_hip(e, "red"));
     if ((e = hipMalloc(&c->d_slot_sort, PIC_MAX_SLOTS * sizeof(int))) != hipSuccess)
         return fail(record_hip(e, "slots"));
+    /* the clears above ran on the null stream, which the context's does not
+     * wait for */
+    if ((e = hipStreamSynchronize(nullptr)) != hipSuccess) return fail(record_hip(e, "clear"));
     (void)rc;
     *out = c;
     return PIC_SUCCESS;
@@ -831,6 +835,7 @@ int pic_destroy(pic_ctx *c) {
         if (c->h_alt32[k]) (void)hipFree(c->h_alt32[k]);
     }
     free_adjoint(c);
+    readback_detach();
     for (int k = 0; k < 3; k++)
         if (c->d_jfix[k]) (void)hipFree(c->d_jfix[k]);
     free_parts(c->p);
@@ -1038,22 +1043,12 @@ int pic_load_field(pic_ctx *c, int which, const double *host) {
 int pic_get_field(pic_ctx *c, int which, double *host) {
     if (!c || which < 0 || which >= PIC_NFIELDS || !host) return PIC_ERR_INVALID;
     HIPCHK(hipSetDevice(c->dev));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    if (!c->fp32) {
-        HIPCHK(hipMemcpy(host, c->f.f[which], c->g.G * sizeof(double), hipMemcpyDeviceToHost));
-    } else if (which >= PIC_JX && which <= PIC_JZ) {
-        std::vector<long long> t(c->g.G);
-        HIPCHK(hipMemcpy(t.data(), c->f32.J[which - PIC_JX], c->g.G * sizeof(long long),
-                         hipMemcpyDeviceToHost));
-        for (long n = 0; n < c->g.G; n++) host[n] = (double)t[n] * PIC_J_INV;
-    } else {
-        std::vector<float> t(c->g.G);
-        const float *src = which < PIC_HX ? c->f32.E[which]
-                           : which < PIC_JX ? c->f32.H[which - PIC_HX] : c->f32.Q[which - PIC_QX];
-        HIPCHK(hipMemcpy(t.data(), src, c->g.G * sizeof(float), hipMemcpyDeviceToHost));
-        for (long n = 0; n < c->g.G; n++) host[n] = (double)t[n];
-    }
-    return PIC_SUCCESS;
+    if (!c->fp32) return readback(c, host, c->f.f[which], c->g.G, ReadAs::f64);
+    if (which >= PIC_JX && which <= PIC_JZ)
+        return readback(c, host, c->f32.J[which - PIC_JX], c->g.G, ReadAs::fixed_to_f64);
+    const float *src = which < PIC_HX ? c->f32.E[which]
+                       : which < PIC_JX ? c->f32.H[which - PIC_HX] : c->f32.Q[which - PIC_QX];
+    return readback(c, host, src, c->g.G, ReadAs::f32_to_f64);
 }
 
 /* ------------------------------------------------------------------ stages */
@@ -1200,9 +1195,7 @@ int pic_get_cell_counts(pic_ctx *c, int *counts) {
     int rc = check_ready(c);
     if (rc) return rc;
     if (!counts) return PIC_ERR_INVALID;
-    HIPCHK(hipStreamSynchronize(c->stream));
-    HIPCHK(hipMemcpy(counts, count_ptr(c), c->NC * sizeof(int), hipMemcpyDeviceToHost));
-    return PIC_SUCCESS;
+    return readback(c, counts, count_ptr(c), c->NC, ReadAs::i32);
 }
 
 int pic_get_particles(pic_ctx *c, double *x, double *y, double *z, double *px, double *py,
@@ -1237,10 +1230,10 @@ int pic_get_particles(pic_ctx *c, double *x, double *y, double *z, double *px, d
     HIPCHK(hipStreamSynchronize(c->stream));
     double *outs[6] = {x, y, z, px, py, pz};
     for (int k = 0; k < 6; k++)
-        if (outs[k] && P) HIPCHK(hipMemcpy(outs[k], d[k], P * sizeof(double), hipMemcpyDeviceToHost));
+        if (outs[k] && (rc = readback(c, outs[k], d[k], P, ReadAs::f64))) return rc;
     std::vector<unsigned char> sp(Pn);
     if (P) HIPCHK(hipMemcpy(sp.data(), d_sp, P, hipMemcpyDeviceToHost));
-    if (cell && P) HIPCHK(hipMemcpy(cell, d_cell, P * sizeof(int), hipMemcpyDeviceToHost));
+    if (cell && (rc = readback(c, cell, d_cell, P, ReadAs::i32))) return rc;
     for (long j = 0; j < P; j++) {
         int s = sp[j];
         if (sort) sort[j] = c->slot_sort[s];
@@ -1284,9 +1277,7 @@ int pic_cell_moments(pic_ctx *c, int sort, int op, double *out) {
     else
         launch_cell_moments64(c->NC, c->p, c->sp, c->d_slot_sort, sort, op, c->d_cmom, c->stream);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(c->stream));
-    HIPCHK(hipMemcpy(out, c->d_cmom, n * sizeof(double), hipMemcpyDeviceToHost));
-    return PIC_SUCCESS;
+    return readback(c, out, c->d_cmom, n, ReadAs::f64);
 }
 
 /* ------------------------------------------------------- decision tape */
@@ -1397,8 +1388,8 @@ int pic_gauss_residual(pic_ctx *c, double *res, double *max_drift, int set_refer
     HIPCHK(hipMemcpyAsync(c->h_red, c->d_red, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     if (first) c->gres_ref_set = true;
-    if (res) HIPCHK(hipMemcpy(res, c->d_gres, c->NC * sizeof(double), hipMemcpyDeviceToHost));
     if (max_drift) *max_drift = c->h_red[0];
+    if (res) return readback(c, res, c->d_gres, c->NC, ReadAs::f64);
     return PIC_SUCCESS;
 }
 

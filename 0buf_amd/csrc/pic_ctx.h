@@ -119,6 +119,13 @@ int alloc_parts(P &p, long ncell, int cap, bool with_count, bool with_id);
 template <class P>
 void free_parts(P &p);
 void free_adjoint(pic_ctx *c);   /* pic_adjoint.hip */
+/* pic_readback.hip: n elements at src on the device into host memory, after
+ * what the context's stream holds; returns with the elements there */
+enum class ReadAs { f64, i32, f32_to_f64, fixed_to_f64 /* int64 current */ };
+int readback(pic_ctx *c, void *dst, const void *src, long n, ReadAs as);
+/* each context's life: what readbacks keep between calls goes with the last */
+void readback_attach();
+void readback_detach();
 /* pic_noalloc.hip: device address of this device's scratch array, taken once
  * per device with the device current */
 int noalloc_init(int dev);
