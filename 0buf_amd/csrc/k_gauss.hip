@@ -299,7 +299,8 @@ __global__ __launch_bounds__(FINAL_T) void k_moments_final(const double *partial
 inline unsigned blocks_for(long n, int per) { return (unsigned)((n + per - 1) / per); }
 
 template <class P>
-void rho(const Grid &g, const TileGeom &t, P p, SpeciesTable sp, long long *r, hipStream_t s) {
+void rho(const Grid &g, P p, SpeciesTable sp, long long *r, hipStream_t s) {
+    const TileGeom t = make_tile_geom(g.Nx, g.Ny, g.Nz, false);
     hipLaunchKernelGGL((k_rho<2, 4, 8, P>), dim3((unsigned)t.ntiles), dim3(PIC_BLOCK), 0, s, g, t,
                        p, sp, r);
 }
@@ -344,13 +345,11 @@ void moments(const Grid &g, long ncell, P p, SpeciesTable sp, const int *slot_so
 
 }  // namespace
 
-void launch_rho64(const Grid &g, const TileGeom &t, PartPtrs p, SpeciesTable sp, long long *r,
-                  hipStream_t s) {
-    rho(g, t, p, sp, r, s);
+void launch_rho64(const Grid &g, PartPtrs p, SpeciesTable sp, long long *r, hipStream_t s) {
+    rho(g, p, sp, r, s);
 }
-void launch_rho32(const Grid &g, const TileGeom &t, PartPtrs32 p, SpeciesTable sp, long long *r,
-                  hipStream_t s) {
-    rho(g, t, p, sp, r, s);
+void launch_rho32(const Grid &g, PartPtrs32 p, SpeciesTable sp, long long *r, hipStream_t s) {
+    rho(g, p, sp, r, s);
 }
 void launch_gauss64(const Grid &g, FieldPtrs f, const long long *r, double *res,
                     const double *ref, unsigned long long *drift, hipStream_t s) {

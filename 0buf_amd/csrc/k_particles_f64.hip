@@ -45,6 +45,7 @@ namespace {
 #endif
 
 constexpr int TXC = 2, TYC = 4, TZC = 8;
+constexpr int TXS = 2, TYS = 2, TZS = 4;   /* tiles of small boxes (make_tile_geom) */
 constexpr int GS64 = 16;    /* slots of an FP64 array in one 128-byte line */
 constexpr int JCOPIES = PIC_JCOPIES64;
 
@@ -771,8 +772,17 @@ void launch_push_deposit_f64(const Grid &g, const TileGeom &t, FieldPtrs f, Part
     a.d = diff ? *diff : DiffArgs{};
     a.snap_on = diff && diff->snap.p[0] != nullptr;
     /* dynamic LDS: one 4-byte entry per line group */
-    const size_t lds = (size_t)4 * TXC * TYC * TZC * ((p.cap + GS64 - 1) / GS64);
+    const size_t lds = (size_t)4 * t.TX * t.TY * t.TZ * ((p.cap + GS64 - 1) / GS64);
     const int nt = push_threads(t.ntiles);
+    if (!diff && t.TZ == TZS) {
+        if (t.ntiles <= 512)   /* two a CU: 51.1 against 52.0 us a step at 128 */
+            hipLaunchKernelGGL((k_push_deposit<TXS, TYS, TZS, false, false, 512>),
+                               dim3((unsigned)t.ntiles), dim3(512), lds, s, a);
+        else                   /* 73.3 against 83.8 us at 1020 */
+            hipLaunchKernelGGL((k_push_deposit<TXS, TYS, TZS, false, false, PIC_BLOCK>),
+                               dim3((unsigned)t.ntiles), dim3(PIC_BLOCK), lds, s, a);
+        return;
+    }
     const bool tape = diff && diff->tape_mode != PIC_TAPE_OFF;
     auto launch = [&](auto diff_on, auto tape_on, auto threads) {
         constexpr int NT = decltype(threads)::value;
@@ -799,8 +809,12 @@ void launch_arrive_fold_f64(const Grid &g, const TileGeom &t, PartPtrs p, QueueP
     const unsigned tiles = what & PIC_ARRIVE ? (unsigned)t.ntiles : 0;
     const unsigned blocks = tiles + (what & PIC_FOLD ? fold_blocks(g) : 0);
     const FoldJ<double> J{{f.f[PIC_JX], f.f[PIC_JY], f.f[PIC_JZ]}};
-    hipLaunchKernelGGL((k_arrive_fold<TXC, TYC, TZC, double>), dim3(blocks),
-                       dim3(PIC_BLOCK), 0, s, g, t, p, q, st, J, tiles);
+    if (t.TZ == TZS)
+        hipLaunchKernelGGL((k_arrive_fold<TXS, TYS, TZS, double>), dim3(blocks), dim3(PIC_BLOCK),
+                           0, s, g, t, p, q, st, J, tiles);
+    else
+        hipLaunchKernelGGL((k_arrive_fold<TXC, TYC, TZC, double>), dim3(blocks), dim3(PIC_BLOCK),
+                           0, s, g, t, p, q, st, J, tiles);
 }
 
 void launch_scatter_load(const long *offsets, long ncell, const double *src[6],
@@ -837,14 +851,33 @@ void launch_copy_parts(long ncell, PartPtrs from, PartPtrs to, hipStream_t s) {
                        ncell, from, to);
 }
 
-TileGeom make_tile_geom(int Nx, int Ny, int Nz) {
-    TileGeom t;
-    t.TX = TXC;
-    t.TY = TYC;
-    t.TZ = TZC;
-    t.ntx = (Nx + TXC - 1) / TXC;
-    t.nty = (Ny + TYC - 1) / TYC;
-    t.ntz = (Nz + TZC - 1) / TZC;
-    t.ntiles = (long)t.ntx * t.nty * t.ntz;
-    return t;
+/* With few tiles the push lasts as long as the fullest CU takes: tiles of 16
+ * cells spread a small box over more CUs and leave a shorter last round, for a
+ * sixth more work per cell (halo nodes staged and flushed, workgroup starts).
+ * So they are taken where 16 cells x rounds x 1.2 is below the large tiles' 64
+ * cells x rounds, up to two large tiles a CU.  Whole steps, FP64, 32 to 51
+ * particles per cell, us with large / small tiles:
+ *   large tiles  32  66.6 / 51.1      256  64.4 / 64.5      483  96.8 /  99.0
+ *                64  68.4 / 53.2      306  92.4 / 73.3      512  99.7 / 107.5
+ *               128  61.4 / 54.2 */
+TileGeom make_tile_geom(int Nx, int Ny, int Nz, bool small_ok) {
+    auto tiles = [&](int X, int Y, int Z) {
+        TileGeom t;
+        t.TX = X;
+        t.TY = Y;
+        t.TZ = Z;
+        t.ntx = (Nx + X - 1) / X;
+        t.nty = (Ny + Y - 1) / Y;
+        t.ntz = (Nz + Z - 1) / Z;
+        t.ntiles = (long)t.ntx * t.nty * t.ntz;
+        return t;
+    };
+    constexpr long CUS = 256;
+    auto cells_per_cu = [&](const TileGeom &t) {
+        return (t.ntiles + CUS - 1) / CUS * t.TX * t.TY * t.TZ;
+    };
+    const TileGeom large = tiles(TXC, TYC, TZC), small = tiles(TXS, TYS, TZS);
+    return small_ok && large.ntiles <= 2 * CUS && 6 * cells_per_cu(small) < 5 * cells_per_cu(large)
+               ? small
+               : large;
 }

@@ -194,7 +194,10 @@ int alloc_queue(QueuePtrs32 &q, const TileGeom &t, int qcap) {
 }
 
 int queue_capacity(const TileGeom &t, int cap) {
-    long c = (long)t.TX * t.TY * t.TZ * cap / 2;
+    /* half the tile's slots; of a small tile all, since a few full cells may
+     * empty at once */
+    const long cells = (long)t.TX * t.TY * t.TZ;
+    long c = cells < 64 ? cells * cap : cells * cap / 2;
     c = (c + 63) / 64 * 64;
     return (int)std::max(64L, c);
 }
@@ -755,7 +758,8 @@ int pic_create(const pic_params *prm, pic_ctx **out) {
     g.tau = prm->tau;
     g.ghost_mode = prm->ghost_mode;
     c->NC = (long)g.Nx * g.Ny * g.Nz;
-    c->t = make_tile_geom(g.Nx, g.Ny, g.Nz);
+    c->t = make_tile_geom(g.Nx, g.Ny, g.Nz,
+                          prm->precision == PIC_FP64 && !prm->differentiable);
     int rc = PIC_SUCCESS;
     auto fail = [&](int r) {
         pic_destroy(c);
@@ -1375,10 +1379,10 @@ int pic_gauss_residual(pic_ctx *c, double *res, double *max_drift, int set_refer
     const double *ref = first ? nullptr : c->d_gres_ref;
     unsigned long long *drift = (unsigned long long *)c->d_red;
     if (c->fp32) {
-        launch_rho32(g, c->t, c->p32, c->sp, c->d_rho, c->stream);
+        launch_rho32(g, c->p32, c->sp, c->d_rho, c->stream);
         launch_gauss32(g, c->f32, c->d_rho, c->d_gres, ref, drift, c->stream);
     } else {
-        launch_rho64(g, c->t, c->p, c->sp, c->d_rho, c->stream);
+        launch_rho64(g, c->p, c->sp, c->d_rho, c->stream);
         launch_gauss64(g, c->f, c->d_rho, c->d_gres, ref, drift, c->stream);
     }
     HIPCHK(hipGetLastError());

@@ -428,7 +428,8 @@ void launch_e32(const Grid &g, FieldPtrs32 f, hipStream_t s);
 void launch_e_periodic32(const Grid &g, FieldPtrs32 f, hipStream_t s);
 void launch_fold_j32(const Grid &g, FieldPtrs32 f, hipStream_t s);
 void launch_energy32(const Grid &g, FieldPtrs32 f, const EnergyOut &o, hipStream_t s);
-TileGeom make_tile_geom(int Nx, int Ny, int Nz);
+/* tiles of 2x4x8 cells, or with small_ok (FP64 plain form) 2x2x4 in small boxes */
+TileGeom make_tile_geom(int Nx, int Ny, int Nz, bool small_ok);
 
 /* Differentiable form of the FP64 step: the push deposits J as int64 fixed
  * point with resolution 2^-48 (order-free, so a recomputed step is bitwise
@@ -545,10 +546,8 @@ void launch_generate_species(const Grid &g, const pic_species_spec &spec, const 
  * cell-centre lattice into an int64 fixed-point array of G entries, then
  * per bulk centre res = div E - rho; with ref, *drift (0 before) receives
  * the bits of max |res - ref| */
-void launch_rho64(const Grid &g, const TileGeom &t, PartPtrs p, SpeciesTable sp, long long *rho,
-                  hipStream_t s);
-void launch_rho32(const Grid &g, const TileGeom &t, PartPtrs32 p, SpeciesTable sp, long long *rho,
-                  hipStream_t s);
+void launch_rho64(const Grid &g, PartPtrs p, SpeciesTable sp, long long *rho, hipStream_t s);
+void launch_rho32(const Grid &g, PartPtrs32 p, SpeciesTable sp, long long *rho, hipStream_t s);
 void launch_gauss64(const Grid &g, FieldPtrs f, const long long *rho, double *res,
                     const double *ref, unsigned long long *drift, hipStream_t s);
 void launch_gauss32(const Grid &g, FieldPtrs32 f, const long long *rho, double *res,
