@@ -870,6 +870,7 @@ TileGeom make_tile_geom(int Nx, int Ny, int Nz, bool small_ok) {
         t.nty = (Ny + Y - 1) / Y;
         t.ntz = (Nz + Z - 1) / Z;
         t.ntiles = (long)t.ntx * t.nty * t.ntz;
+        t.order = nullptr;
         return t;
     };
     constexpr long CUS = 256;

@@ -88,6 +88,80 @@ __global__ __launch_bounds__(SCAN_T) void k_record_offsets(Grid g, TileGeom t, c
     if (tid == 0) *done = 0;
 }
 
+/* particles of each tile, from the cells' offsets: along z a tile's cells are
+ * consecutive */
+__global__ __launch_bounds__(PIC_BLOCK) void k_tile_counts(Grid g, TileGeom t, const long *off,
+                                                          int *cnt) {
+    const unsigned tile = blockIdx.x * PIC_BLOCK + threadIdx.x;
+    if (tile >= (unsigned)t.ntiles) return;
+    const unsigned a = tile / (unsigned)t.ntz, x = a / (unsigned)t.nty;
+    const int I0 = (int)x * TXC, L0 = (int)(a - x * (unsigned)t.nty) * TYC,
+              K0 = (int)(tile - a * (unsigned)t.ntz) * TZC;
+    const int K1 = K0 + TZC < g.Nz ? K0 + TZC : g.Nz;
+    long n = 0;
+    for (int i = I0; i < I0 + TXC && i < g.Nx; i++)
+        for (int l = L0; l < L0 + TYC && l < g.Ny; l++) {
+            const long row = ((long)i * g.Ny + l) * g.Nz;
+            n += off[row + K1] - off[row + K0];
+        }
+    cnt[tile] = (int)n;
+}
+
+/* The order in which workgroups take the tiles: by load in classes of a
+ * quarter of the mean (a uniform plasma is one class), the fullest first, each
+ * class in tile order, dealt to the XCDs in contiguous runs.  A profiled beam's
+ * tiles on the axis hold several times the mean; started last, in their place
+ * among the others, they left the chip waiting for a few workgroups: the push
+ * issued on 51% of its cycles, on 80% in a uniform plasma.  One launch, us, in
+ * tile order / fullest first (two launches of 5 us per checkpoint): 128x64x64
+ * cells FP64 with a beam of 8 cells' width, push 1199 / 943, particle adjoint
+ * 1870 / 1634, arrival 165 / 117; 256x64x64 FP32, push 1436 / 1177, adjoint
+ * 2909 / 2518. */
+constexpr int ORDER_T = 512, CLASSES = 16;
+
+__global__ __launch_bounds__(ORDER_T) void k_tile_order(int n, const int *cnt, const long *total,
+                                                       int *order) {
+    __shared__ int at[CLASSES * ORDER_T];   /* per class and thread: its next position */
+    __shared__ int part[ORDER_T / 64];
+    __shared__ int start[CLASSES + 1];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const float per = *total > 0 ? 4.0f * (float)n / (float)*total : 0.0f;
+    auto cls = [&](int c) {
+        const float q = (float)c * per + 0.5f;
+        return CLASSES - 1 - (q < (float)(CLASSES - 1) ? (int)q : CLASSES - 1);
+    };
+    const int chunk = (n + ORDER_T - 1) / ORDER_T;
+    const int b = min(tid * chunk, n), e = min(b + chunk, n);
+    for (int c = 0; c < CLASSES; c++) at[c * ORDER_T + tid] = 0;
+    for (int i = b; i < e; i++) at[cls(cnt[i]) * ORDER_T + tid]++;
+    __syncthreads();
+    /* exclusive scan over all entries, CLASSES consecutive ones a thread */
+    int sum = 0;
+    for (int k = 0; k < CLASSES; k++) sum += at[tid * CLASSES + k];
+    int wave;
+    int run = wave_excl_scan(sum, wave);
+    if (lane == 0) part[w] = wave;
+    __syncthreads();
+    for (int k = 0; k < w; k++) run += part[k];
+    for (int k = 0; k < CLASSES; k++) {
+        const int v = at[tid * CLASSES + k];
+        at[tid * CLASSES + k] = run;
+        run += v;
+    }
+    __syncthreads();
+    if (tid < CLASSES) start[tid] = at[tid * ORDER_T];
+    if (tid == CLASSES) start[CLASSES] = n;
+    __syncthreads();
+    for (int i = b; i < e; i++) {
+        const int c = cls(cnt[i]), s = start[c], m = start[c + 1] - s;
+        const int j = at[c * ORDER_T + tid]++ - s;   /* of the class's m tiles */
+        const int q = m >> 3, r = m & 7, cut = r * (q + 1);
+        const int x = j < cut ? j / (q + 1) : r + (j - cut) / q;
+        const int first = j < cut ? x * (q + 1) : cut + (x - r) * q;
+        order[s + (j - first) * 8 + x] = i;
+    }
+}
+
 /* six arrays of n 4-byte words in one launch (the fields of a step
  * record), blockIdx.y = array */
 struct Six {
@@ -115,6 +189,15 @@ void launch_copy6(void *const dst[6], const void *const src[6], size_t bytes, hi
     if (blocks > 2048) blocks = 2048;
     if (blocks < 1) blocks = 1;
     hipLaunchKernelGGL(k_copy6, dim3((unsigned)blocks, 6), dim3(PIC_BLOCK), 0, s, a, n);
+}
+
+void launch_tile_order(const Grid &g, const TileGeom &t, const long *off, int *cnt, int *order,
+                       hipStream_t s) {
+    const long cells = (long)g.Nx * g.Ny * g.Nz;
+    hipLaunchKernelGGL(k_tile_counts, dim3((unsigned)((t.ntiles + PIC_BLOCK - 1) / PIC_BLOCK)),
+                       dim3(PIC_BLOCK), 0, s, g, t, off, cnt);
+    hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(ORDER_T), 0, s, (int)t.ntiles, cnt, off + cells,
+                       order);
 }
 
 void launch_record_offsets(const Grid &g, const TileGeom &t, const int *count, int cap,

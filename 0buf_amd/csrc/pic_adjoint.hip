@@ -65,6 +65,7 @@ struct AdjointStore {
     std::vector<long *> recoff;       /* ntiles + 1 offsets per record */
     long room = 0;                    /* particles a record holds */
     long *tile_sum = nullptr;         /* scratch of the offset scan */
+    int *tile_order = nullptr;        /* the context's tile order, and the tiles' counts */
     std::vector<FieldSet> recf;       /* E^n, H^{n+1/2} of each recorded step */
     void *Eend[3] = {nullptr, nullptr, nullptr};   /* E at the end of the segment */
     AdjLam lam{};
@@ -158,6 +159,12 @@ int save_state(pic_ctx *c, Compact &dst, FieldSet &f) {
     int rc = reserve_state(c, dst, f, P);
     if (rc) return rc;
     HIPCHK(hipMemcpy(dst.off, off.data(), (NC + 1) * sizeof(long), hipMemcpyHostToDevice));
+    /* the order of the tiles for the steps to come, in both directions: any
+     * permutation gives the same results */
+    AdjointStore *s = c->adj;
+    if (!s->tile_order) HIPCHK(hipMalloc(&s->tile_order, 2 * c->t.ntiles * sizeof(int)));
+    launch_tile_order(c->g, c->t, dst.off, s->tile_order + c->t.ntiles, s->tile_order, c->stream);
+    c->t.order = s->tile_order;
     HIPCHK(hipMemcpyAsync(dst.count, live_count(c), NC * sizeof(int), hipMemcpyDeviceToDevice,
                           c->stream));
     if (c->fp32) {
@@ -297,6 +304,8 @@ void free_adjoint(pic_ctx *c) {
     for (auto *o : s->recoff)
         if (o) (void)hipFree(o);
     if (s->tile_sum) (void)hipFree(s->tile_sum);
+    c->t.order = nullptr;
+    if (s->tile_order) (void)hipFree(s->tile_order);
     for (auto &f : s->recf) free_fields(f);
     free_lam(s);
     for (int k = 0; k < 3; k++)

@@ -171,6 +171,7 @@ struct TileGeom {
     int TX, TY, TZ;
     int ntx, nty, ntz;
     long ntiles;
+    const int *order;    /* on the device: the tile of each workgroup, or null (tile_of_block) */
 };
 
 /* Tile of workgroup b, one workgroup per tile: workgroups are dealt to the 8
@@ -183,7 +184,7 @@ struct TileAt {
 };
 __device__ __forceinline__ TileAt tile_of_block(const TileGeom &t, unsigned b) {
     const unsigned nt = (unsigned)t.ntiles, q = nt >> 3, r = nt & 7u, x = b & 7u;
-    const unsigned tile = x * q + (x < r ? x : r) + (b >> 3);
+    const unsigned tile = t.order ? (unsigned)t.order[b] : x * q + (x < r ? x : r) + (b >> 3);
     const unsigned a = tile / (unsigned)t.ntz, c = a / (unsigned)t.nty;
     return TileAt{(int)tile, (int)c, (int)(a - c * (unsigned)t.nty),
                   (int)(tile - a * (unsigned)t.ntz)};
@@ -458,6 +459,11 @@ void launch_jfix_to_f64(const Grid &g, FieldPtrs f, DiffArgs d, hipStream_t s);
  * before t (counts capped at cap), off[ntiles] the total (tile_sum: one entry
  * per tile, done: 0 between launches); a total beyond
  * `room` raises PIC_F_RECORD (the push writes no record entry past room) */
+/* the fullest tiles first (k_records.hip): order[b] = the tile workgroup b
+ * takes, from the cells' particle offsets (off[cells] the total); cnt: one
+ * scratch entry per tile */
+void launch_tile_order(const Grid &g, const TileGeom &t, const long *off, int *cnt, int *order,
+                       hipStream_t s);
 /* six device arrays of `bytes` (a multiple of 4) each, in one launch */
 void launch_copy6(void *const dst[6], const void *const src[6], size_t bytes, hipStream_t s);
 void launch_record_offsets(const Grid &g, const TileGeom &t, const int *count, int cap,
