@@ -24,11 +24,19 @@
 #include "pic_internal.h"
 
 /* workgroups [0, tiles): the arrivals of one tile each (tiles: all, or 0);
- * those behind them: the periodic fold of the current */
+ * [tiles, fold_end): the periodic fold of the current; those behind them: where
+ * the current still is fixed point, its conversion at the nodes without a fold
+ * (as a launch of its own before the fold the conversion took 5 us of a small
+ * step) */
 template <int TX, int TY, int TZ, class JT>
 __global__ __launch_bounds__(PIC_BLOCK) void k_arrive_fold(Grid g, TileGeom t, PartPtrs p,
                                                            QueuePtrs q, DevStatus *st,
-                                                           FoldJ<JT> f, unsigned tiles) {
+                                                           FoldJ<JT> f, unsigned tiles,
+                                                           unsigned fold_end) {
+    if (blockIdx.x >= fold_end) {
+        convert_inner(g, f, (blockIdx.x - fold_end) * PIC_BLOCK + threadIdx.x);
+        return;
+    }
     if (blockIdx.x >= tiles) {
         fold_class(g, f, (blockIdx.x - tiles) * PIC_BLOCK + threadIdx.x);
         return;

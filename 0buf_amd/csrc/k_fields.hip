@@ -94,43 +94,84 @@ struct HOut {
     T *H[3];
 };
 
+/* The sum over PIC_BLOCK consecutive threads, one sum for each PIC_BLOCK threads of the workgroup: the
+ * pairs t, t + 128, then t, t + 64, ... in turn.  Thread 0 of each holds it. */
+__device__ __forceinline__ double sub_tree(double (*red)[PIC_BLOCK], double s) {
+    const int sub = threadIdx.x / PIC_BLOCK, t = threadIdx.x % PIC_BLOCK;
+    red[sub][t] = s;
+    __syncthreads();
+    if (t < 64) {
+        const double *r = red[sub] + t;
+        s = (r[0] + r[128]) + (r[64] + r[192]);
+        for (int d = 32; d > 0; d >>= 1) s += __shfl_down(s, d);
+    }
+    __syncthreads();
+    return s;
+}
+
 /* MagneticStageOne (gpu_plasma.h:524-538) -> GPU_emh1 / emh1_Element
  * (kernels.cu:1052-1089) for the three components, ranges from
  * MagneticFieldTrace (gpu_plasma.h:735-767), shifts from
  * getMagneticFieldTraceShifts (722-733); fused with the J := 0 of
- * SetCurrentsToZero (gpu_plasma.h:2058-2069). */
-template <typename T, typename JT>
+ * SetCurrentsToZero (gpu_plasma.h:2058-2069).  REC: also copies E and the new H
+ * for a step record; ENERGY: also the energy of the E it reads, a partial per
+ * workgroup.  Both ride on what is read anyway: as launches of their own they
+ * took 4 us each of a small step. */
+template <typename T>
+struct HalfRec {
+    T *E[3], *H[3];
+};
+template <typename T, typename JT, bool REC, bool ENERGY>
 __global__ __launch_bounds__(PIC_BLOCK) void k_h_half(Grid g, FV<T, JT> f, YeeC<T> c,
-                                                     DevStatus *reset) {
-    const unsigned n = xcd_block() * PIC_BLOCK + threadIdx.x;
+                                                     DevStatus *reset, HalfRec<T> rec,
+                                                     double *partials) {
+    const unsigned block = xcd_block(), n = block * PIC_BLOCK + threadIdx.x;
     if (reset && n == 0) *reset = DevStatus{0, 0, 0, 0, 0};
-    if (n >= (unsigned)g.G) return;
-    int i, l, k;
-    decode32(g, n, i, l, k);
-    const T c1x = c.c1x, c1y = c.c1y, c1z = c.c1z;
-    const unsigned sy = (unsigned)g.sy, sx = (unsigned)g.sx;
-    const T *Ex = f.E[0], *Ey = f.E[1], *Ez = f.E[2];
-    if (l <= g.Ny && k <= g.Nz) {   /* Qx over [0,Nx+1]x[0,Ny]x[0,Nz] */
-        T e1_n1 = Ey[n + 1], e1_n = Ey[n], e2_n2 = Ez[n + sy], e2_n = Ez[n];
-        T t = (T)0.5 * (c1z * (e1_n1 - e1_n) - c1y * (e2_n2 - e2_n));
-        f.Q[0][n] = t;
-        f.H[0][n] += t;
+    double energy = 0.0;
+    if (n < (unsigned)g.G) {
+        int i, l, k;
+        decode32(g, n, i, l, k);
+        const T c1x = c.c1x, c1y = c.c1y, c1z = c.c1z;
+        const unsigned sy = (unsigned)g.sy, sx = (unsigned)g.sx;
+        const T *Ex = f.E[0], *Ey = f.E[1], *Ez = f.E[2];
+        if (l <= g.Ny && k <= g.Nz) {   /* Qx over [0,Nx+1]x[0,Ny]x[0,Nz] */
+            T e1_n1 = Ey[n + 1], e1_n = Ey[n], e2_n2 = Ez[n + sy], e2_n = Ez[n];
+            T t = (T)0.5 * (c1z * (e1_n1 - e1_n) - c1y * (e2_n2 - e2_n));
+            f.Q[0][n] = t;
+            f.H[0][n] += t;
+        }
+        if (i <= g.Nx && k <= g.Nz) {   /* Qy over [0,Nx]x[0,Ny+1]x[0,Nz] */
+            T e1_n1 = Ez[n + sx], e1_n = Ez[n], e2_n2 = Ex[n + 1], e2_n = Ex[n];
+            T t = (T)0.5 * (c1x * (e1_n1 - e1_n) - c1z * (e2_n2 - e2_n));
+            f.Q[1][n] = t;
+            f.H[1][n] += t;
+        }
+        if (i <= g.Nx && l <= g.Ny) {   /* Qz over [0,Nx]x[0,Ny]x[0,Nz+1] */
+            T e1_n1 = Ex[n + sy], e1_n = Ex[n], e2_n2 = Ey[n + sx], e2_n = Ey[n];
+            T t = (T)0.5 * (c1y * (e1_n1 - e1_n) - c1x * (e2_n2 - e2_n));
+            f.Q[2][n] = t;
+            f.H[2][n] += t;
+        }
+        f.J[0][n] = (JT)0;
+        f.J[1][n] = (JT)0;
+        f.J[2][n] = (JT)0;
+        if constexpr (REC) {
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                rec.E[d][n] = f.E[d][n];
+                rec.H[d][n] = f.H[d][n];
+            }
+        }
+        if constexpr (ENERGY) {
+            const double a = (double)Ex[n], b = (double)Ey[n], e = (double)Ez[n];
+            energy = a * a + b * b + e * e;
+        }
     }
-    if (i <= g.Nx && k <= g.Nz) {   /* Qy over [0,Nx]x[0,Ny+1]x[0,Nz] */
-        T e1_n1 = Ez[n + sx], e1_n = Ez[n], e2_n2 = Ex[n + 1], e2_n = Ex[n];
-        T t = (T)0.5 * (c1x * (e1_n1 - e1_n) - c1z * (e2_n2 - e2_n));
-        f.Q[1][n] = t;
-        f.H[1][n] += t;
+    if constexpr (ENERGY) {
+        __shared__ double red[1][PIC_BLOCK];
+        energy = sub_tree(red, energy);
+        if (threadIdx.x == 0) partials[block] = energy;
     }
-    if (i <= g.Nx && l <= g.Ny) {   /* Qz over [0,Nx]x[0,Ny]x[0,Nz+1] */
-        T e1_n1 = Ex[n + sy], e1_n = Ex[n], e2_n2 = Ey[n + sx], e2_n = Ey[n];
-        T t = (T)0.5 * (c1y * (e1_n1 - e1_n) - c1x * (e2_n2 - e2_n));
-        f.Q[2][n] = t;
-        f.H[2][n] += t;
-    }
-    f.J[0][n] = (JT)0;
-    f.J[1][n] = (JT)0;
-    f.J[2][n] = (JT)0;
 }
 
 /* MagneticFieldStageTwo (gpu_plasma.h:540-551) -> GPU_emh2 (kernels.cu:1024-1049) */
@@ -219,8 +260,10 @@ __device__ __forceinline__ T hn1(const Grid &g, const FV<T, JT> &f, int d, unsig
  *     from it (0 from N, N+1 from 1).  Ghosts lie outside the E update
  *     ranges and are never a source, so no node is both written and read. */
 template <typename T, typename JT>
-__global__ __launch_bounds__(PIC_BLOCK) void k_h2_e(Grid g, FV<T, JT> f, HOut<T> out, YeeC<T> c) {
+__global__ __launch_bounds__(PIC_BLOCK) void k_h2_e(Grid g, FV<T, JT> f, HOut<T> out, YeeC<T> c,
+                                                   const DevStatus *st, DevStatus *h_st) {
     const unsigned n = xcd_block() * PIC_BLOCK + threadIdx.x;
+    if (st && n == 0) *h_st = *st;   /* (the launches before this one raised what there is) */
     if (n >= (unsigned)g.G) return;
     int i, l, k;
     decode32(g, n, i, l, k);
@@ -380,21 +423,6 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_fold_j(Grid g, FV<T, JT> f, int d
  * the same without the last step. */
 constexpr int ENERGY_T = 1024, ENERGY_PARTS = 1024, SUB = ENERGY_T / PIC_BLOCK;
 
-/* The sum over PIC_BLOCK consecutive threads, SUB sums in a workgroup: the
- * pairs t, t + 128, then t, t + 64, ... in turn.  Thread 0 of each holds it. */
-__device__ __forceinline__ double sub_tree(double (*red)[PIC_BLOCK], double s) {
-    const int sub = threadIdx.x / PIC_BLOCK, t = threadIdx.x % PIC_BLOCK;
-    red[sub][t] = s;
-    __syncthreads();
-    if (t < 64) {
-        const double *r = red[sub] + t;
-        s = (r[0] + r[128]) + (r[64] + r[192]);
-        for (int d = 32; d > 0; d >>= 1) s += __shfl_down(s, d);
-    }
-    __syncthreads();
-    return s;
-}
-
 template <typename T, typename JT>
 __global__ __launch_bounds__(ENERGY_T) void k_energy(Grid g, FV<T, JT> f, EnergyOut o) {
     __shared__ double red[SUB][PIC_BLOCK];
@@ -432,6 +460,17 @@ __global__ __launch_bounds__(ENERGY_T) void k_energy(Grid g, FV<T, JT> f, Energy
     }
 }
 
+/* row blockIdx.x: its partials added up as k_energy's last workgroup does */
+__global__ __launch_bounds__(PIC_BLOCK) void k_energy_sums(const double *partials, int blocks,
+                                                          double *h_out) {
+    __shared__ double red[1][PIC_BLOCK];
+    const double *p = partials + (long)blockIdx.x * PIC_ENERGY_ROW;
+    double s = 0.0;
+    for (int j = threadIdx.x; j < blocks; j += PIC_BLOCK) s += p[j];
+    s = sub_tree(red, s);
+    if (threadIdx.x == 0) h_out[blockIdx.x] = s;
+}
+
 __global__ void k_reset_status(DevStatus *st) {
     st->flags = 0;
     st->max_dep = 0;
@@ -443,14 +482,29 @@ __global__ void k_reset_status(DevStatus *st) {
 inline unsigned blocks_for(long n) { return (unsigned)((n + PIC_BLOCK - 1) / PIC_BLOCK); }
 
 template <typename T, typename JT>
-void h_half(const Grid &g, FV<T, JT> f, DevStatus *reset, hipStream_t s) {
-    hipLaunchKernelGGL((k_h_half<T, JT>), dim3(blocks_for(g.G)), dim3(PIC_BLOCK), 0, s, g, f,
-                       yee_coef<T>(g), reset);
+void h_half(const Grid &g, FV<T, JT> f, const HalfOut &o, hipStream_t s) {
+    HalfRec<T> rec{};
+    for (int k = 0; o.rec && k < 3; k++) {
+        rec.E[k] = (T *)o.rec[k];
+        rec.H[k] = (T *)o.rec[3 + k];
+    }
+    const dim3 grid(blocks_for(g.G)), block(PIC_BLOCK);
+    const YeeC<T> c = yee_coef<T>(g);
+    if (o.rec)
+        hipLaunchKernelGGL((k_h_half<T, JT, true, false>), grid, block, 0, s, g, f, c, o.reset, rec,
+                           nullptr);
+    else if (o.partials)
+        hipLaunchKernelGGL((k_h_half<T, JT, false, true>), grid, block, 0, s, g, f, c, o.reset,
+                           rec, o.partials);
+    else
+        hipLaunchKernelGGL((k_h_half<T, JT, false, false>), grid, block, 0, s, g, f, c, o.reset,
+                           rec, nullptr);
 }
 template <typename T, typename JT>
-void h2_e(const Grid &g, FV<T, JT> f, HOut<T> out, hipStream_t s) {
+void h2_e(const Grid &g, FV<T, JT> f, HOut<T> out, const DevStatus *st, DevStatus *h_st,
+          hipStream_t s) {
     hipLaunchKernelGGL((k_h2_e<T, JT>), dim3(blocks_for(g.G)), dim3(PIC_BLOCK), 0, s, g, f, out,
-                       yee_coef<T>(g));
+                       yee_coef<T>(g), st, h_st);
 }
 template <typename T, typename JT>
 void h2(const Grid &g, FV<T, JT> f, hipStream_t s) {
@@ -488,8 +542,8 @@ void energy(const Grid &g, FV<T, JT> f, const EnergyOut &o, hipStream_t s) {
 
 }  // namespace
 
-void launch_h_half(const Grid &g, FieldPtrs f, DevStatus *reset, hipStream_t s) {
-    h_half(g, view(f), reset, s);
+void launch_h_half(const Grid &g, FieldPtrs f, const HalfOut &o, hipStream_t s) {
+    h_half(g, view(f), o, s);
 }
 void launch_h2(const Grid &g, FieldPtrs f, hipStream_t s) { h2(g, view(f), s); }
 void launch_e(const Grid &g, FieldPtrs f, hipStream_t s) { e_update(g, view(f), s); }
@@ -499,8 +553,8 @@ void launch_energy(const Grid &g, FieldPtrs f, const EnergyOut &o, hipStream_t s
     energy(g, view(f), o, s);
 }
 
-void launch_h_half32(const Grid &g, FieldPtrs32 f, DevStatus *reset, hipStream_t s) {
-    h_half(g, view(f), reset, s);
+void launch_h_half32(const Grid &g, FieldPtrs32 f, const HalfOut &o, hipStream_t s) {
+    h_half(g, view(f), o, s);
 }
 void launch_h2_32(const Grid &g, FieldPtrs32 f, hipStream_t s) { h2(g, view(f), s); }
 void launch_e32(const Grid &g, FieldPtrs32 f, hipStream_t s) { e_update(g, view(f), s); }
@@ -512,11 +566,19 @@ void launch_energy32(const Grid &g, FieldPtrs32 f, const EnergyOut &o, hipStream
     energy(g, view(f), o, s);
 }
 
-void launch_h2_e(const Grid &g, FieldPtrs f, double *const h_out[3], hipStream_t s) {
-    h2_e(g, view(f), HOut<double>{{h_out[0], h_out[1], h_out[2]}}, s);
+void launch_h2_e(const Grid &g, FieldPtrs f, double *const h_out[3], const DevStatus *st,
+                 DevStatus *h_st, hipStream_t s) {
+    h2_e(g, view(f), HOut<double>{{h_out[0], h_out[1], h_out[2]}}, st, h_st, s);
 }
-void launch_h2_e32(const Grid &g, FieldPtrs32 f, float *const h_out[3], hipStream_t s) {
-    h2_e(g, view(f), HOut<float>{{h_out[0], h_out[1], h_out[2]}}, s);
+void launch_h2_e32(const Grid &g, FieldPtrs32 f, float *const h_out[3], const DevStatus *st,
+                   DevStatus *h_st, hipStream_t s) {
+    h2_e(g, view(f), HOut<float>{{h_out[0], h_out[1], h_out[2]}}, st, h_st, s);
+}
+
+void launch_energy_sums(const Grid &g, const double *partials, int rows, double *h_out,
+                        hipStream_t s) {
+    hipLaunchKernelGGL(k_energy_sums, dim3((unsigned)rows), dim3(PIC_BLOCK), 0, s, partials,
+                       (int)blocks_for(g.G), h_out);
 }
 
 void launch_reset_status(DevStatus *st, hipStream_t s) {

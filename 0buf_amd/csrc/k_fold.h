@@ -10,9 +10,12 @@
 
 #include "pic_internal.h"
 
+/* fix (FP64 differentiable form, else null): the current still lies there as
+ * int64 in units of 2^-48, to be converted on the way and cleared */
 template <typename JT>
 struct FoldJ {
     JT *J[3];
+    long long *fix[3];
 };
 
 /* k_fold_j's four operations on one line, restricted to one partner pair:
@@ -117,6 +120,13 @@ __device__ __forceinline__ void class_pairs(const NodeClass &c, JT (&v)[8], int 
         if (!(s & (1 << d)) && c.member(s)) pair(v[s], v[s | (1 << d)], s);
 }
 
+template <typename JT>
+__device__ __forceinline__ JT from_fixed(long long *fix, unsigned n) {
+    const long long v = fix[n];
+    fix[n] = 0;
+    return (JT)((double)v * (1.0 / PIC_J_SCALE64));
+}
+
 /* the three k_fold_j launches x, y, z in one: thread t takes one class of
  * more than one node, folds its current in registers (x pairs, then y, then
  * z, as the launches run, with the same additions) and writes it back */
@@ -127,11 +137,26 @@ __device__ __forceinline__ void fold_class(const Grid &g, const FoldJ<JT> &f, un
     const bool at_n[3] = {c.ri == g.Nx, c.rl == g.Ny, c.rk == g.Nz};
     for (int cc = 0; cc < 3; cc++)
         on_class(c, f.J[cc], [&](JT (&v)[8]) {
+            if (f.fix[cc]) {
+#pragma unroll
+                for (int s = 0; s < 8; s++)
+                    if (c.member(s)) v[s] = from_fixed<JT>(f.fix[cc], c.m[s]);
+            }
 #pragma unroll
             for (int d = 0; d < 3; d++)
                 class_pairs(c, v, d,
                             [&](JT &r, JT &p, int) { fold_pair(r, p, d, cc, at_n[d]); });
         });
+}
+
+/* the nodes no class holds, node n: the conversion alone */
+template <typename JT>
+__device__ __forceinline__ void convert_inner(const Grid &g, const FoldJ<JT> &f, unsigned n) {
+    if (n >= (unsigned)g.G) return;
+    const unsigned t = n / (unsigned)g.sy, k = n - t * (unsigned)g.sy;
+    const unsigned i = t / (unsigned)(g.Ny + 2), l = t - i * (unsigned)(g.Ny + 2);
+    if (i < 2 || (int)i >= g.Nx || l < 2 || (int)l >= g.Ny || k < 2 || (int)k >= g.Nz) return;
+    for (int cc = 0; cc < 3; cc++) f.J[cc][n] = from_fixed<JT>(f.fix[cc], n);
 }
 
 /* workgroups of PIC_BLOCK threads that fold every class */

@@ -1079,7 +1079,7 @@ void launch_arrive_fold_f32(const Grid &g, const TileGeom &t, PartPtrs32 p, Layo
     constexpr int per = PIC_BLOCK / 64;
     const unsigned tiles = what & PIC_ARRIVE ? (unsigned)((t.ntiles + per - 1) / per) : 0;
     const unsigned blocks = tiles + (what & PIC_FOLD ? fold_blocks(g) : 0);
-    const FoldJ<long long> J{{f.J[0], f.J[1], f.J[2]}};
+    const FoldJ<long long> J{{f.J[0], f.J[1], f.J[2]}, {nullptr, nullptr, nullptr}};
     hipLaunchKernelGGL((k_arrive_fold32<TXC, TYC, TZC>), dim3(blocks), dim3(PIC_BLOCK), 0, s, g, t,
                        p, L, st, J, tiles);
 }

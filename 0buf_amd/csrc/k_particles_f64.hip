@@ -805,16 +805,22 @@ void launch_jfix_to_f64(const Grid &g, FieldPtrs f, DiffArgs d, hipStream_t s) {
 }
 
 void launch_arrive_fold_f64(const Grid &g, const TileGeom &t, PartPtrs p, QueuePtrs q,
-                            DevStatus *st, FieldPtrs f, int what, hipStream_t s) {
+                            DevStatus *st, FieldPtrs f, long long *const jfix[3], int what,
+                            hipStream_t s) {
     const unsigned tiles = what & PIC_ARRIVE ? (unsigned)t.ntiles : 0;
-    const unsigned blocks = tiles + (what & PIC_FOLD ? fold_blocks(g) : 0);
-    const FoldJ<double> J{{f.f[PIC_JX], f.f[PIC_JY], f.f[PIC_JZ]}};
+    const unsigned fold_end = tiles + (what & PIC_FOLD ? fold_blocks(g) : 0);
+    const unsigned blocks = fold_end + (jfix ? blocks_for(g.G) : 0);
+    FoldJ<double> J{};
+    for (int k = 0; k < 3; k++) {
+        J.J[k] = f.f[PIC_JX + k];
+        if (jfix) J.fix[k] = jfix[k];
+    }
     if (t.TZ == TZS)
         hipLaunchKernelGGL((k_arrive_fold<TXS, TYS, TZS, double>), dim3(blocks), dim3(PIC_BLOCK),
-                           0, s, g, t, p, q, st, J, tiles);
+                           0, s, g, t, p, q, st, J, tiles, fold_end);
     else
         hipLaunchKernelGGL((k_arrive_fold<TXC, TYC, TZC, double>), dim3(blocks), dim3(PIC_BLOCK),
-                           0, s, g, t, p, q, st, J, tiles);
+                           0, s, g, t, p, q, st, J, tiles, fold_end);
 }
 
 void launch_scatter_load(const long *offsets, long ncell, const double *src[6],

@@ -28,10 +28,10 @@
 #include "pic_ctx.h"
 
 namespace picx {
-void enq_h_half(pic_ctx *c, bool begin_step);
-void enq_push(pic_ctx *c);
+void enq_h_half(pic_ctx *c, const HalfOut &o);
+void enq_push(pic_ctx *c, bool convert);
 void enq_arrive_fold(pic_ctx *c, int what);
-void enq_h2_e(pic_ctx *c);
+void enq_h2_e(pic_ctx *c, bool with_status);
 }  // namespace picx
 
 using namespace picx;
@@ -219,23 +219,21 @@ int restore_state(pic_ctx *c, const Compact &src, const FieldSet &f) {
  * (check_segment). */
 int recorded_step(pic_ctx *c, AdjointStore *s, int r) {
     FieldSet &f = s->recf[r];
-    const size_t bytes = c->g.G * elem(c);
-    enq_h_half(c, false);
-    const void *src[6];
-    for (int k = 0; k < 6; k++) src[k] = live_field(c, k);
-    launch_copy6(f.f, src, bytes, c->stream);
+    HalfOut o;
+    o.rec = f.f;
+    enq_h_half(c, o);
     launch_record_offsets(c->g, c->t, live_count(c), live_cap(c), s->tile_sum, c->d_done,
                           s->recoff[r], s->room, c->d_st, c->stream);
     if (c->fp32) c->rec_snap32 = s->rec32[r];
     else c->rec_snap = s->rec[r];
     c->rec_off = s->recoff[r];
     c->rec_room = s->room;
-    enq_push(c);
+    enq_push(c, false);
     c->rec_snap = PartPtrs{};
     c->rec_snap32 = PartPtrs32{};
     c->rec_off = nullptr;
     c->rec_room = 0;
-    enq_arrive_fold(c, PIC_ARRIVE | PIC_FOLD);
+    enq_arrive_fold(c, PIC_ARRIVE | PIC_FOLD | PIC_FIX);
     if (c->fp32) {
         /* the status is checked at the segment's end; only where the first
          * forward needed the repair of a full spill list is each step's
@@ -252,7 +250,7 @@ int recorded_step(pic_ctx *c, AdjointStore *s, int r) {
             }
         }
     }
-    enq_h2_e(c);
+    enq_h2_e(c, false);
     HIPCHK(hipGetLastError());
     return PIC_SUCCESS;
 }
@@ -395,18 +393,17 @@ int pic_forward_record(pic_ctx *c, int nsteps, int ckpt_every, double *energy) {
     const long P = pic_particle_count(c);
     for (int k = 0; k <= nck; k++)
         if ((rc = reserve_state(c, s->ck[k], s->ckf[k], P))) return rc;
+    RunEnergy run;
+    if ((rc = run.start(c, nsteps))) return rc;
     HIPCHK(hipEventRecord(s->ev[0], c->stream));
     for (int t = 0; t < nsteps; t++) {
         if (t % ckpt_every == 0) {
             rc = save_state(c, s->ck[t / ckpt_every], s->ckf[t / ckpt_every]);
             if (rc) return rc;
         }
-        rc = enq_step(c);
-        if (rc) return rc;
-        rc = finish_step(c, true);
+        rc = run.step(t, energy);
         if (rc) return rc;
         s->anomalies += c->last.dropped + c->last.duplicated;
-        if (energy) energy[t] = c->h_red[0];
     }
     rc = save_state(c, s->ck[nck], s->ckf[nck]);
     if (rc) return rc;

@@ -469,13 +469,13 @@ int despill(pic_ctx *c) { return unpack_live32(c, true); }
 int *qcount_ptr(pic_ctx *c) { return c->fp32 ? c->q32.count : c->q.count; }
 
 /* stage launchers dispatching on the form */
-/* begin_step: the status of a new step starts clear */
-void enq_h_half(pic_ctx *c, bool begin_step) {
-    DevStatus *reset = begin_step ? c->d_st : nullptr;
-    if (c->fp32) launch_h_half32(c->g, c->f32, reset, c->stream);
-    else launch_h_half(c->g, c->f, reset, c->stream);
+void enq_h_half(pic_ctx *c, const HalfOut &o) {
+    if (c->fp32) launch_h_half32(c->g, c->f32, o, c->stream);
+    else launch_h_half(c->g, c->f, o, c->stream);
 }
-void enq_push(pic_ctx *c) {
+/* convert: the FP64 differentiable form's fixed-point current into J at once
+ * (else enq_arrive_fold's PIC_FIX does it) */
+void enq_push(pic_ctx *c, bool convert) {
     if (c->fp32) {
         launch_push_deposit_f32(c->g, c->t, c->f32, c->p32, c->alt32, c->lay32, c->q32, c->sp,
                                 c->prm.departure_cap, c->d_st,
@@ -498,21 +498,24 @@ void enq_push(pic_ctx *c) {
         }
         launch_push_deposit_f64(c->g, c->t, c->f, c->p, c->q, c->sp, c->prm.departure_cap,
                                 c->d_st, &d, c->stream);
-        launch_jfix_to_f64(c->g, c->f, d, c->stream);
+        if (convert) launch_jfix_to_f64(c->g, c->f, d, c->stream);
     } else {
         launch_push_deposit_f64(c->g, c->t, c->f, c->p, c->q, c->sp, c->prm.departure_cap,
                                 c->d_st, nullptr, c->stream);
     }
 }
 /* the arrivals of the push, the periodic fold of the current, or both in one
- * launch (PIC_ARRIVE, PIC_FOLD) */
+ * launch (PIC_ARRIVE, PIC_FOLD); PIC_FIX: the fold of a current that enq_push
+ * did not convert */
 void enq_arrive_fold(pic_ctx *c, int what) {
     if (c->fp32) {
         /* the push placed the arrivals; the counts take them in */
         launch_arrive_fold_f32(c->g, c->t, c->p32, c->lay32, c->d_st, c->f32, what, c->stream);
         if (what & PIC_ARRIVE) c->arrival_pending = true;
     } else {
-        launch_arrive_fold_f64(c->g, c->t, c->p, c->q, c->d_st, c->f, what, c->stream);
+        const bool fix = c->diff && (what & PIC_FIX);
+        launch_arrive_fold_f64(c->g, c->t, c->p, c->q, c->d_st, c->f, fix ? c->d_jfix : nullptr,
+                               what, c->stream);
     }
 }
 void enq_fold(pic_ctx *c) {
@@ -535,12 +538,13 @@ void enq_e_periodic(pic_ctx *c) {
  * E update and periodic E ghosts (equal to enq_h2, enq_e, enq_e_periodic bit
  * for bit), H^{n+1} landing in the second H arrays, which then become the
  * live ones */
-void enq_h2_e(pic_ctx *c) {
+void enq_h2_e(pic_ctx *c, bool with_status) {
+    const DevStatus *st = with_status ? c->d_st : nullptr;
     if (c->fp32) {
-        launch_h2_e32(c->g, c->f32, c->h_alt32, c->stream);
+        launch_h2_e32(c->g, c->f32, c->h_alt32, st, c->h_st, c->stream);
         for (int k = 0; k < 3; k++) std::swap(c->f32.H[k], c->h_alt32[k]);
     } else {
-        launch_h2_e(c->g, c->f, c->h_alt, c->stream);
+        launch_h2_e(c->g, c->f, c->h_alt, st, c->h_st, c->stream);
         for (int k = 0; k < 3; k++) std::swap(c->f.f[PIC_HX + k], c->h_alt[k]);
     }
 }
@@ -584,27 +588,82 @@ void accumulate_profile(pic_ctx *c) {
 }
 
 /* one whole step enqueued on the context stream (Plasma::Step,
- * gpu_plasma.h:605-620) in five launches; the energy and the status land in
- * h_red[0] and h_st by the time the stream is done */
-int enq_step(pic_ctx *c) {
+ * gpu_plasma.h:605-620); the status lands in h_st by the time the stream is
+ * done.  Alone in five launches, the energy in h_red[0]; in a run whose next
+ * step sums the energy (`energy` false; `before`: where the partials of the
+ * state it starts from go, or null) in four. */
+int enq_step(pic_ctx *c, double *before, bool energy) {
+    HalfOut o;
+    o.reset = c->d_st;
+    o.partials = before;
     mark(c, PIC_STAGE_H_HALF);
-    enq_h_half(c, true);
+    enq_h_half(c, o);
     mark(c, PIC_STAGE_PUSH_DEPOSIT);
-    enq_push(c);
+    enq_push(c, c->prof);
     mark(c, PIC_STAGE_MIGRATE);
     /* with stage timing on, the arrival and the fold are launched apart, so
      * that each stage's events bracket its own kernels; the fold, H second
      * half, E update and periodic E ghosts are the E stage's (FOLD_J, H2,
      * E_PERIODIC: 0) */
-    enq_arrive_fold(c, c->prof ? PIC_ARRIVE : PIC_ARRIVE | PIC_FOLD);
+    enq_arrive_fold(c, c->prof ? PIC_ARRIVE : PIC_ARRIVE | PIC_FOLD | PIC_FIX);
     mark(c, PIC_STAGE_E);
     if (c->prof) enq_arrive_fold(c, PIC_FOLD);
-    enq_h2_e(c);
+    enq_h2_e(c, !energy);
     mark(c, PIC_STAGE_ENERGY);
-    enq_energy(c, true);
+    if (energy) enq_energy(c, true);
     mark(c, PIC_NSTAGES);
     HIPCHK(hipGetLastError());
     return PIC_SUCCESS;
+}
+
+/* The energies of a run of several steps.  A small step is bound by its
+ * launches, so the first half step of H, which reads E anyway, leaves the
+ * energy of the state it starts from as a partial per workgroup, and one launch
+ * per ENERGY_ROWS steps adds them up: the same bits as the step's own launch,
+ * on grids where a workgroup's nodes are one of that launch's partials (up to
+ * 1024 workgroups; on larger ones, and with stage timing on, each step sums
+ * its energy itself). */
+constexpr int ENERGY_ROWS = 32;
+
+int RunEnergy::start(pic_ctx *ctx, int nsteps) {
+    c = ctx;
+    n = nsteps;
+    rows = first = 0;
+    defer = !c->prof && n > 1 && (c->g.G + PIC_BLOCK - 1) / PIC_BLOCK <= PIC_ENERGY_ROW;
+    if (defer && !c->d_erow)
+        HIPCHK(hipMalloc(&c->d_erow, (size_t)ENERGY_ROWS * PIC_ENERGY_ROW * sizeof(double)));
+    return PIC_SUCCESS;
+}
+
+/* step s of the run, whole: enqueued, waited for, examined; energies (may be
+ * null) filled as far as they are there */
+int RunEnergy::step(int s, double *energies) {
+    const bool last = !defer || s == n - 1;
+    double *before = defer && s > 0 ? c->d_erow + (long)rows * PIC_ENERGY_ROW : nullptr;
+    int rc = enq_step(c, before, last);
+    if (rc) return rc;
+    if (before) rows++;
+    const bool flush = rows > 0 && (rows == ENERGY_ROWS || last);
+    if (flush) launch_energy_sums(c->g, c->d_erow, rows, c->h_red + 1, c->stream);
+    rc = finish_step(c, true);
+    if (flush) take(energies);
+    if (last && energies) energies[s] = c->h_red[0];
+    if (rc && !last) {   /* the run ends here: what it still owes */
+        if (rows) launch_energy_sums(c->g, c->d_erow, rows, c->h_red + 1, c->stream);
+        enq_energy(c, false);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(c->stream));
+        take(energies);
+        if (energies) energies[s] = c->h_red[0];
+    }
+    return rc;
+}
+
+void RunEnergy::take(double *energies) {
+    if (energies)
+        for (int k = 0; k < rows; k++) energies[first + k] = c->h_red[1 + k];
+    first += rows;
+    rows = 0;
 }
 
 /* waits for the stream and examines the status of what ran; have_status: a
@@ -856,6 +915,7 @@ int pic_destroy(pic_ctx *c) {
     if (c->h_st) hipHostFree(c->h_st);
     if (c->d_part) hipFree(c->d_part);
     if (c->d_done) hipFree(c->d_done);
+    if (c->d_erow) hipFree(c->d_erow);
     if (c->d_red) hipFree(c->d_red);
     if (c->h_red) hipHostFree(c->h_red);
     if (c->d_slot_sort) hipFree(c->d_slot_sort);
@@ -1059,7 +1119,9 @@ int pic_get_field(pic_ctx *c, int which, double *host) {
 int pic_yee_h_half(pic_ctx *c) {
     int rc = check_ready(c);
     if (rc) return rc;
-    enq_h_half(c, true);
+    HalfOut o;
+    o.reset = c->d_st;
+    enq_h_half(c, o);
     HIPCHK(hipGetLastError());
     return PIC_SUCCESS;
 }
@@ -1070,7 +1132,7 @@ int pic_push_deposit(pic_ctx *c) {
     /* an arrival whose status was not examined (no pic_sync since): its
      * repair comes first */
     if (c->arrival_pending && (rc = finish_step(c))) return rc;
-    enq_push(c);
+    enq_push(c, true);
     HIPCHK(hipGetLastError());
     return PIC_SUCCESS;
 }
@@ -1132,7 +1194,7 @@ int pic_step(pic_ctx *c, int nt, double *energy) {
     if (rc) return rc;
     HIPCHK(hipSetDevice(c->dev));
     if (c->arrival_pending && (rc = finish_step(c))) return rc;
-    rc = enq_step(c);
+    rc = enq_step(c, nullptr, true);
     if (rc) return rc;
     rc = finish_step(c, true);
     accumulate_profile(c);
@@ -1141,8 +1203,17 @@ int pic_step(pic_ctx *c, int nt, double *energy) {
 }
 
 int pic_run(pic_ctx *c, int nt0, int nsteps, double *energies) {
+    (void)nt0;
+    if (nsteps <= 0) return PIC_SUCCESS;
+    int rc = check_ready(c);
+    if (rc) return rc;
+    HIPCHK(hipSetDevice(c->dev));
+    if (c->arrival_pending && (rc = finish_step(c))) return rc;
+    RunEnergy run;
+    if ((rc = run.start(c, nsteps))) return rc;
     for (int s = 0; s < nsteps; s++) {
-        int rc = pic_step(c, nt0 + s, energies ? &energies[s] : nullptr);
+        rc = run.step(s, energies);
+        accumulate_profile(c);
         if (rc) return rc;
     }
     return PIC_SUCCESS;

@@ -77,6 +77,7 @@ struct pic_ctx {
     double *d_part = nullptr;
     int npart = 1024;
     unsigned *d_done = nullptr;   /* workgroups done with the energy reduction */
+    double *d_erow = nullptr;     /* RunEnergy's partials */
     double *d_red = nullptr;
     double *h_red = nullptr;
     Staged staged;
@@ -101,7 +102,16 @@ extern thread_local char g_hip_err[256];
 int record_hip(hipError_t e, const char *where);
 int commit(pic_ctx *c);
 int check_ready(pic_ctx *c);
-int enq_step(pic_ctx *c);
+int enq_step(pic_ctx *c, double *before, bool energy);
+/* the steps of a run of n and their energies (pic_api.hip) */
+struct RunEnergy {
+    pic_ctx *c;
+    int n, rows, first;
+    bool defer;
+    int start(pic_ctx *ctx, int nsteps);
+    int step(int s, double *energies);
+    void take(double *energies);
+};
 int finish_step(pic_ctx *c, bool have_status = false);
 /* FP32 form: put every particle into the bucket arrays (unpack the packed
  * set with its pending arrivals) before anything other than the push reads

@@ -62,6 +62,8 @@ struct FieldPtrs {
  * resolution 2^-40 (exact, order-free accumulation) */
 #define PIC_J_SCALE 1099511627776.0           /* 2^40 */
 #define PIC_J_INV (1.0 / 1099511627776.0)
+/* ... of the FP64 differentiable form's current: 2^-48 */
+#define PIC_J_SCALE64 281474976710656.0       /* 2^48 */
 
 struct FieldPtrs32 {
     float *E[3], *H[3], *Q[3];
@@ -405,8 +407,11 @@ inline int push_threads(long ntiles) {
  * second H arrays; the caller swaps them with the live ones), the E update
  * and the periodic E ghosts, equal to launch_h2, launch_e,
  * launch_e_periodic bit for bit */
-void launch_h2_e(const Grid &g, FieldPtrs f, double *const h_out[3], hipStream_t s);
-void launch_h2_e32(const Grid &g, FieldPtrs32 f, float *const h_out[3], hipStream_t s);
+/* st (may be null): the step's status, copied to h_st (pinned host memory) */
+void launch_h2_e(const Grid &g, FieldPtrs f, double *const h_out[3], const DevStatus *st,
+                 DevStatus *h_st, hipStream_t s);
+void launch_h2_e32(const Grid &g, FieldPtrs32 f, float *const h_out[3], const DevStatus *st,
+                   DevStatus *h_st, hipStream_t s);
 /* where an energy reduction leaves its result */
 struct EnergyOut {
     double *partials;        /* 1024 */
@@ -415,15 +420,29 @@ struct EnergyOut {
     const DevStatus *st;     /* the step's status, copied to h_st (null: not) */
     DevStatus *h_st;         /* pinned host memory */
 };
-/* reset (may be null): the status to clear for the step that begins */
-void launch_h_half(const Grid &g, FieldPtrs f, DevStatus *reset, hipStream_t s);
+/* what else the first half step of H leaves behind: reset (may be null), the
+ * status to clear for the step that begins; rec (null: not), copies of E and of
+ * the half-stepped H for a step record; partials (null: not; grids of at most
+ * 1024 blocks of PIC_BLOCK nodes), the energy of each block of nodes of the E it
+ * starts from, for launch_energy_sums */
+struct HalfOut {
+    DevStatus *reset = nullptr;
+    void *const *rec = nullptr;
+    double *partials = nullptr;
+};
+/* the energies of `rows` states from their blocks' energies, 1024 a row, into
+ * h_out (pinned host memory): the bits launch_energy gives */
+void launch_energy_sums(const Grid &g, const double *partials, int rows, double *h_out,
+                        hipStream_t s);
+constexpr int PIC_ENERGY_ROW = 1024;
+void launch_h_half(const Grid &g, FieldPtrs f, const HalfOut &o, hipStream_t s);
 void launch_h2(const Grid &g, FieldPtrs f, hipStream_t s);
 void launch_e(const Grid &g, FieldPtrs f, hipStream_t s);
 void launch_e_periodic(const Grid &g, FieldPtrs f, hipStream_t s);
 void launch_fold_j(const Grid &g, FieldPtrs f, hipStream_t s);
 void launch_energy(const Grid &g, FieldPtrs f, const EnergyOut &o, hipStream_t s);
 void launch_reset_status(DevStatus *st, hipStream_t s);
-void launch_h_half32(const Grid &g, FieldPtrs32 f, DevStatus *reset, hipStream_t s);
+void launch_h_half32(const Grid &g, FieldPtrs32 f, const HalfOut &o, hipStream_t s);
 void launch_h2_32(const Grid &g, FieldPtrs32 f, hipStream_t s);
 void launch_e32(const Grid &g, FieldPtrs32 f, hipStream_t s);
 void launch_e_periodic32(const Grid &g, FieldPtrs32 f, hipStream_t s);
@@ -438,7 +457,6 @@ TileGeom make_tile_geom(int Nx, int Ny, int Nz, bool small_ok);
  * when snap.p[0] is set the push also writes the pre-step particle state into
  * the compact record `snap`: tile t's particles, in the push's flat order,
  * at snap_off[t] + (flat index), and each cell's count in snap.count. */
-#define PIC_J_SCALE64 281474976710656.0       /* 2^48 */
 struct DiffArgs {
     long long *jfix[3];
     PartPtrs snap;
@@ -464,16 +482,17 @@ void launch_jfix_to_f64(const Grid &g, FieldPtrs f, DiffArgs d, hipStream_t s);
  * scratch entry per tile */
 void launch_tile_order(const Grid &g, const TileGeom &t, const long *off, int *cnt, int *order,
                        hipStream_t s);
-/* six device arrays of `bytes` (a multiple of 4) each, in one launch */
-void launch_copy6(void *const dst[6], const void *const src[6], size_t bytes, hipStream_t s);
 void launch_record_offsets(const Grid &g, const TileGeom &t, const int *count, int cap,
                            long *tile_sum, unsigned *done, long *off, long room, DevStatus *st,
                            hipStream_t s);
 /* the arrivals of a push and the periodic fold of the current, in one launch,
  * or one of the two */
-enum { PIC_ARRIVE = 1, PIC_FOLD = 2 };
+enum { PIC_ARRIVE = 1, PIC_FOLD = 2, PIC_FIX = 4 };
+/* jfix: with the fold, the differentiable form's fixed-point current
+ * converted on the way and cleared (null: the current is in f already) */
 void launch_arrive_fold_f64(const Grid &g, const TileGeom &t, PartPtrs p, QueuePtrs q,
-                            DevStatus *st, FieldPtrs f, int what, hipStream_t s);
+                            DevStatus *st, FieldPtrs f, long long *const jfix[3], int what,
+                            hipStream_t s);
 void launch_scatter_load(const long *offsets, long ncell, const double *src[6],
                          const unsigned char *srcsp, PartPtrs p, hipStream_t s);
 void launch_repack(long ncell, PartPtrs from, PartPtrs to, hipStream_t s);
