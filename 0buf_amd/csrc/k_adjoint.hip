@@ -45,11 +45,13 @@ constexpr int copy_stride(int n) { return (n + 6) / 16 * 16 + 9; }   /* >= n, 9 
 
 inline unsigned blocks_for(long n) { return (unsigned)((n + PIC_BLOCK - 1) / PIC_BLOCK); }
 
-__device__ __forceinline__ void decode(const Grid &g, long n, int &i, int &l, int &k) {
-    k = (int)(n % g.sy);
-    long t = n / g.sy;
-    l = (int)(t % (g.Ny + 2));
-    i = (int)(t / (g.Ny + 2));
+/* 32-bit arithmetic: the grid has fewer than 2^31 nodes */
+__device__ __forceinline__ void decode32(const Grid &g, unsigned n, int &i, int &l, int &k) {
+    const unsigned sy = (unsigned)g.sy, ny2 = (unsigned)(g.Ny + 2), t = n / sy;
+    k = (int)(n - t * sy);
+    const unsigned ii = t / ny2;
+    l = (int)(t - ii * ny2);
+    i = (int)ii;
 }
 
 __global__ __launch_bounds__(PIC_BLOCK) void k_adj_seed_energy(Grid g, const double *Ex,
@@ -74,23 +76,22 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_adj_e_periodic(Grid g, AdjLam lam
     const unsigned t = blockIdx.x * PIC_BLOCK + threadIdx.x;
     if (t >= shell_count(g)) return;
     const NodeClass c = node_class(g, t);
-    for (int cc = 0; cc < 3; cc++)
-        on_class(c, lam.E[cc], [&](double (&v)[8]) {
-            auto back = [&](int d, auto in_range) {
-                class_pairs(c, v, d, [&](double &r, double &p, int s) {
-                    if (!in_range(s)) return;
-                    r += p;
-                    p = 0.0;
-                });
-            };
-            if (g.ghost_mode == 1 && cc != 1) back(1, [](int) { return true; });
-            if (cc == 0) back(2, [&](int s) { return c.i(s) <= g.Nx; });
-            if (cc == 1) back(2, [&](int s) { return c.l(s) <= g.Ny; });
-            if (cc == 1)
-                back(0, [&](int s) { return c.l(s) <= g.Ny && c.k(s) >= 1 && c.k(s) <= g.Nz; });
-            if (cc == 2)
-                back(0, [&](int s) { return c.l(s) >= 1 && c.l(s) <= g.Ny && c.k(s) <= g.Nz; });
-        });
+    on_class(c, lam.E, [&](int cc, double (&v)[8]) {
+        auto back = [&](int d, auto in_range) {
+            class_pairs(c, v, d, [&](double &r, double &p, int s) {
+                if (!in_range(s)) return;
+                r += p;
+                p = 0.0;
+            });
+        };
+        if (g.ghost_mode == 1 && cc != 1) back(1, [](int) { return true; });
+        if (cc == 0) back(2, [&](int s) { return c.i(s) <= g.Nx; });
+        if (cc == 1) back(2, [&](int s) { return c.l(s) <= g.Ny; });
+        if (cc == 1)
+            back(0, [&](int s) { return c.l(s) <= g.Ny && c.k(s) >= 1 && c.k(s) <= g.Nz; });
+        if (cc == 2)
+            back(0, [&](int s) { return c.l(s) >= 1 && c.l(s) <= g.Ny && c.k(s) <= g.Nz; });
+    });
 }
 
 /* E-update ranges (emeElement, kernels.cu:1162-1181) */
@@ -121,22 +122,29 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_adj_curl_e(Grid g, AdjLam lam) {
     const long n = (long)blockIdx.x * PIC_BLOCK + threadIdx.x;
     if (n >= g.G) return;
     int i, l, k;
-    decode(g, n, i, l, k);
+    decode32(g, (unsigned)n, i, l, k);
     const double c1x = g.tau / g.hx, c1y = g.tau / g.hy, c1z = g.tau / g.hz, tau = g.tau;
     const double *LEx = lam.E[0], *LEy = lam.E[1], *LEz = lam.E[2];
     const long sy = g.sy, sx = g.sx;
-    const double ex = in_ex(g, i, l, k) ? LEx[n] : 0.0;
-    const double ey = in_ey(g, i, l, k) ? LEy[n] : 0.0;
-    const double ez = in_ez(g, i, l, k) ? LEz[n] : 0.0;
-    const double ex_l = in_ex(g, i, l + 1, k) ? LEx[n + sy] : 0.0;
-    const double ex_k = in_ex(g, i, l, k + 1) ? LEx[n + 1] : 0.0;
-    const double ey_i = in_ey(g, i + 1, l, k) ? LEy[n + sx] : 0.0;
-    const double ey_k = in_ey(g, i, l, k + 1) ? LEy[n + 1] : 0.0;
-    const double ez_i = in_ez(g, i + 1, l, k) ? LEz[n + sx] : 0.0;
-    const double ez_l = in_ez(g, i, l + 1, k) ? LEz[n + sy] : 0.0;
-    const double hx = lam.H[0][n] + (c1z * (ey - ey_k) - c1y * (ez - ez_l));
-    const double hy = lam.H[1][n] + (-c1z * (ex - ex_k) + c1x * (ez - ez_i));
-    const double hz = lam.H[2][n] + (c1y * (ex - ex_l) - c1x * (ey - ey_i));
+    /* every load first (the node itself past the end), then the ranges: behind
+     * the tests they were waited for in turn */
+    const long nl = n + sy < g.G ? n + sy : n, nk = n + 1 < g.G ? n + 1 : n,
+               ni = n + sx < g.G ? n + sx : n;
+    const double vx = LEx[n], vy = LEy[n], vz = LEz[n], vxl = LEx[nl], vxk = LEx[nk],
+                 vyi = LEy[ni], vyk = LEy[nk], vzi = LEz[ni], vzl = LEz[nl];
+    const double H0 = lam.H[0][n], H1 = lam.H[1][n], H2 = lam.H[2][n];
+    const double ex = in_ex(g, i, l, k) ? vx : 0.0;
+    const double ey = in_ey(g, i, l, k) ? vy : 0.0;
+    const double ez = in_ez(g, i, l, k) ? vz : 0.0;
+    const double ex_l = in_ex(g, i, l + 1, k) ? vxl : 0.0;
+    const double ex_k = in_ex(g, i, l, k + 1) ? vxk : 0.0;
+    const double ey_i = in_ey(g, i + 1, l, k) ? vyi : 0.0;
+    const double ey_k = in_ey(g, i, l, k + 1) ? vyk : 0.0;
+    const double ez_i = in_ez(g, i + 1, l, k) ? vzi : 0.0;
+    const double ez_l = in_ez(g, i, l + 1, k) ? vzl : 0.0;
+    const double hx = H0 + (c1z * (ey - ey_k) - c1y * (ez - ez_l));
+    const double hy = H1 + (-c1z * (ex - ex_k) + c1x * (ez - ez_i));
+    const double hz = H2 + (c1y * (ex - ex_l) - c1x * (ey - ey_i));
     lam.H[0][n] = hx;
     lam.H[1][n] = hy;
     lam.H[2][n] = hz;
@@ -157,20 +165,19 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_adj_fold_j(Grid g, AdjLam lam) {
     if (t >= shell_count(g)) return;
     const NodeClass c = node_class(g, t);
     const bool at_n[3] = {c.ri == g.Nx, c.rl == g.Ny, c.rk == g.Nz};
-    for (int cc = 0; cc < 3; cc++)
-        on_class(c, lam.J[cc], [&](double (&v)[8]) {
+    on_class(c, lam.J, [&](int cc, double (&v)[8]) {
 #pragma unroll
-            for (int d = 2; d >= 0; d--)
-                class_pairs(c, v, d, [&](double &r, double &p, int) {
-                    if (at_n[d] || d != cc) {          /* both ends take the sum */
-                        r += p;
-                        p = r;
-                    } else if (d != 1) {
-                        r += p;
-                        p = 0.0;
-                    }
-                });
-        });
+        for (int d = 2; d >= 0; d--)
+            class_pairs(c, v, d, [&](double &r, double &p, int) {
+                if (at_n[d] || d != cc) {          /* both ends take the sum */
+                    r += p;
+                    p = r;
+                } else if (d != 1) {
+                    r += p;
+                    p = 0.0;
+                }
+            });
+    });
 }
 
 /* transpose of Q = Ch E:  Qx = 1/2(c1z(Ey[k+1]-Ey) - c1y(Ez[l+1]-Ez)) etc.,
@@ -179,28 +186,26 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_adj_curl_h(Grid g, AdjLam lam) {
     const long n = (long)blockIdx.x * PIC_BLOCK + threadIdx.x;
     if (n >= g.G) return;
     int i, l, k;
-    decode(g, n, i, l, k);
+    decode32(g, (unsigned)n, i, l, k);
     const double c1x = g.tau / g.hx, c1y = g.tau / g.hy, c1z = g.tau / g.hz;
     const long sy = g.sy, sx = g.sx;
-    auto mux = [&](int ii, int ll, int kk, long m) {
-        return in_qx(g, ii, ll, kk) ? lam.Q[0][m] + lam.H[0][m] : 0.0;
-    };
-    auto muy = [&](int ii, int ll, int kk, long m) {
-        return in_qy(g, ii, ll, kk) ? lam.Q[1][m] + lam.H[1][m] : 0.0;
-    };
-    auto muz = [&](int ii, int ll, int kk, long m) {
-        return in_qz(g, ii, ll, kk) ? lam.Q[2][m] + lam.H[2][m] : 0.0;
-    };
-    const double mx = mux(i, l, k, n), my = muy(i, l, k, n), mz = muz(i, l, k, n);
-    const double mx_k = k >= 1 ? mux(i, l, k - 1, n - 1) : 0.0;
-    const double mx_l = l >= 1 ? mux(i, l - 1, k, n - sy) : 0.0;
-    const double my_k = k >= 1 ? muy(i, l, k - 1, n - 1) : 0.0;
-    const double my_i = i >= 1 ? muy(i - 1, l, k, n - sx) : 0.0;
-    const double mz_l = l >= 1 ? muz(i, l - 1, k, n - sy) : 0.0;
-    const double mz_i = i >= 1 ? muz(i - 1, l, k, n - sx) : 0.0;
-    lam.E[0][n] += 0.5 * (c1z * (my - my_k) + c1y * (mz_l - mz));
-    lam.E[1][n] += 0.5 * (c1z * (mx_k - mx) + c1x * (mz - mz_i));
-    lam.E[2][n] += 0.5 * (c1y * (mx - mx_l) + c1x * (my_i - my));
+    /* every load first (the node itself where a neighbour is missing) */
+    const long nk = k >= 1 ? n - 1 : n, nl = l >= 1 ? n - sy : n, ni = i >= 1 ? n - sx : n;
+    auto mu = [&](int d, long m) { return lam.Q[d][m] + lam.H[d][m]; };
+    const double x = mu(0, n), y = mu(1, n), z = mu(2, n), xk = mu(0, nk), xl = mu(0, nl),
+                 yk = mu(1, nk), yi = mu(1, ni), zl = mu(2, nl), zi = mu(2, ni);
+    const double E0 = lam.E[0][n], E1 = lam.E[1][n], E2 = lam.E[2][n];
+    const double mx = in_qx(g, i, l, k) ? x : 0.0, my = in_qy(g, i, l, k) ? y : 0.0,
+                 mz = in_qz(g, i, l, k) ? z : 0.0;
+    const double mx_k = k >= 1 && in_qx(g, i, l, k - 1) ? xk : 0.0;
+    const double mx_l = l >= 1 && in_qx(g, i, l - 1, k) ? xl : 0.0;
+    const double my_k = k >= 1 && in_qy(g, i, l, k - 1) ? yk : 0.0;
+    const double my_i = i >= 1 && in_qy(g, i - 1, l, k) ? yi : 0.0;
+    const double mz_l = l >= 1 && in_qz(g, i, l - 1, k) ? zl : 0.0;
+    const double mz_i = i >= 1 && in_qz(g, i - 1, l, k) ? zi : 0.0;
+    lam.E[0][n] = E0 + 0.5 * (c1z * (my - my_k) + c1y * (mz_l - mz));
+    lam.E[1][n] = E1 + 0.5 * (c1z * (mx_k - mx) + c1x * (mz - mz_i));
+    lam.E[2][n] = E2 + 0.5 * (c1y * (mx - mx_l) + c1x * (my_i - my));
 }
 
 /* ---------------------------------------------------------------- particles */

@@ -33,9 +33,11 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_arrive_fold(Grid g, TileGeom t, P
                                                            QueuePtrs q, DevStatus *st,
                                                            FoldJ<JT> f, unsigned tiles,
                                                            unsigned fold_end) {
-    if (blockIdx.x >= fold_end) {
-        convert_inner(g, f, (blockIdx.x - fold_end) * PIC_BLOCK + threadIdx.x);
-        return;
+    if constexpr (std::is_floating_point_v<JT>) {
+        if (blockIdx.x >= fold_end) {
+            convert_inner(g, f, (blockIdx.x - fold_end) * PIC_BLOCK + threadIdx.x);
+            return;
+        }
     }
     if (blockIdx.x >= tiles) {
         fold_class(g, f, (blockIdx.x - tiles) * PIC_BLOCK + threadIdx.x);

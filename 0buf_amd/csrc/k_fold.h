@@ -8,6 +8,8 @@
 #ifndef K_FOLD_H
 #define K_FOLD_H
 
+#include <type_traits>
+
 #include "pic_internal.h"
 
 /* fix (FP64 differentiable form, else null): the current still lies there as
@@ -17,6 +19,10 @@ struct FoldJ {
     JT *J[3];
     long long *fix[3];
 };
+
+__device__ __forceinline__ double from_fixed(long long v) {
+    return (double)v * (1.0 / PIC_J_SCALE64);
+}
 
 /* k_fold_j's four operations on one line, restricted to one partner pair:
  * r at the representative (position N or 1), p at its partner (0 or N+1),
@@ -97,17 +103,29 @@ __device__ __forceinline__ NodeClass node_class(const Grid &g, unsigned t) {
     return c;
 }
 
-/* the values of one component at the class's nodes, op on them, and back:
- * op(v) works on v[8] in registers */
+/* the values of the three components at the class's nodes, op(component, v) on
+ * each component's v[8] in registers, and back.  Every load is issued before
+ * the first operation (a component after the other, each waited for memory on
+ * its own: the arrival and fold of a small step 4.6 against 5.7 us, with the
+ * conversion of a fixed-point current 8.6 against 11). */
+template <typename JT, class Load, class Op>
+__device__ __forceinline__ void on_class(const NodeClass &c, JT *const (&J)[3], Load load, Op op) {
+    JT v[3][8];
+#pragma unroll
+    for (int cc = 0; cc < 3; cc++)
+#pragma unroll
+        for (int s = 0; s < 8; s++) v[cc][s] = c.member(s) ? load(cc, c.m[s]) : (JT)0;
+#pragma unroll
+    for (int cc = 0; cc < 3; cc++) op(cc, v[cc]);
+#pragma unroll
+    for (int cc = 0; cc < 3; cc++)
+#pragma unroll
+        for (int s = 0; s < 8; s++)
+            if (c.member(s)) J[cc][c.m[s]] = v[cc][s];
+}
 template <typename JT, class Op>
-__device__ __forceinline__ void on_class(const NodeClass &c, JT *J, Op op) {
-    JT v[8];
-#pragma unroll
-    for (int s = 0; s < 8; s++) v[s] = c.member(s) ? J[c.m[s]] : (JT)0;
-    op(v);
-#pragma unroll
-    for (int s = 0; s < 8; s++)
-        if (c.member(s)) J[c.m[s]] = v[s];
+__device__ __forceinline__ void on_class(const NodeClass &c, JT *const (&J)[3], Op op) {
+    on_class(c, J, [&](int cc, unsigned m) { return J[cc][m]; }, op);
 }
 
 /* pair(v at the representative's side, v at the partner's, member s) over the
@@ -120,13 +138,6 @@ __device__ __forceinline__ void class_pairs(const NodeClass &c, JT (&v)[8], int 
         if (!(s & (1 << d)) && c.member(s)) pair(v[s], v[s | (1 << d)], s);
 }
 
-template <typename JT>
-__device__ __forceinline__ JT from_fixed(long long *fix, unsigned n) {
-    const long long v = fix[n];
-    fix[n] = 0;
-    return (JT)((double)v * (1.0 / PIC_J_SCALE64));
-}
-
 /* the three k_fold_j launches x, y, z in one: thread t takes one class of
  * more than one node, folds its current in registers (x pairs, then y, then
  * z, as the launches run, with the same additions) and writes it back */
@@ -135,28 +146,35 @@ __device__ __forceinline__ void fold_class(const Grid &g, const FoldJ<JT> &f, un
     if (t >= shell_count(g)) return;
     const NodeClass c = node_class(g, t);
     const bool at_n[3] = {c.ri == g.Nx, c.rl == g.Ny, c.rk == g.Nz};
-    for (int cc = 0; cc < 3; cc++)
-        on_class(c, f.J[cc], [&](JT (&v)[8]) {
-            if (f.fix[cc]) {
+    auto fold = [&](int cc, JT (&v)[8]) {
 #pragma unroll
+        for (int d = 0; d < 3; d++)
+            class_pairs(c, v, d, [&](JT &r, JT &p, int) { fold_pair(r, p, d, cc, at_n[d]); });
+    };
+    if constexpr (std::is_floating_point_v<JT>) {
+        if (f.fix[0]) {
+            on_class(c, f.J, [&](int cc, unsigned m) { return from_fixed(f.fix[cc][m]); }, fold);
+            for (int cc = 0; cc < 3; cc++)
                 for (int s = 0; s < 8; s++)
-                    if (c.member(s)) v[s] = from_fixed<JT>(f.fix[cc], c.m[s]);
-            }
-#pragma unroll
-            for (int d = 0; d < 3; d++)
-                class_pairs(c, v, d,
-                            [&](JT &r, JT &p, int) { fold_pair(r, p, d, cc, at_n[d]); });
-        });
+                    if (c.member(s)) f.fix[cc][c.m[s]] = 0;
+            return;
+        }
+    }
+    on_class(c, f.J, fold);
 }
 
 /* the nodes no class holds, node n: the conversion alone */
-template <typename JT>
-__device__ __forceinline__ void convert_inner(const Grid &g, const FoldJ<JT> &f, unsigned n) {
+__device__ __forceinline__ void convert_inner(const Grid &g, const FoldJ<double> &f, unsigned n) {
     if (n >= (unsigned)g.G) return;
     const unsigned t = n / (unsigned)g.sy, k = n - t * (unsigned)g.sy;
     const unsigned i = t / (unsigned)(g.Ny + 2), l = t - i * (unsigned)(g.Ny + 2);
     if (i < 2 || (int)i >= g.Nx || l < 2 || (int)l >= g.Ny || k < 2 || (int)k >= g.Nz) return;
-    for (int cc = 0; cc < 3; cc++) f.J[cc][n] = from_fixed<JT>(f.fix[cc], n);
+    long long v[3];
+    for (int cc = 0; cc < 3; cc++) v[cc] = f.fix[cc][n];
+    for (int cc = 0; cc < 3; cc++) {
+        f.J[cc][n] = from_fixed(v[cc]);
+        f.fix[cc][n] = 0;
+    }
 }
 
 /* workgroups of PIC_BLOCK threads that fold every class */
