@@ -405,6 +405,7 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
     }
     __syncthreads();
     const int T = sOff[C];
+    const long rec0 = uniform(a.snap_off[tile]);
 
     const double hx = g.hx, hy = g.hy, hz = g.hz, tau = g.tau;
     unsigned bad = 0;
@@ -417,7 +418,7 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
         const int c = lo;
         const int ca = c / (TY * TZ), cb = (c / TZ) % TY, cc = c % TZ;
         const int gi = I0 + ca, gl = L0 + cb, gk = K0 + cc;
-        const long pidx = a.snap_off[tile] + fidx;    /* compact record */
+        const long pidx = rec0 + fidx;    /* compact record */
         Geo G;
         G.n0 = (ca * BY + cb) * BZ + cc;
         G.hx = hx; G.hy = hy; G.hz = hz;

@@ -215,6 +215,7 @@ __global__ __launch_bounds__(NT) void k_adj_particles32(AdjArgs32 a) {
     }
     __syncthreads();
     const int T = sOff[C];
+    const long rec0 = uniform(a.snap_off[tile]);
 
     for (int fidx = tid; fidx < T; fidx += NT) {
         int blo = 0, bhi = C;
@@ -224,7 +225,7 @@ __global__ __launch_bounds__(NT) void k_adj_particles32(AdjArgs32 a) {
         }
         const int c = blo;
         const int ca = c / (TY * TZ), cb = (c / TZ) % TY, cc = c % TZ;
-        const long pidx = a.snap_off[tile] + fidx;    /* compact record */
+        const long pidx = rec0 + fidx;    /* compact record */
         const float o[3] = {a.p.p[0][pidx], a.p.p[1][pidx], a.p.p[2][pidx]};
         const float pu = a.p.p[3][pidx], pv = a.p.p[4][pidx], pw = a.p.p[5][pidx];
         const unsigned char s = a.p.sp[pidx];

@@ -283,6 +283,11 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
     int *const ID = DIFF ? a.p.id + pbase : nullptr;
     Leaver64 *const QT = a.q.e + tile * (long)a.q.qcap;   /* the tile's departure queue */
 
+    /* where the tile's record starts and how many of its particles have room
+     * there, read before the loop: a load in it waits for every one before */
+    const long snap0 = snap ? uniform(a.d.snap_off[tile]) : 0;
+    const unsigned snap_n = record_room(snap, snap0, a.d.snap_room);
+
     const double hx = g.hx, hy = g.hy, hz = g.hz, tau = g.tau;
     unsigned bad = 0;
     /* each wavefront owns whole cells and walks their particles in chunks of
@@ -335,16 +340,16 @@ __global__ __launch_bounds__(NT, 4) void k_push_deposit(PushArgs a) {
                 if (tin) tw = a.d.tape_row[pid];
                 if (!tin || !((tw >> TAPE_VALID) & 1ull) || ((tw >> TAPE_BAD) & 1ull)) bad = 1;
             }
-            const long r = snap ? a.d.snap_off[tile] + sOff[c] + j : 0;
-            if (snap && r < a.d.snap_room) {
-                a.d.snap.p[0][r] = x;
-                a.d.snap.p[1][r] = y;
-                a.d.snap.p[2][r] = z;
-                a.d.snap.p[3][r] = pu;
-                a.d.snap.p[4][r] = pv;
-                a.d.snap.p[5][r] = pw;
-                a.d.snap.sp[r] = s;
-                a.d.snap.id[r] = pid;
+            const unsigned r = (unsigned)(sOff[c] + j);
+            if (r < snap_n) {
+                slot(a.d.snap.p[0] + snap0, r) = x;
+                slot(a.d.snap.p[1] + snap0, r) = y;
+                slot(a.d.snap.p[2] + snap0, r) = z;
+                slot(a.d.snap.p[3] + snap0, r) = pu;
+                slot(a.d.snap.p[4] + snap0, r) = pv;
+                slot(a.d.snap.p[5] + snap0, r) = pw;
+                slot(a.d.snap.sp + snap0, r) = s;
+                slot(a.d.snap.id + snap0, r) = pid;
             }
 
             /* relative to the owner cell's corner */

@@ -203,6 +203,20 @@ __device__ __forceinline__ T &slot(T *base, unsigned rel) {
     return *(T *)((char *)base + rel * (unsigned)sizeof(T));
 }
 
+/* a value every lane holds, in scalar registers */
+__device__ __forceinline__ long uniform(long v) {
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)v),
+                   hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32));
+    return (long)((unsigned long)hi << 32 | lo);
+}
+
+/* of a tile's step record that starts at entry `start`: the entries it may
+ * write, 0 where none is kept (a tile's particles address in 32 bits) */
+__device__ __forceinline__ unsigned record_room(bool on, long start, long room) {
+    const long n = room - start;
+    return !on || n <= 0 ? 0u : n < (1L << 29) ? (unsigned)n : 1u << 29;
+}
+
 /* Stable in-place compaction by wavefronts.  Each wavefront of a push
  * workgroup owns whole cells of the tile (wave_first_cell) and walks them in
  * flat order, one chunk of up to 64 consecutive particles at a time
