@@ -112,8 +112,7 @@ def run_form(pic, params, cfg, parts, bx0, precision, steps, warmup, stage_steps
     """Load the workload into a context of the given precision (drawn on the
     GPU by the device initializer, or the host-generated `parts`); `warmup`
     untimed steps; `steps` timed steps of pic_step as a caller runs it (stage
-    timing off, so the arrival runs on its second stream beside the field
-    stages), bracketed by torch.cuda.synchronize; then `stage_steps` more
+    timing off), bracketed by torch.cuda.synchronize; then `stage_steps` more
     steps with stage timing on (HIP events on the context's stream around
     each stage) for the per-stage and push-kernel times."""
     import torch
