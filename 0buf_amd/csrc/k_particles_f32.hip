@@ -701,24 +701,23 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_scatter_load32(const long *off, l
                                                              const float *s4, const float *s5,
                                                              const unsigned char *ssp,
                                                              PartPtrs32 p) {
-    const long e = (long)blockIdx.x * PIC_BLOCK + threadIdx.x;
-    if (e >= ncell * p.cap) return;
-    const long c = e / p.cap;
-    const int j = (int)(e % p.cap);
-    const long n = off[c + 1] - off[c];
-    if (j == 0) {
+    const long c = group_cell_index();
+    if (c >= ncell) return;
+    const long first = off[c], n = off[c + 1] - first;
+    if (threadIdx.x % CELL_LANES == 0) {
         p.count[c] = (int)n;
         if (p.bcount) p.bcount[c] = (int)n;
     }
-    if (j >= n) return;
-    const long src = off[c] + j;
-    p.p[0][e] = s0[src];
-    p.p[1][e] = s1[src];
-    p.p[2][e] = s2[src];
-    p.p[3][e] = s3[src];
-    p.p[4][e] = s4[src];
-    p.p[5][e] = s5[src];
-    p.sp[e] = ssp[src];
+    for (int j = threadIdx.x % CELL_LANES; j < n && j < p.cap; j += CELL_LANES) {
+        const long e = c * p.cap + j, src = first + j;
+        p.p[0][e] = s0[src];
+        p.p[1][e] = s1[src];
+        p.p[2][e] = s2[src];
+        p.p[3][e] = s3[src];
+        p.p[4][e] = s4[src];
+        p.p[5][e] = s5[src];
+        p.sp[e] = ssp[src];
+    }
 }
 
 /* bulk cell of halo-box cell h of a tile (periodic wrap) */
@@ -838,25 +837,25 @@ template <int TX, int TY, int TZ>
 __global__ __launch_bounds__(PIC_BLOCK) void k_unpack32(Grid g, TileGeom t, long ncell,
                                                        PartPtrs32 p, Layout32 L, PartPtrs32 to,
                                                        const long *off) {
-    const long i = (long)blockIdx.x * PIC_BLOCK + threadIdx.x;
-    if (i >= ncell * to.cap) return;
-    const long cell = i / to.cap;
-    const int j = (int)(i % to.cap);
-    const long e = off ? off[cell] + j : i;
+    const long cell = group_cell_index();
+    if (cell >= ncell) return;
+    const int lane = threadIdx.x % CELL_LANES;
     const int cnt = min(p.count[cell], to.cap), bc = max(0, min(p.bcount[cell], cnt));
     const int nin = min(PIC_INBOX, cnt - bc);
-    if (j < bc) {
-        long tile;
-        int lc;
-        cell_tile<TX, TY, TZ>(g, t, cell, tile, lc);
-        const long src = tile * L.tcap + L.pstart[cell] + j;
+    long tile;
+    int lc;
+    cell_tile<TX, TY, TZ>(g, t, cell, tile, lc);
+    const long src0 = tile * L.tcap + L.pstart[cell], dst0 = off ? off[cell] : cell * to.cap;
+    for (int j = lane; j < bc; j += CELL_LANES) {
+        const long src = src0 + j, e = dst0 + j;
         for (int k = 0; k < 6; k++) to.p[k][e] = p.p[k][src];
         to.sp[e] = p.sp[src];
         if (to.id) to.id[e] = p.id[src];
-    } else if (j < bc + nin) {
-        const long rec = 2 * (cell * PIC_INBOX + (j - bc));
+    }
+    for (int r = lane; r < nin; r += CELL_LANES) {
+        const long rec = 2 * (cell * PIC_INBOX + r);
         const float4 A = p.inbox[rec], B = p.inbox[rec + 1];
-        place32_at(to, e, A, B, __float_as_uint(B.z));
+        place32_at(to, dst0 + bc + r, A, B, __float_as_uint(B.z));
     }
 }
 
@@ -953,23 +952,23 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_gather_particles32(Grid g, long n
                                                                  double *d4, double *d5,
                                                                  unsigned char *dsp, int *dcell,
                                                                  int *did) {
-    const long e = (long)blockIdx.x * PIC_BLOCK + threadIdx.x;
-    if (e >= ncell * p.cap) return;
-    const long c = e / p.cap;
-    const int j = (int)(e % p.cap);
-    if (j >= off[c + 1] - off[c]) return;
-    const long dst = off[c] + j;
+    const long c = group_cell_index();
+    if (c >= ncell) return;
+    const long first = off[c], n = off[c + 1] - first;
     const int i = (int)(c / ((long)g.Ny * g.Nz)), l = (int)((c / g.Nz) % g.Ny),
               k = (int)(c % g.Nz);
-    d0[dst] = ((double)i + (double)p.p[0][e]) * g.hx;
-    d1[dst] = ((double)l + (double)p.p[1][e]) * g.hy;
-    d2[dst] = ((double)k + (double)p.p[2][e]) * g.hz;
-    d3[dst] = p.p[3][e];
-    d4[dst] = p.p[4][e];
-    d5[dst] = p.p[5][e];
-    dsp[dst] = p.sp[e];
-    if (dcell) dcell[dst] = (int)c;
-    if (did) did[dst] = p.id ? p.id[e] : -1;
+    for (int j = threadIdx.x % CELL_LANES; j < n && j < p.cap; j += CELL_LANES) {
+        const long e = c * p.cap + j, dst = first + j;
+        d0[dst] = ((double)i + (double)p.p[0][e]) * g.hx;
+        d1[dst] = ((double)l + (double)p.p[1][e]) * g.hy;
+        d2[dst] = ((double)k + (double)p.p[2][e]) * g.hz;
+        d3[dst] = p.p[3][e];
+        d4[dst] = p.p[4][e];
+        d5[dst] = p.p[5][e];
+        dsp[dst] = p.sp[e];
+        if (dcell) dcell[dst] = (int)c;
+        if (did) did[dst] = p.id ? p.id[e] : -1;
+    }
 }
 
 __global__ __launch_bounds__(PIC_BLOCK) void k_gather_raw32(long ncell, const long *off,
@@ -977,30 +976,29 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_gather_raw32(long ncell, const lo
                                                            float *d2, float *d3, float *d4,
                                                            float *d5, unsigned char *dsp,
                                                            int *did) {
-    const long e = (long)blockIdx.x * PIC_BLOCK + threadIdx.x;
-    if (e >= ncell * p.cap) return;
-    const long c = e / p.cap;
-    const int j = (int)(e % p.cap);
-    if (j >= off[c + 1] - off[c]) return;
-    const long dst = off[c] + j;
-    d0[dst] = p.p[0][e];
-    d1[dst] = p.p[1][e];
-    d2[dst] = p.p[2][e];
-    d3[dst] = p.p[3][e];
-    d4[dst] = p.p[4][e];
-    d5[dst] = p.p[5][e];
-    dsp[dst] = p.sp[e];
-    if (did) did[dst] = p.id[e];
+    const long c = group_cell_index();
+    if (c >= ncell) return;
+    const long first = off[c], n = off[c + 1] - first;
+    for (int j = threadIdx.x % CELL_LANES; j < n && j < p.cap; j += CELL_LANES) {
+        const long e = c * p.cap + j, dst = first + j;
+        d0[dst] = p.p[0][e];
+        d1[dst] = p.p[1][e];
+        d2[dst] = p.p[2][e];
+        d3[dst] = p.p[3][e];
+        d4[dst] = p.p[4][e];
+        d5[dst] = p.p[5][e];
+        dsp[dst] = p.sp[e];
+        if (did) did[dst] = p.id[e];
+    }
 }
 
 __global__ __launch_bounds__(PIC_BLOCK) void k_scatter_ids32(const long *off, long ncell,
                                                             const int *src, PartPtrs32 p) {
-    const long e = (long)blockIdx.x * PIC_BLOCK + threadIdx.x;
-    if (e >= ncell * p.cap) return;
-    const long c = e / p.cap;
-    const int j = (int)(e % p.cap);
-    if (j >= off[c + 1] - off[c]) return;
-    p.id[e] = src[off[c] + j];
+    const long c = group_cell_index();
+    if (c >= ncell) return;
+    const long first = off[c], n = off[c + 1] - first;
+    for (int j = threadIdx.x % CELL_LANES; j < n && j < p.cap; j += CELL_LANES)
+        p.id[c * p.cap + j] = src[first + j];
 }
 
 inline unsigned blocks_for(long n) { return (unsigned)((n + PIC_BLOCK - 1) / PIC_BLOCK); }
@@ -1097,7 +1095,7 @@ void launch_unpack32(const Grid &g, const TileGeom &t, PartPtrs32 p, Layout32 L,
     if (from_queue)
         hipLaunchKernelGGL((k_place_spills32<TXC, TYC, TZC>), dim3((unsigned)t.ntiles),
                            dim3(PIC_BLOCK), 0, s, g, t, p, *from_queue, to);
-    hipLaunchKernelGGL((k_unpack32<TXC, TYC, TZC>), dim3(blocks_for(ncell * to.cap)),
+    hipLaunchKernelGGL((k_unpack32<TXC, TYC, TZC>), dim3(cell_blocks(ncell)),
                        dim3(PIC_BLOCK), 0, s, g, t, ncell, p, L, to, (const long *)nullptr);
     if (!from_queue)
         hipLaunchKernelGGL((k_unspill32<TXC, TYC, TZC>), dim3((unsigned)t.ntiles),
@@ -1115,7 +1113,7 @@ void launch_gather_packed32(const Grid &g, const TileGeom &t, PartPtrs32 p, Layo
     to.sp = dsp;
     to.id = did;
     to.cap = p.cap;
-    hipLaunchKernelGGL((k_unpack32<TXC, TYC, TZC>), dim3(blocks_for(ncell * to.cap)),
+    hipLaunchKernelGGL((k_unpack32<TXC, TYC, TZC>), dim3(cell_blocks(ncell)),
                        dim3(PIC_BLOCK), 0, s, g, t, ncell, p, L, to, offsets);
     hipLaunchKernelGGL((k_unspill32<TXC, TYC, TZC>), dim3((unsigned)t.ntiles), dim3(PIC_BLOCK),
                        0, s, g, t, p, L, to, offsets);
@@ -1134,27 +1132,27 @@ void launch_clear_flags32(DevStatus *st, unsigned mask, hipStream_t s) {
 
 void launch_scatter_load32(const long *offsets, long ncell, const float *src[6],
                            const unsigned char *srcsp, PartPtrs32 p, hipStream_t s) {
-    hipLaunchKernelGGL(k_scatter_load32, dim3(blocks_for(ncell * p.cap)), dim3(PIC_BLOCK), 0, s,
+    hipLaunchKernelGGL(k_scatter_load32, dim3(cell_blocks(ncell)), dim3(PIC_BLOCK), 0, s,
                        offsets, ncell, src[0], src[1], src[2], src[3], src[4], src[5], srcsp, p);
 }
 
 void launch_gather_particles32(const Grid &g, long ncell, const long *offsets, PartPtrs32 p,
                                double *dst[6], unsigned char *dsp, int *dcell, int *did,
                                hipStream_t s) {
-    hipLaunchKernelGGL(k_gather_particles32, dim3(blocks_for(ncell * p.cap)), dim3(PIC_BLOCK), 0,
+    hipLaunchKernelGGL(k_gather_particles32, dim3(cell_blocks(ncell)), dim3(PIC_BLOCK), 0,
                        s, g, ncell, offsets, p, dst[0], dst[1], dst[2], dst[3], dst[4], dst[5],
                        dsp, dcell, did);
 }
 
 void launch_gather_raw32(long ncell, const long *offsets, PartPtrs32 p, float *dst[6],
                          unsigned char *dsp, int *did, hipStream_t s) {
-    hipLaunchKernelGGL(k_gather_raw32, dim3(blocks_for(ncell * p.cap)), dim3(PIC_BLOCK), 0, s,
+    hipLaunchKernelGGL(k_gather_raw32, dim3(cell_blocks(ncell)), dim3(PIC_BLOCK), 0, s,
                        ncell, offsets, p, dst[0], dst[1], dst[2], dst[3], dst[4], dst[5], dsp,
                        did);
 }
 
 void launch_scatter_ids32(const long *offsets, long ncell, const int *src, PartPtrs32 p,
                           hipStream_t s) {
-    hipLaunchKernelGGL(k_scatter_ids32, dim3(blocks_for(ncell * p.cap)), dim3(PIC_BLOCK), 0, s,
+    hipLaunchKernelGGL(k_scatter_ids32, dim3(cell_blocks(ncell)), dim3(PIC_BLOCK), 0, s,
                        offsets, ncell, src, p);
 }

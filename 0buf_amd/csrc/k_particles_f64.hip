@@ -656,21 +656,20 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_scatter_load(const long *off, lon
                                                            const double *s2, const double *s3,
                                                            const double *s4, const double *s5,
                                                            const unsigned char *ssp, PartPtrs p) {
-    const long e = (long)blockIdx.x * PIC_BLOCK + threadIdx.x;
-    if (e >= ncell * p.cap) return;
-    const long c = e / p.cap;
-    const int j = (int)(e % p.cap);
-    const long n = off[c + 1] - off[c];
-    if (j == 0) p.count[c] = (int)n;
-    if (j >= n) return;
-    const long src = off[c] + j;
-    p.p[0][e] = s0[src];
-    p.p[1][e] = s1[src];
-    p.p[2][e] = s2[src];
-    p.p[3][e] = s3[src];
-    p.p[4][e] = s4[src];
-    p.p[5][e] = s5[src];
-    p.sp[e] = ssp[src];
+    const long c = group_cell_index();
+    if (c >= ncell) return;
+    const long first = off[c], n = off[c + 1] - first;
+    if (threadIdx.x % CELL_LANES == 0) p.count[c] = (int)n;
+    for (int j = threadIdx.x % CELL_LANES; j < n && j < p.cap; j += CELL_LANES) {
+        const long e = c * p.cap + j, src = first + j;
+        p.p[0][e] = s0[src];
+        p.p[1][e] = s1[src];
+        p.p[2][e] = s2[src];
+        p.p[3][e] = s3[src];
+        p.p[4][e] = s4[src];
+        p.p[5][e] = s5[src];
+        p.sp[e] = ssp[src];
+    }
 }
 
 __global__ __launch_bounds__(PIC_BLOCK) void k_repack(long ncell, PartPtrs from, PartPtrs to) {
@@ -706,12 +705,11 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_copy_parts(long ncell, PartPtrs f
 
 __global__ __launch_bounds__(PIC_BLOCK) void k_scatter_ids(const long *off, long ncell,
                                                           const int *src, PartPtrs p) {
-    const long e = (long)blockIdx.x * PIC_BLOCK + threadIdx.x;
-    if (e >= ncell * p.cap) return;
-    const long c = e / p.cap;
-    const int j = (int)(e % p.cap);
-    if (j >= off[c + 1] - off[c]) return;
-    p.id[e] = src[off[c] + j];
+    const long c = group_cell_index();
+    if (c >= ncell) return;
+    const long first = off[c], n = off[c + 1] - first;
+    for (int j = threadIdx.x % CELL_LANES; j < n && j < p.cap; j += CELL_LANES)
+        p.id[c * p.cap + j] = src[first + j];
 }
 
 __global__ __launch_bounds__(PIC_BLOCK) void k_fix_arrivals(QueuePtrs q, int oldcap, PartPtrs to) {
@@ -739,21 +737,21 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_gather_particles(long ncell, cons
                                                                double *d2, double *d3, double *d4,
                                                                double *d5, unsigned char *dsp,
                                                                int *dcell, int *did) {
-    const long e = (long)blockIdx.x * PIC_BLOCK + threadIdx.x;
-    if (e >= ncell * p.cap) return;
-    const long c = e / p.cap;
-    const int j = (int)(e % p.cap);
-    if (j >= off[c + 1] - off[c]) return;
-    const long dst = off[c] + j;
-    d0[dst] = p.p[0][e];
-    d1[dst] = p.p[1][e];
-    d2[dst] = p.p[2][e];
-    d3[dst] = p.p[3][e];
-    d4[dst] = p.p[4][e];
-    d5[dst] = p.p[5][e];
-    dsp[dst] = p.sp[e];
-    if (dcell) dcell[dst] = (int)c;
-    if (did) did[dst] = p.id ? p.id[e] : -1;
+    const long c = group_cell_index();
+    if (c >= ncell) return;
+    const long first = off[c], n = off[c + 1] - first;
+    for (int j = threadIdx.x % CELL_LANES; j < n && j < p.cap; j += CELL_LANES) {
+        const long e = c * p.cap + j, dst = first + j;
+        d0[dst] = p.p[0][e];
+        d1[dst] = p.p[1][e];
+        d2[dst] = p.p[2][e];
+        d3[dst] = p.p[3][e];
+        d4[dst] = p.p[4][e];
+        d5[dst] = p.p[5][e];
+        dsp[dst] = p.sp[e];
+        if (dcell) dcell[dst] = (int)c;
+        if (did) did[dst] = p.id ? p.id[e] : -1;
+    }
 }
 
 inline unsigned blocks_for(long n) { return (unsigned)((n + PIC_BLOCK - 1) / PIC_BLOCK); }
@@ -830,7 +828,7 @@ void launch_arrive_fold_f64(const Grid &g, const TileGeom &t, PartPtrs p, QueueP
 
 void launch_scatter_load(const long *offsets, long ncell, const double *src[6],
                          const unsigned char *srcsp, PartPtrs p, hipStream_t s) {
-    hipLaunchKernelGGL(k_scatter_load, dim3(blocks_for(ncell * p.cap)), dim3(PIC_BLOCK), 0, s,
+    hipLaunchKernelGGL(k_scatter_load, dim3(cell_blocks(ncell)), dim3(PIC_BLOCK), 0, s,
                        offsets, ncell, src[0], src[1], src[2], src[3], src[4], src[5], srcsp, p);
 }
 
@@ -846,14 +844,14 @@ void launch_fix_arrivals(const TileGeom &t, QueuePtrs q, int oldcap, PartPtrs to
 
 void launch_gather_particles(long ncell, const long *offsets, PartPtrs p, double *dst[6],
                              unsigned char *dsp, int *dcell, int *did, hipStream_t s) {
-    hipLaunchKernelGGL(k_gather_particles, dim3(blocks_for(ncell * p.cap)), dim3(PIC_BLOCK), 0, s,
+    hipLaunchKernelGGL(k_gather_particles, dim3(cell_blocks(ncell)), dim3(PIC_BLOCK), 0, s,
                        ncell, offsets, p, dst[0], dst[1], dst[2], dst[3], dst[4], dst[5], dsp,
                        dcell, did);
 }
 
 void launch_scatter_ids(const long *offsets, long ncell, const int *src, PartPtrs p,
                         hipStream_t s) {
-    hipLaunchKernelGGL(k_scatter_ids, dim3(blocks_for(ncell * p.cap)), dim3(PIC_BLOCK), 0, s,
+    hipLaunchKernelGGL(k_scatter_ids, dim3(cell_blocks(ncell)), dim3(PIC_BLOCK), 0, s,
                        offsets, ncell, src, p);
 }
 
