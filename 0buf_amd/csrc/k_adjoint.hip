@@ -39,8 +39,9 @@ constexpr int TXC = 2, TYC = 4, TZC = 8;
  * adding into copy l % ACOPIES, copies 9 mod 16 doubles apart (the reasons
  * stand at the FP32 adjoint's).  Measured, one step at 24.6M particles,
  * 128x64x64 cells, before the changes below: 2.54 ms with 5 copies, 2.61 with
- * 4, 2.83 with 3; 3.71 with 3 copies on the same banks. */
-constexpr int ACOPIES = 6;
+ * 4, 2.83 with 3; 3.71 with 3 copies on the same banks.  6 copies of whole
+ * boxes leave one workgroup per CU (86 KB). */
+constexpr int ACOPIES = 5;
 constexpr int copy_stride(int n) { return (n + 6) / 16 * 16 + 9; }   /* >= n, 9 mod 16 */
 
 inline unsigned blocks_for(long n) { return (unsigned)((n + PIC_BLOCK - 1) / PIC_BLOCK); }
@@ -332,12 +333,14 @@ template <int TX, int TY, int TZ, int NT>
 __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
     constexpr int C = TX * TY * TZ;
     constexpr int BX = TX + 2, BY = TY + 2, BZ = TZ + 2, NB = BX * BY * BZ;
-    /* Ex, Hy, Hz and Jx (node-type, or dual, along x) take x planes 0..TX only
-     * (NBX nodes), the others all BX planes, as in the FP32 form's boxes */
+    /* Every field component takes all BX planes: a particle exactly on its
+     * cell's upper face stays in the cell (flyDirection's v > v0 + h), and its
+     * node-type components then read the planes behind that face, TX and TX + 1
+     * in the tile's last cell.  (FP32 offsets stay below 1; their boxes end
+     * earlier.)  Jx, dual along x, is read at planes 0..TX only. */
     constexpr int NBX = (TX + 1) * BY * BZ;
-    constexpr int FB[6] = {0, NBX, NBX + NB, NBX + 2 * NB, NBX + 3 * NB, 2 * NBX + 3 * NB};
-    constexpr int FN[6] = {NBX, NB, NB, NB, NBX, NBX};   /* nodes in each box */
-    constexpr int NF = 3 * NBX + 3 * NB, NJ = NBX + 2 * NB, JY0 = FB[1], JZ0 = FB[2];
+    constexpr int NF = 6 * NB, NJ = NBX + 2 * NB, JY0 = NBX, JZ0 = NBX + NB;
+    constexpr int LB[3] = {0, JY0, JZ0}, LN[3] = {NBX, NB, NB};   /* lamJ: start, nodes */
     constexpr int AS = copy_stride(NF);
     static_assert(AS >= NF && AS % 16 == 9, "");
     __shared__ double sF[NF];        /* E, H' of the forward step */
@@ -386,11 +389,10 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
         }
         if (tid < NB) {
 #pragma unroll
-            for (int q = 0; q < 6; q++) {
-                if (tid >= FN[q]) continue;
-                sF[FB[q] + tid] = fv[q];
-                if (q < 3) sL[FB[q] + tid] = lj[q];
-            }
+            for (int q = 0; q < 6; q++) sF[q * NB + tid] = fv[q];
+#pragma unroll
+            for (int q = 0; q < 3; q++)
+                if (tid < LN[q]) sL[LB[q] + tid] = lj[q];
         }
         if (tid < C) sCnt[tid] = cnt;
     }
@@ -454,17 +456,17 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
                           Y = W.iy != 2 ? BZ : 0, Y1 = W.i1y != 2 ? BZ : 0, Z = W.iz - 2,
                           Z1 = W.i1z - 2;
                 o[0] = X + Y1 + Z1;
-                Ef[0] = interp_grad<BY, BZ>(sF + FB[0], o[0], s11, s41, s61, gw[0]);
+                Ef[0] = interp_grad<BY, BZ>(sF + 0 * NB, o[0], s11, s41, s61, gw[0]);
                 o[1] = X1 + Y + Z1;
-                Ef[1] = interp_grad<BY, BZ>(sF + FB[1], o[1], s21, s31, s61, gw[1]);
+                Ef[1] = interp_grad<BY, BZ>(sF + 1 * NB, o[1], s21, s31, s61, gw[1]);
                 o[2] = X1 + Y1 + Z;
-                Ef[2] = interp_grad<BY, BZ>(sF + FB[2], o[2], s21, s41, s51, gw[2]);
+                Ef[2] = interp_grad<BY, BZ>(sF + 2 * NB, o[2], s21, s41, s51, gw[2]);
                 o[3] = X1 + Y + Z;
-                Hf[0] = interp_grad<BY, BZ>(sF + FB[3], o[3], s21, s31, s51, gw[3]);
+                Hf[0] = interp_grad<BY, BZ>(sF + 3 * NB, o[3], s21, s31, s51, gw[3]);
                 o[4] = X + Y1 + Z;
-                Hf[1] = interp_grad<BY, BZ>(sF + FB[4], o[4], s11, s41, s51, gw[4]);
+                Hf[1] = interp_grad<BY, BZ>(sF + 4 * NB, o[4], s11, s41, s51, gw[4]);
                 o[5] = X + Y + Z1;
-                Hf[2] = interp_grad<BY, BZ>(sF + FB[5], o[5], s11, s31, s61, gw[5]);
+                Hf[2] = interp_grad<BY, BZ>(sF + 5 * NB, o[5], s11, s31, s61, gw[5]);
             }
         }
         const Boris B = boris_move<true>(pu, pv, pw, Ef[0], Ef[1], Ef[2], Hf[0], Hf[1], Hf[2], tau1);
@@ -585,17 +587,17 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
         /* gather: scatter into the adjoint box, position derivative through
          * the weights (every far weight has d/dx = 1/h) */
         if (live && W.ok) {
-            interp_scatter<BY, BZ>(myA + FB[0], o[0], W.s1, 1. - W.s1, W.s4, 1. - W.s4, W.s6,
+            interp_scatter<BY, BZ>(myA + 0 * NB, o[0], W.s1, 1. - W.s1, W.s4, 1. - W.s4, W.s6,
                                    1. - W.s6, lE[0]);
-            interp_scatter<BY, BZ>(myA + FB[1], o[1], W.s2, 1. - W.s2, W.s3, 1. - W.s3, W.s6,
+            interp_scatter<BY, BZ>(myA + 1 * NB, o[1], W.s2, 1. - W.s2, W.s3, 1. - W.s3, W.s6,
                                    1. - W.s6, lE[1]);
-            interp_scatter<BY, BZ>(myA + FB[2], o[2], W.s2, 1. - W.s2, W.s4, 1. - W.s4, W.s5,
+            interp_scatter<BY, BZ>(myA + 2 * NB, o[2], W.s2, 1. - W.s2, W.s4, 1. - W.s4, W.s5,
                                    1. - W.s5, lE[2]);
-            interp_scatter<BY, BZ>(myA + FB[3], o[3], W.s2, 1. - W.s2, W.s3, 1. - W.s3, W.s5,
+            interp_scatter<BY, BZ>(myA + 3 * NB, o[3], W.s2, 1. - W.s2, W.s3, 1. - W.s3, W.s5,
                                    1. - W.s5, lH[0]);
-            interp_scatter<BY, BZ>(myA + FB[4], o[4], W.s1, 1. - W.s1, W.s4, 1. - W.s4, W.s5,
+            interp_scatter<BY, BZ>(myA + 4 * NB, o[4], W.s1, 1. - W.s1, W.s4, 1. - W.s4, W.s5,
                                    1. - W.s5, lH[1]);
-            interp_scatter<BY, BZ>(myA + FB[5], o[5], W.s1, 1. - W.s1, W.s3, 1. - W.s3, W.s6,
+            interp_scatter<BY, BZ>(myA + 5 * NB, o[5], W.s1, 1. - W.s1, W.s3, 1. - W.s3, W.s6,
                                    1. - W.s6, lH[2]);
             const double rh[3] = {a.dc.rhx, a.dc.rhy, a.dc.rhz};
             for (int d = 0; d < 3; d++) {
@@ -614,8 +616,7 @@ __global__ __launch_bounds__(NT) void k_adj_particles(AdjArgs a) {
     if (tid < NB) {   /* thread n adds box node n of the six adjoint boxes */
 #pragma unroll
         for (int q = 0; q < 6; q++) {
-            if (tid >= FN[q]) continue;
-            const int e = FB[q] + tid;
+            const int e = q * NB + tid;
             double val = sA[e];
             for (int r = 1; r < ACOPIES; r++) val += sA[r * AS + e];
             if (val != 0.0 && node_in)
