@@ -113,11 +113,14 @@ __device__ __forceinline__ void pqr_lds(double *sJ, const Geo &c, const DivConst
     const double wz0 = fma(dx1, dy1, s3), wz1 = fma(dx1, dy, -s3), wz2 = fma(dx, dy1, -s3),
                  wz3 = fma(dx, dy, s3);
     if constexpr (DIFF) {
-        /* every contribution below 8 (2^51 units): a weight inside the dual
-         * cell is at most 13/12 of the face; where that bound does not tell,
+        /* every contribution below 8 (2^51 units): the larger of each pair of
+         * distances bounds the weights, wherever the segment lies (its end may
+         * be many cells away at a large tau); where that bound does not tell,
          * the contributions themselves */
-        if (!(fabs(su) * dc.face[0] < 4.0 && fabs(sv) * dc.face[1] < 4.0 &&
-              fabs(sw) * dc.face[2] < 4.0)) {
+        const double mx = fmax(fabs(dx), fabs(dx1)), my = fmax(fabs(dy), fabs(dy1)),
+                     mz = fmax(fabs(dz), fabs(dz1));
+        if (!(fabs(su) * fma(my, mz, fabs(s1)) < 7.9 && fabs(sv) * fma(mx, mz, fabs(s2)) < 7.9 &&
+              fabs(sw) * fma(mx, my, fabs(s3)) < 7.9)) {
             auto over = [](double a, double w0, double w1, double w2, double w3) {
                 return !(fabs(a * w0) < 8.0 && fabs(a * w1) < 8.0 && fabs(a * w2) < 8.0 &&
                          fabs(a * w3) < 8.0);

@@ -26,7 +26,6 @@ struct DivConst {
     double r12;               /* 1/12 */
     double Dx, Dy, Dz;        /* (tau hy) hz, (tau hx) hz, (tau hx) hy (cell.h:1578-1580) */
     double rDx, rDy, rDz;
-    double face[3];           /* 13/12 of the cell's faces: the largest weight of a segment */
 };
 
 inline DivConst make_divconst(const Grid &g) {
@@ -41,9 +40,6 @@ inline DivConst make_divconst(const Grid &g) {
     d.rDx = 1.0 / d.Dx;
     d.rDy = 1.0 / d.Dy;
     d.rDz = 1.0 / d.Dz;
-    d.face[0] = 13.0 / 12.0 * g.hy * g.hz;
-    d.face[1] = 13.0 / 12.0 * g.hx * g.hz;
-    d.face[2] = 13.0 / 12.0 * g.hx * g.hy;
     return d;
 }
 
