@@ -129,6 +129,20 @@ void give_ring(Ring *r) {
     free_ring(r);
 }
 
+/* the context's device for the time of a call, which may come from a thread
+ * whose current device is another: events and pinned memory belong to the
+ * device current when they are made */
+struct OnDevice {
+    int before = -1;
+    hipError_t enter(int dev) {
+        const hipError_t e = hipGetDevice(&before);
+        return e == hipSuccess ? hipSetDevice(dev) : e;
+    }
+    ~OnDevice() {
+        if (before >= 0) (void)hipSetDevice(before);
+    }
+};
+
 struct Lease {
     Ring *ring = nullptr;
     ~Lease() {
@@ -156,6 +170,8 @@ void readback_detach() {
 
 int readback(pic_ctx *c, void *dst_, const void *src_, long n, ReadAs as) {
     if (n <= 0) return PIC_SUCCESS;
+    OnDevice here;
+    HIPCHK(here.enter(c->dev));
     char *const dst = (char *)dst_;
     const char *const src = (const char *)src_;
     const size_t width = as == ReadAs::f32_to_f64 || as == ReadAs::i32 ? 4 : 8;

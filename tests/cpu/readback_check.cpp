@@ -1,0 +1,131 @@
+/*
+ * readback_check.cpp -- pic_readback.hip on the CPU, over a stand-in for the
+ * few runtime calls it makes: two devices, whose memory is the host's, copies
+ * that happen when their event or stream is waited for, an event that belongs to
+ * the device current at its creation, and a wait that can be made to fail.
+ *
+ *   device    a context on the device that is not current
+ */
+#include <cstdio>
+#include <cstring>
+#include <map>
+#include <string>
+#include <vector>
+
+#include "pic_ctx.h"
+
+struct ihipStream_t {
+    int dev;
+};
+struct ihipEvent_t {
+    int dev;
+};
+
+namespace {
+struct Copy {
+    void *dst;
+    const void *src;
+    size_t n;
+};
+std::vector<Copy> queued;
+int current = 0;
+
+hipError_t drain() {
+    for (const Copy &c : queued) std::memcpy(c.dst, c.src, c.n);
+    queued.clear();
+    return hipSuccess;
+}
+}  // namespace
+
+extern "C" {
+hipError_t hipGetDevice(int *d) {
+    *d = current;
+    return hipSuccess;
+}
+hipError_t hipSetDevice(int d) {
+    if (d < 0 || d > 1) return hipErrorInvalidDevice;
+    current = d;
+    return hipSuccess;
+}
+hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *) {
+    a->type = hipMemoryTypeUnregistered;
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+    *p = new char[n];
+    return hipSuccess;
+}
+hipError_t hipHostFree(void *p) {
+    delete[] (char *)p;
+    return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+    *e = new ihipEvent_t{current};
+    return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t e) {
+    delete e;
+    return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+    return e->dev == s->dev ? hipSuccess : hipErrorInvalidHandle;
+}
+hipError_t hipEventSynchronize(hipEvent_t) { return drain(); }
+hipError_t hipStreamSynchronize(hipStream_t) { return drain(); }
+hipError_t hipMemcpy(void *dst, const void *src, size_t n, hipMemcpyKind) {
+    std::memcpy(dst, src, n);
+    return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t) {
+    queued.push_back({dst, src, n});
+    return hipSuccess;
+}
+}
+
+namespace picx {
+thread_local char g_hip_err[256];
+int record_hip(hipError_t, const char *) { return PIC_ERR_HIP; }
+}  // namespace picx
+
+namespace {
+int bad = 0;
+void expect(bool ok, const char *what) {
+    if (ok) return;
+    std::printf("%s\n", what);
+    bad = 1;
+}
+
+struct Box {
+    ihipStream_t stream;
+    pic_ctx c;
+    explicit Box(int dev) : stream{dev} {
+        c.dev = dev;
+        c.stream = &stream;
+        picx::readback_attach();
+    }
+    ~Box() { picx::readback_detach(); }
+};
+
+/* more than the ring holds, and no whole number of chunks */
+constexpr long N = 3'000'001;
+
+int device() {
+    std::vector<int> src(N), dst(N, -1);
+    for (long k = 0; k < N; k++) src[k] = (int)(k * 2654435761u);
+    Box a(0), b(1);
+    for (Box *x : {&b, &a, &b}) {
+        dst.assign(N, -1);
+        expect(picx::readback(&x->c, dst.data(), src.data(), N, picx::ReadAs::i32) == PIC_SUCCESS,
+               "a context on the device that is not current cannot be read");
+        expect(dst == src, "values differ");
+        expect(current == 0, "the caller's current device changed");
+    }
+    return bad;
+}
+}  // namespace
+
+int main(int argc, char **argv) {
+    const std::map<std::string, int (*)()> checks = {{"device", device}};
+    return argc == 2 && checks.count(argv[1]) ? checks.at(argv[1])() : 2;
+}
