@@ -200,13 +200,20 @@ int readback(pic_ctx *c, void *dst_, const void *src_, long n, ReadAs as) {
         move_chunk(dst, chunk(i), i * per, (long)(size(i) / width), as);
     };
     /* the pages of a chunk's destination, faulted in while the chunk is on its
-     * way (and the kernels before it run) */
+     * way (and the kernels before it run), by a write that changes nothing (0
+     * for 0; the instruction takes the page for writing either way): a copy
+     * that fails leaves the array as it was */
     const size_t out_width = as == ReadAs::i32 ? 4 : 8;
     auto touch = [&](long i) {
-        volatile char *const p = dst + i * per * out_width;
+        char *const p = dst + i * per * out_width;
         const size_t len = size(i) / width * out_width;
-        for (size_t k = 0; k < len; k += 4096) p[k] = 0;
-        p[len - 1] = 0;
+        auto take = [](char *at) {
+            char was = 0;
+            __atomic_compare_exchange_n(at, &was, (char)0, false, __ATOMIC_RELAXED,
+                                        __ATOMIC_RELAXED);
+        };
+        for (size_t k = 0; k < len; k += 4096) take(p + k);
+        take(p + len - 1);
     };
     auto issue = [&](long i) -> hipError_t {
         hipError_t e = hipMemcpyAsync(chunk(i), src + i * CHUNK, size(i), hipMemcpyDeviceToHost,

@@ -5,6 +5,7 @@
  * the device current at its creation, and a wait that can be made to fail.
  *
  *   device    a context on the device that is not current
+ *   failed    a call that fails leaves the caller's array as it was
  */
 #include <cstdio>
 #include <cstring>
@@ -29,8 +30,13 @@ struct Copy {
 };
 std::vector<Copy> queued;
 int current = 0;
+bool fail = false;
 
 hipError_t drain() {
+    if (fail) {
+        queued.clear();
+        return hipErrorUnknown;
+    }
     for (const Copy &c : queued) std::memcpy(c.dst, c.src, c.n);
     queued.clear();
     return hipSuccess;
@@ -123,9 +129,27 @@ int device() {
     }
     return bad;
 }
+
+int failed() {
+    const std::vector<double> src(N, 1.0);
+    Box a(0);
+    for (long n : {N, 300'000L}) {   /* through the ring, and one chunk */
+        for (picx::ReadAs as : {picx::ReadAs::f64, picx::ReadAs::f32_to_f64}) {
+            std::vector<double> dst(n, -1.0);
+            fail = true;
+            expect(picx::readback(&a.c, dst.data(), src.data(), n, as) == PIC_ERR_HIP,
+                   "a failed copy is not reported");
+            fail = false;
+            expect(dst == std::vector<double>(n, -1.0), "a failed call wrote into the array");
+            expect(picx::readback(&a.c, dst.data(), src.data(), n, picx::ReadAs::f64) == PIC_SUCCESS &&
+                       dst == std::vector<double>(n, 1.0), "the next call does not read");
+        }
+    }
+    return bad;
+}
 }  // namespace
 
 int main(int argc, char **argv) {
-    const std::map<std::string, int (*)()> checks = {{"device", device}};
+    const std::map<std::string, int (*)()> checks = {{"device", device}, {"failed", failed}};
     return argc == 2 && checks.count(argv[1]) ? checks.at(argv[1])() : 2;
 }
