@@ -19,6 +19,7 @@
  */
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <cstring>
 #include <mutex>
 #include <new>
@@ -223,17 +224,30 @@ int readback(pic_ctx *c, void *dst_, const void *src_, long n, ReadAs as) {
     std::atomic<long> next{0}, ready{0}, moved[RING];
     for (auto &m : moved) m.store(0, std::memory_order_relaxed);
     std::atomic<bool> stop{false};
+    /* a worker whose chunk is not there within a millisecond or so (a long
+     * kernel runs before it) sleeps until the next one arrives */
+    constexpr int SPINS = 1 << 15;
+    std::mutex arrival;
+    std::condition_variable arrives;
+    auto publish = [&](auto change) {
+        {
+            std::lock_guard<std::mutex> hold(arrival);
+            change();
+        }
+        arrives.notify_all();
+    };
     auto work = [&]() {
         for (;;) {
             const long i = next.fetch_add(1, std::memory_order_relaxed);
             if (i >= nch) return;
             touch(i);
-            int spins = 0;
-            while (ready.load(std::memory_order_acquire) <= i) {
-                if (stop.load(std::memory_order_relaxed)) return;
-                if (++spins < 4096) relax();
-                else std::this_thread::yield();   /* a long kernel runs before it */
+            auto there = [&] { return ready.load(std::memory_order_acquire) > i || stop.load(); };
+            for (int spins = 0; spins < SPINS && !there(); spins++) relax();
+            if (!there()) {
+                std::unique_lock<std::mutex> hold(arrival);
+                arrives.wait(hold, there);
             }
+            if (ready.load(std::memory_order_acquire) <= i) return;   /* stopped */
             move(i);
             moved[i % S].store(i + 1, std::memory_order_release);
         }
@@ -263,12 +277,12 @@ int readback(pic_ctx *c, void *dst_, const void *src_, long n, ReadAs as) {
                 move(arrived);
                 moved[arrived % S].store(arrived + 1, std::memory_order_relaxed);
             }
-            ready.store(++arrived, std::memory_order_release);
+            publish([&] { ready.store(++arrived, std::memory_order_release); });
         } else {
             relax();
         }
     }
-    if (e != hipSuccess) stop.store(true, std::memory_order_relaxed);
+    if (e != hipSuccess) publish([&] { stop.store(true); });
     for (int k = 0; k < nw; k++) pool[k].join();
     if (e != hipSuccess) {
         (void)hipStreamSynchronize(c->stream);

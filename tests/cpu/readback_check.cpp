@@ -6,11 +6,16 @@
  *
  *   device    a context on the device that is not current
  *   failed    a call that fails leaves the caller's array as it was
+ *   waiting   a call that waits for a long kernel leaves the CPUs alone
  */
+#include <sys/resource.h>
+
+#include <chrono>
 #include <cstdio>
 #include <cstring>
 #include <map>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "pic_ctx.h"
@@ -31,8 +36,11 @@ struct Copy {
 std::vector<Copy> queued;
 int current = 0;
 bool fail = false;
+int kernel_ms = 0;   /* what the first wait takes */
 
 hipError_t drain() {
+    std::this_thread::sleep_for(std::chrono::milliseconds(kernel_ms));
+    kernel_ms = 0;
     if (fail) {
         queued.clear();
         return hipErrorUnknown;
@@ -147,9 +155,28 @@ int failed() {
     }
     return bad;
 }
+
+double cpu_seconds() {
+    rusage r;
+    getrusage(RUSAGE_SELF, &r);
+    return r.ru_utime.tv_sec + r.ru_stime.tv_sec +
+           1e-6 * (r.ru_utime.tv_usec + r.ru_stime.tv_usec);
+}
+
+int waiting() {
+    const std::vector<double> src(N, 1.0);
+    std::vector<double> dst(N, -1.0);
+    Box a(0);
+    kernel_ms = 1000;
+    const double before = cpu_seconds();
+    expect(picx::readback(&a.c, dst.data(), src.data(), N, picx::ReadAs::f64) == PIC_SUCCESS &&
+               dst == src, "values differ");
+    expect(cpu_seconds() - before < 0.5, "half a second of CPU time while a kernel runs");
+    return bad;
+}
 }  // namespace
 
 int main(int argc, char **argv) {
-    const std::map<std::string, int (*)()> checks = {{"device", device}, {"failed", failed}};
+    const std::map<std::string, int (*)()> checks = {{"device", device}, {"failed", failed}, {"waiting", waiting}};
     return argc == 2 && checks.count(argv[1]) ? checks.at(argv[1])() : 2;
 }

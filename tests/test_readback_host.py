@@ -27,7 +27,7 @@ def check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("name", ["device", "failed"])
+@pytest.mark.parametrize("name", ["device", "failed", "waiting"])
 def test_readback(check, name):
     r = subprocess.run([check, name], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
