@@ -689,23 +689,6 @@ __global__ __launch_bounds__(PIC_BLOCK) void k_repack(long ncell, PartPtrs from,
     if (to.id) to.id[dst] = from.id[e];
 }
 
-/* bucket copy with any capacities (checkpoint save and restore): occupied
- * slots, ids and counts */
-__global__ __launch_bounds__(PIC_BLOCK) void k_copy_parts(long ncell, PartPtrs from, PartPtrs to) {
-    const long e = (long)blockIdx.x * PIC_BLOCK + threadIdx.x;
-    if (e >= ncell * from.cap) return;
-    const long c = e / from.cap;
-    const int j = (int)(e % from.cap);
-    int n = from.count[c];
-    if (n > from.cap) n = from.cap;
-    if (j == 0) to.count[c] = n;
-    if (j >= n) return;
-    const long dst = c * to.cap + j;
-    for (int k = 0; k < 6; k++) to.p[k][dst] = from.p[k][e];
-    to.sp[dst] = from.sp[e];
-    if (to.id) to.id[dst] = from.id[e];
-}
-
 __global__ __launch_bounds__(PIC_BLOCK) void k_scatter_ids(const long *off, long ncell,
                                                           const int *src, PartPtrs p) {
     const long c = group_cell_index();
@@ -856,11 +839,6 @@ void launch_scatter_ids(const long *offsets, long ncell, const int *src, PartPtr
                         hipStream_t s) {
     hipLaunchKernelGGL(k_scatter_ids, dim3(cell_blocks(ncell)), dim3(PIC_BLOCK), 0, s,
                        offsets, ncell, src, p);
-}
-
-void launch_copy_parts(long ncell, PartPtrs from, PartPtrs to, hipStream_t s) {
-    hipLaunchKernelGGL(k_copy_parts, dim3(blocks_for(ncell * from.cap)), dim3(PIC_BLOCK), 0, s,
-                       ncell, from, to);
 }
 
 /* With few tiles the push lasts as long as the fullest CU takes: tiles of 16

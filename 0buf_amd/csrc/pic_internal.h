@@ -652,7 +652,6 @@ void launch_adj_particles_f32(const Grid &g, const TileGeom &t, AdjFwd32 fwd, Pa
 void launch_scale_lam(LamParts lp, double sx, double sy, double sz, hipStream_t s);
 void launch_adj_seed_energy32(const Grid &g, const float *const E[3], double w, AdjLam l,
                               hipStream_t s);
-void launch_copy_parts(long ncell, PartPtrs from, PartPtrs to, hipStream_t s);
 void launch_mismatch(const void *a, const void *b, long n, int elem_bytes, DevStatus *st,
                      hipStream_t s);
 
